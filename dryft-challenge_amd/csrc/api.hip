@@ -749,14 +749,8 @@ int qdec_prefill_gemm(const qdec_pgemm_args *a, qdec_stream_t stream) {
   const uint32_t f = a->flags;
   if (f != 0u && f != QDEC_RES_OUT && f != QDEC_GLU)
     return set_error(QDEC_EUNSUPPORTED, "qdec_prefill_gemm: flags 0x%x not supported (0, RES_OUT or GLU)", f);
-  // Workgroup tile (activation rows x weight rows): 256 x 256 reads a third
-  // fewer LDS bytes per MFMA than 256 x 128 but makes half the workgroups;
-  // 64 x 64 makes 8x the workgroups of 256 x 128 for few rows.  Picked by
-  // the launch size: 256 x 256 from 600 workgroups (at 16K rows QKV and
-  // gate/up ~+10%, down +6%, O even with 640 workgroups; at 8K rows O and
-  // down, 320 workgroups, are 10% faster on 256 x 128), 256 x 128 from 512,
-  // else 64 x 64 (a 512-token prompt: O and down would have 40 workgroups
-  // of 256 x 128) -- unless one round of large tiles fills 128-256 CUs.
+  // Workgroup tile (activation rows x weight rows), picked below when 0 x 0.
+  const bool glu = (f & QDEC_GLU) != 0;
   int trows = a->tile_rows, tcols = a->tile_cols;
   const bool pair_ok = (trows == 0 && tcols == 0) || (trows == 256 && (tcols == 128 || tcols == 256)) ||
                        (trows == 64 && tcols == 64);
@@ -768,21 +762,24 @@ int qdec_prefill_gemm(const qdec_pgemm_args *a, qdec_stream_t stream) {
   const bool whole256 = a->tiles % (kPgRows / 16) == 0;
   if (trows == 0 && !whole256) trows = 64, tcols = 64;
   if (trows == 0) {
-    // Workgroups of each large tile; from 600 (256 x 256) or 512 (256 x 128)
-    // they run in several rounds.  Below that a large tile still pays when
-    // one round of them covers half to all of the 256 CUs: the prefill of
-    // one sequence on MI355X, ms (64 x 64 / chosen), gate/up 256 x 256 at
-    // 512 rows 9.46 / 8.67 and at 768 rows 12.41 / 10.49, gate/up 256 x 128
-    // at 256 rows 7.11 / 6.85, QKV 256 x 128 at 1024 rows 14.62 / 14.11.
+    // The least of the tiles' costs, in rounds of 256 x 256 tiles: the
+    // 256-row tiles run one per CU, so ceil(tiles / 256) rounds, a round of
+    // 256 x 160 or 256 x 128 costing 0.80 or 0.59 of one (narrower tiles load
+    // more per MFMA); 64 x 64 tiles run three per CU without whole rounds at
+    // about half the rate.  MI355X, us (64 x 64 / 256 x 128 / 256 x 160 /
+    // 256 x 256): O at 1024 rows 39 / 51 / 66 / 86, at 4096 119 / 108 / 77 /
+    // 93, at 8192 226 / 166 / 147 / 186, at 32768 1202 / 641 / 613 / 544;
+    // gate/up at 256 rows 50 / 40 / - / 116, at 512 89 / 75 / - / 67, at 8192
+    // 1148 / 691 / - / 635; QKV at 1024 50 / 39 / - / 63.
+    static const struct { int cols; double cost; } kTiles[] = {{256, 1.0}, {160, 0.80}, {128, 0.59}};
     const int64_t row_tiles = a->tiles / 16;
-    const int64_t w256 = a->n % 256 == 0 ? (a->n / 256) * row_tiles : 0;
-    const int64_t w128 = a->n % 128 == 0 ? (a->n / 128) * row_tiles : 0;
-    if (w256 >= 600 || (w256 >= 128 && w256 <= 256)) {
-      trows = 256, tcols = 256;
-    } else if (w128 >= 512 || (w128 >= 128 && w128 <= 256)) {
-      trows = 256, tcols = 128;
-    } else {
-      trows = 64, tcols = 64;
+    double best = 2.0 * (double)row_tiles * a->n / (256.0 * kPgWorkgroups);
+    trows = 64, tcols = 64;
+    for (const auto &t : kTiles) {
+      if (a->n % t.cols || (glu && t.cols == 160)) continue;
+      const int64_t T = (a->n / t.cols) * row_tiles;
+      const double cost = t.cost * (double)((T + kPgWorkgroups - 1) / kPgWorkgroups);
+      if (cost < best) best = cost, trows = 256, tcols = t.cols;
     }
   }
   if (a->rows < 1 || a->k < kPgStageK || a->k % kPgStageK || a->n < tcols || a->n % tcols)
@@ -807,7 +804,6 @@ int qdec_prefill_gemm(const qdec_pgemm_args *a, qdec_stream_t stream) {
   p.k = a->k;
   p.tiles = a->tiles;
   p.ofrag = a->out_frag;
-  const bool glu = (f & QDEC_GLU) != 0;
   p.n_out = glu ? a->n / 2 : a->n;
   p.up_tiles = a->n / 32;
   p.tile_rows = trows;

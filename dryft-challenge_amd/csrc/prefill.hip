@@ -13,41 +13,16 @@ namespace qdec {
 namespace {
 
 // ------------------------------------------------------------------ product
-// A workgroup of 2 x NWM wavefronts computes a (16 NWM XW) x (32 WN) tile of
-// the transposed product D = W . x^T: a weight fragment (16 weight rows x 32
+// The transposed product D = W . x^T: a weight fragment (16 weight rows x 32
 // k) is the A operand and an activation fragment (32 k x 16 rows) the B
 // operand of v_mfma_f32_16x16x32_bf16, and both are one contiguous KiB in
-// their layouts.  Wave (wn, wm) owns WN weight x XW activation fragments.
-// Every fragment moves from global memory straight into LDS
+// their layouts.  Every fragment moves from global memory straight into LDS
 // (global_load_lds_dwordx4: one instruction per 1 KiB fragment, no
-// registers) through a ring of stage buffers, RING - 1 stages in flight
-// while one computes:
-//   256 x 256 (8 waves of WN 8 x XW 4): stages of one k step (32 KiB),
-//     RING 4 -- a third fewer LDS bytes per MFMA than 256 x 128;
-//   256 x 128 (8 waves of WN 4 x XW 4): stages of two k steps (48 KiB),
-//     RING 3 -- twice the workgroups;
-//   64 x 64 (4 waves of WN 2 x XW 2): stages of two k steps (16 KiB),
-//     RING 3 -- for few rows: 8x the workgroups of 256 x 128, several per
-//     CU.
-// Eight waves of half the accumulators (~240 and ~100 registers) run two
-// per SIMD, so one wave's LDS reads overlap another's MFMAs: 5-15% over four
-// waves of twice the tile per wave.
-template <int WN, int XW, int NWM = 2>
-struct PgShape {
-  static constexpr int NW = 2 * NWM;                // waves: 2 along n x NWM along rows
-  static constexpr int Wf = 2 * WN;                 // weight fragments per k step
-  static constexpr int Xf = NWM * XW;               // activation fragments per k step
-  static constexpr int KS = WN == 8 ? 1 : 2;        // k steps per stage
-  static constexpr int RING = WN == 8 ? 4 : 3;      // stage buffers
-  static constexpr int Frags = Wf + Xf;             // fragments per k step
-  static constexpr int Stage = KS * Frags;          // fragments per stage
-  static constexpr int Loads = Stage / NW;          // loads per wave per stage
-  static constexpr int WQ = Wf / NW;                // weight loads per wave per k step
-  static_assert(Wf % NW == 0 && Xf % NW == 0, "each wave loads whole fragments");
-};
+// registers) through a ring of stages, RING - 1 in flight while one computes.
+// Two kernels: pgemm_kernel for tiles of 256 rows (below), and
+// pgemm_small_kernel for few rows: 4 waves of 2 x 2 fragments on 64 x 64
+// tiles, stages of two k steps (16 KiB), three workgroups per CU.
 constexpr int kPgGroupN = 4;  // column tiles walked together (x reuse in L2)
-constexpr int kPg256Xw = 4;   // 256 x 256 and 256 x 128 tiles: activation fragments per wave
-constexpr int kPg128Xw = 4;   //   (4: 8 waves; 8 would be 4 waves of twice the accumulators)
 
 __device__ __forceinline__ uint4 ld16(const uint16_t *p) { return *reinterpret_cast<const uint4 *>(p); }
 
@@ -64,6 +39,13 @@ __device__ __forceinline__ void dma16(const void *g, uint32_t lds_addr) {
       : "=&s"(saved)
       : "v"(g), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
       : "memory");
+}
+// The same from a wave-uniform base and a lane offset, without saving M0
+// (for kernels none of whose other instructions read it).
+__device__ __forceinline__ void dma16s(const char *base, uint32_t lane_off, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :: "v"(lane_off), "s"(base), "s"(lds_addr)
+               : "memory");
 }
 __device__ __forceinline__ uint32_t lds_addr(const void *p) { return (uint32_t)reinterpret_cast<uintptr_t>(p); }
 
@@ -84,57 +66,77 @@ __device__ __forceinline__ float max_xor16_32(float v) {
 constexpr int vmcnt_enc(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 constexpr int kVmcnt0 = vmcnt_enc(0);
 
-template <uint32_t FLAGS, int WN, int XW, int NWM>
-__global__ void __launch_bounds__(128 * NWM, 1) pgemm_kernel(const PgemmParams p) {
-  using S = PgShape<WN, XW, NWM>;
+template <int V>
+struct Int {
+  static constexpr int value = V;
+};
+
+// SwiGLU of one gate / up pair, both already rounded: bf16(silu(g)) * u.
+__device__ __forceinline__ float swiglu(float g, float u) { return rbf(g / (1.0f + expf(-g))) * u; }
+
+// Tiles of 256 rows x (32 WN) columns, eight waves as 2 (columns) x 4 (rows),
+// each WN weight x 4 activation fragments: 256 x 256 (WN 8, 32 KiB stages,
+// RING 5), 256 x 160 (WN 5, 26 KiB, RING 6) and 256 x 128 (WN 4, 24 KiB,
+// RING 6).  One workgroup per CU walks its tiles with the ring running on:
+// the next tile's first stages load while this one ends and stores.
+//
+// What bounds it is the matrix cores' power: at 32K rows the same code runs
+// gate/up at 1310 TFLOP/s on random data and 1650 on zeros.  A step's
+// fragment reads, loads and MFMAs are interleaved by hand (each group of 4
+// MFMAs between scheduling barriers): left to the compiler, the 12 reads
+// came first and the MFMAs of both waves of a SIMD waited together (1150).
+// The loads of a step are spread the same way; PRE groups of MFMAs run
+// ahead of the barrier, so the matrix cores are busy while the waves meet.
+template <int WN>
+struct PgTile {
+  static constexpr int XW = 4, NW = 8;
+  static constexpr int Wf = 2 * WN, Xf = 4 * XW;  // fragments per k step
+  static constexpr int Frags = Wf + Xf;
+  static constexpr int Loads = Frags / NW;        // per wave and k step; waves below LoadsRem one more
+  static constexpr int LoadsRem = Frags % NW;
+  static constexpr int LoadsMax = Loads + (LoadsRem ? 1 : 0);
+  static constexpr int RING = 163840 / (Frags * 1024) > 6 ? 6 : 163840 / (Frags * 1024);
+  static constexpr int PRE = (3 * WN) / 8;        // MFMA groups ahead of the barrier
+};
+
+template <uint32_t FLAGS, int WN>
+__global__ void __launch_bounds__(512, 2) pgemm_kernel(const PgemmParams p) {
+  using S = PgTile<WN>;
   constexpr bool GLU = (FLAGS & QDEC_GLU) != 0;
   constexpr bool RES = (FLAGS & QDEC_RES_OUT) != 0;
-  __shared__ uint4 lds[S::RING * S::Stage * 64];  // [ring slot][k step][fragment][lane]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int XW = S::XW, RING = S::RING;
+  static_assert(!GLU || WN % 2 == 0, "gate and up fragments pair up within a wave");
+  __shared__ uint4 lds[RING * S::Frags * 64];  // [ring slot][fragment][lane]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
   const int wn = wave & 1, wm = wave >> 1;
+  const int KS = p.k >> 5;  // even
 
   // Tile order: workgroup i runs on XCD i % 8, so each XCD gets a contiguous
-  // range of the sequence; the sequence walks groups of kPgGroupN column
-  // tiles across all row tiles (the group's weights stay in L2, each row
-  // tile of x is read by the group's workgroups together).
-  int id = blockIdx.x;
-  const int G = gridDim.x;
-  if ((G & 7) == 0) id = (id & 7) * (G >> 3) + (id >> 3);
-  const int ntm = p.tiles / S::Xf;
-  const int gsz = kPgGroupN * ntm;
-  const int g = id / gsz, r = id - g * gsz;
-  const int gn = min(kPgGroupN, p.wg_n - g * kPgGroupN);
-  const int tm = r / gn, tn = g * kPgGroupN + (r - (r / gn) * gn);
-
-  const int KS = p.k >> 5;
+  // range of the sequence, dealt to its workgroups in turn; the sequence
+  // walks groups of kPgGroupN column tiles across all row tiles (the group's
+  // weights stay in L2, each row tile of x is read by the group's workgroups
+  // together).
+  const int ntm = p.tiles / S::Xf, T = ntm * p.wg_n;
+  const int nx = min(8, (int)gridDim.x), xcd = blockIdx.x & 7;
+  const int seq_end = (int)((int64_t)T * (xcd + 1) / nx);
+  const int per = ((int)gridDim.x + 7 - xcd) >> 3;  // workgroups on this XCD
+  int seq = (int)((int64_t)T * xcd / nx) + (blockIdx.x >> 3);
+  if (seq >= seq_end) return;
+  auto place = [&](int id, int &tm, int &tn) {
+    const int gsz = kPgGroupN * ntm;
+    const int g = id / gsz, r = id - g * gsz;
+    const int gn = min(kPgGroupN, p.wg_n - g * kPgGroupN);
+    tm = r / gn;
+    tn = g * kPgGroupN + (r - tm * gn);
+  };
   // Weight tile of workgroup fragment f (GLU: WN gate tiles, then the WN
   // matching up tiles).
-  auto wtile = [&](int f) -> int {
+  auto wtile = [&](int tn, int f) -> int {
     if constexpr (GLU)
       return f < WN ? tn * WN + f : p.up_tiles + tn * WN + f - WN;
     else
       return tn * S::Wf + f;
-  };
-  // Loads of one k step: this wave moves fragments wave + NW q (q < WQ:
-  // weights, then activations).
-  const uint16_t *wb[S::WQ];
-#pragma unroll
-  for (int q = 0; q < S::WQ; ++q) wb[q] = p.w + (size_t)wtile(wave + S::NW * q) * KS * 512 + lane * 8;
-  const uint16_t *xb = p.x + (size_t)(tm * S::Xf + wave) * 512 + lane * 8;
-  const size_t xks = (size_t)p.tiles * 512;  // elements per k step of x
-  const uint32_t lds0 = lds_addr(lds);
-  auto dma = [&](int s, int slot) {
-#pragma unroll
-    for (int j = 0; j < S::KS; ++j) {
-      const int ks = s * S::KS + j;
-      const uint32_t dst = lds0 + (uint32_t)(((slot * S::KS + j) * S::Frags + wave) * 1024);
-#pragma unroll
-      for (int q = 0; q < S::WQ; ++q) dma16(wb[q] + (size_t)ks * 512, dst + q * S::NW * 1024);
-#pragma unroll
-      for (int q = 0; q < S::Xf / S::NW; ++q)
-        dma16(xb + ks * xks + q * S::NW * 512, dst + (S::WQ + q) * S::NW * 1024);
-    }
   };
   // This wave's weight fragments (GLU: gate i pairs with up i + WN/2).
   auto wf = [&](int i) -> int {
@@ -144,120 +146,288 @@ __global__ void __launch_bounds__(128 * NWM, 1) pgemm_kernel(const PgemmParams p
       return wn * WN + i;
   };
 
+  // Loads: wave w moves fragments w + 8 q of every k step (weights first).
+  // The load cursor (lseq, lk) runs RING - 1 stages ahead of the compute;
+  // past this workgroup's last tile it loads that tile's stages again, which
+  // nothing reads.
+  const bool hi = wave < S::LoadsRem;
+  const size_t xks = (size_t)p.tiles * 1024;  // bytes per k step of x
+  const uint32_t voff = lane * 16, lds0 = lds_addr(lds);
+  const char *src[S::LoadsMax];
+  auto aim = [&](int id) {
+    int tm, tn;
+    place(id, tm, tn);
+#pragma unroll
+    for (int q = 0; q < S::LoadsMax; ++q) {
+      const int f = min(wave + S::NW * q, S::Frags - 1);
+      src[q] = f < S::Wf ? reinterpret_cast<const char *>(p.w) + (size_t)wtile(tn, f) * KS * 1024
+                         : reinterpret_cast<const char *>(p.x) + (size_t)(tm * S::Xf + f - S::Wf) * 1024;
+    }
+  };
+  auto load = [&](int q, uint32_t slot_base) {
+    const int f = wave + S::NW * q;
+    dma16s(src[q], voff, slot_base + f * 1024);
+    src[q] += f < S::Wf ? (size_t)1024 : xks;
+  };
+  int lseq = seq, lk = 0;
+  aim(seq);
+  auto next_pair = [&]() {  // before the loads of stages lk and lk + 1
+    if (lk == KS) {
+      lk = 0;
+      if (lseq + per < seq_end) lseq += per;
+      aim(lseq);
+    }
+    lk += 2;
+  };
+#pragma unroll
+  for (int st = 0; st < RING - 1; ++st) {
+    if (st % 2 == 0) next_pair();
+#pragma unroll
+    for (int q = 0; q < S::LoadsMax; ++q)
+      if (q < S::Loads || hi) load(q, lds0 + st * S::Frags * 1024);
+  }
+  // Waits until at most `stages` whole stages of this wave's loads (and
+  // `after` younger stores) are outstanding.
+  auto wait_stages = [&](auto stages, auto after) {
+    constexpr int n = decltype(stages)::value * S::Loads + decltype(after)::value;
+    constexpr int nh = n + decltype(stages)::value;
+    static_assert(nh <= 63, "vmcnt");
+    if (S::LoadsRem != 0 && hi)
+      __builtin_amdgcn_s_waitcnt(vmcnt_enc(nh));
+    else
+      __builtin_amdgcn_s_waitcnt(vmcnt_enc(n));
+  };
+  wait_stages(Int<RING - 2>{}, Int<0>{});
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+
   f32x4_t acc[WN][XW];
+  auto clear = [&]() {
 #pragma unroll
-  for (int i = 0; i < WN; ++i)
+    for (int i = 0; i < WN; ++i)
 #pragma unroll
-    for (int q = 0; q < XW; ++q) acc[i][q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int q = 0; q < XW; ++q) acc[i][q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
+  // Two register sets of fragments: step t + 1's are read while step t's
+  // MFMAs run.
+  uint4 a[2][WN], b[2][XW];
+#pragma unroll
+  for (int q = 0; q < XW; ++q) b[0][q] = lds[(S::Wf + wm * XW + q) * 64 + lane];
+#pragma unroll
+  for (int i = 0; i < WN; ++i) a[0][i] = lds[wf(i) * 64 + lane];
+  int rslot = 1, fslot = RING - 1;  // ring slots read and filled next
+  bool stored = false;              // the last tile's stores are younger than the stages waited for
 
-  if constexpr (WN == 8) {
-    // 256 x 256 tiles (one k step per stage): the next step's fragments are
-    // read while this step multiplies (+5-10% there; the other tiles, two
-    // steps per stage, measured slower with it and read each step's
-    // fragments right before its MFMAs).
-    // k steps run through two register sets of fragments: the fragments of
-    // step t+1 are read from LDS while step t's MFMAs run.  Entering a new
-    // stage (before reading its first step) waits for this wave's loads of
-    // it, then a barrier makes every wave's visible and frees the slot of the
-    // stage before it -- all of whose steps are already in registers -- for
-    // the stage RING - 1 ahead.
-    const int nst = p.k / (32 * S::KS);
-    const int nsteps = nst * S::KS;
-    auto slot_of = [&](int st) { return st % S::RING; };
-    auto enter_stage = [&](int st) {
-      const int younger = min(S::RING - 2, nst - 1 - st);
-      if (younger >= 2)
-        __builtin_amdgcn_s_waitcnt(vmcnt_enc(2 * S::Loads));
-      else if (younger == 1)
-        __builtin_amdgcn_s_waitcnt(vmcnt_enc(S::Loads));
-      else
-        __builtin_amdgcn_s_waitcnt(kVmcnt0);
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      if (st + S::RING - 1 < nst) dma(st + S::RING - 1, slot_of(st + S::RING - 1));
+  // One k step: the MFMAs of the fragments in set `cur`; behind PRE groups of
+  // them the barrier that makes stage t + 1 visible and frees the slot of
+  // stage t - 1 (all of whose fragments are in registers) for the loads.
+  constexpr int kStores = GLU ? WN * XW / 2 : WN * XW;
+  auto step = [&](auto curc) {
+    constexpr int cur = decltype(curc)::value, nx = cur ^ 1;
+    auto mma = [&](int i) {
+#pragma unroll
+      for (int q = 0; q < XW; ++q) acc[i][q] = mfma16x16x32(a[cur][i], b[cur][q], acc[i][q]);
     };
-    auto read_frags = [&](int t, uint4 (&a)[WN], uint4 (&bx)[XW]) {
-      const uint4 *L = lds + (size_t)(slot_of(t / S::KS) * S::KS + t % S::KS) * S::Frags * 64 + lane;
-  #pragma unroll
-      for (int i = 0; i < WN; ++i) a[i] = L[wf(i) * 64];
-  #pragma unroll
-      for (int q = 0; q < XW; ++q) bx[q] = L[(S::Wf + wm * XW + q) * 64];
-    };
-    auto mma = [&](const uint4 (&a)[WN], const uint4 (&bx)[XW]) {
-  #pragma unroll
-      for (int i = 0; i < WN; ++i)
-  #pragma unroll
-        for (int q = 0; q < XW; ++q) acc[i][q] = mfma16x16x32(a[i], bx[q], acc[i][q]);
-    };
-    // One step: prepare step t+1 into (na, nb), multiply step t from (ca, cb).
-    auto step = [&](int t, const uint4 (&ca)[WN], const uint4 (&cb)[XW], uint4 (&na)[WN], uint4 (&nb)[XW]) {
-      const int tn = t + 1;
-      if (tn < nsteps) {
-        if (tn % S::KS == 0) enter_stage(tn / S::KS);
-        read_frags(tn, na, nb);
+#pragma unroll
+    for (int i = 0; i < S::PRE; ++i) mma(i);
+    __builtin_amdgcn_sched_barrier(0);
+    if (stored)
+      wait_stages(Int<RING - 3>{}, Int<kStores>{});
+    else
+      wait_stages(Int<RING - 3>{}, Int<0>{});
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint4 *L = lds + rslot * S::Frags * 64 + lane;
+    const uint32_t fill = lds0 + fslot * S::Frags * 1024;
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int REM = WN - S::PRE, RD = XW + WN;
+#pragma unroll
+    for (int i = S::PRE; i < WN; ++i) {
+      const int j = i - S::PRE;
+      const int r0 = (RD * j + REM - 1) / REM, r1 = (RD * (j + 1) + REM - 1) / REM;
+      const int d0 = (S::Loads * j + REM - 1) / REM, d1 = (S::Loads * (j + 1) + REM - 1) / REM;
+#pragma unroll
+      for (int r = r0; r < r1; ++r) {
+        if (r < XW)
+          b[nx][r] = L[(S::Wf + wm * XW + r) * 64];
+        else
+          a[nx][r - XW] = L[wf(r - XW) * 64];
       }
-      mma(ca, cb);
-    };
+#pragma unroll
+      for (int q = d0; q < d1; ++q) load(q, fill);
+      if (i == WN - 1 && S::LoadsRem != 0 && hi) load(S::Loads, fill);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    rslot = rslot + 1 == RING ? 0 : rslot + 1;
+    fslot = fslot + 1 == RING ? 0 : fslot + 1;
+  };
 
-  #pragma unroll
-    for (int st = 0; st < S::RING - 1; ++st)
-      if (st < nst) dma(st, st);
-    uint4 a0[WN], b0[XW], a1[WN], b1[XW];
-    // stage 0 (younger stages in flight as inside the loop)
-    {
-      const int younger = min(S::RING - 2, nst - 1);
-      if (younger >= 2)
-        __builtin_amdgcn_s_waitcnt(vmcnt_enc(2 * S::Loads));
-      else if (younger == 1)
-        __builtin_amdgcn_s_waitcnt(vmcnt_enc(S::Loads));
-      else
-        __builtin_amdgcn_s_waitcnt(kVmcnt0);
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      if (S::RING - 1 < nst) dma(S::RING - 1, S::RING - 1);
+  for (;;) {
+    for (int t = 0; t < KS; t += 2) {
+      if (RING & 1) next_pair();
+      step(Int<0>{});
+      if (!(RING & 1)) next_pair();
+      step(Int<1>{});
+      stored = false;
     }
-    read_frags(0, a0, b0);
-    int t = 0;
-    for (; t + 1 < nsteps; t += 2) {
-      step(t, a0, b0, a1, b1);
-      step(t + 1, a1, b1, a0, b0);
-    }
-    if (t < nsteps) mma(a0, b0);
-  } else {
-    const int nst = p.k / (32 * S::KS);
-  #pragma unroll
-    for (int s = 0; s < S::RING - 1; ++s)
-      if (s < nst) dma(s, s);
-    int slot = 0;
-    for (int s = 0; s < nst; ++s) {
-      // this wave's loads of stage s are done once at most the younger
-      // stages' are outstanding; the barrier makes every wave's visible and
-      // frees the slot of stage s-1 for stage s + RING - 1
-      const int younger = min(S::RING - 2, nst - 1 - s);
-      if (younger >= 2)
-        __builtin_amdgcn_s_waitcnt(vmcnt_enc(2 * S::Loads));
-      else if (younger == 1)
-        __builtin_amdgcn_s_waitcnt(vmcnt_enc(S::Loads));
-      else
-        __builtin_amdgcn_s_waitcnt(kVmcnt0);
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      if (s + S::RING - 1 < nst) dma(s + S::RING - 1, slot == 0 ? S::RING - 1 : slot - 1);
-  #pragma unroll
-      for (int j = 0; j < S::KS; ++j) {
-        const uint4 *L = lds + (size_t)(slot * S::KS + j) * S::Frags * 64 + lane;
-        uint4 a[WN], bx[XW];
-  #pragma unroll
-        for (int i = 0; i < WN; ++i) a[i] = L[wf(i) * 64];
-  #pragma unroll
-        for (int q = 0; q < XW; ++q) bx[q] = L[(S::Wf + wm * XW + q) * 64];
-  #pragma unroll
-        for (int i = 0; i < WN; ++i)
-  #pragma unroll
-          for (int q = 0; q < XW; ++q) acc[i][q] = mfma16x16x32(a[i], bx[q], acc[i][q]);
+    // Epilogue: lane holds columns n0 .. n0+3 of row m for every fragment
+    // pair.  A tile whose rows are all real stores through inline assembly,
+    // so the number of stores the next tile's first waits let pass is known.
+    int tm, tn;
+    place(seq, tm, tn);
+    auto residual = [&](int m, int n0) -> uint2 {
+      if constexpr (RES) return *reinterpret_cast<const uint2 *>(p.res + (size_t)m * p.n_out + n0);
+      return make_uint2(0u, 0u);
+    };
+    auto value = [&](int i, int q, uint2 rv) -> uint2 {
+      if constexpr (GLU) {
+        float o4[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o4[e] = swiglu(rbf(acc[i][q][e]), rbf(acc[i + WN / 2][q][e]));
+        return make_uint2(pack2(o4[0], o4[1]), pack2(o4[2], o4[3]));
+      } else if constexpr (RES) {
+        return make_uint2(pack2(lo16(rv.x) + rbf(acc[i][q][0]), hi16(rv.x) + rbf(acc[i][q][1])),
+                          pack2(lo16(rv.y) + rbf(acc[i][q][2]), hi16(rv.y) + rbf(acc[i][q][3])));
+      } else {
+        return make_uint2(pack2(acc[i][q][0], acc[i][q][1]), pack2(acc[i][q][2], acc[i][q][3]));
       }
-      slot = slot == S::RING - 1 ? 0 : slot + 1;
+    };
+    auto dst = [&](int m, int n0) -> uint16_t * {
+      return p.ofrag ? p.out + frag_off(m, n0, p.tiles) : p.out + (size_t)m * p.n_out + n0;
+    };
+    constexpr int NI = GLU ? WN / 2 : WN;
+    const int m_base = (tm * S::Xf + wm * XW) * 16 + col;
+    if ((tm + 1) * S::Xf * 16 <= p.rows) {
+#pragma unroll
+      for (int q0 = 0; q0 < XW; q0 += 2) {
+        uint2 rv[2][NI];  // residuals of two row fragments, loaded together
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < NI; ++i) rv[u][i] = residual(m_base + (q0 + u) * 16, wtile(tn, wf(i)) * 16 + 4 * grp);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            const int m = m_base + (q0 + u) * 16, n0 = wtile(tn, wf(i)) * 16 + 4 * grp;
+            const uint2 o = value(i, q0 + u, rv[u][i]);
+            asm volatile("global_store_dwordx2 %0, %1, off" ::"v"(dst(m, n0)), "v"(__builtin_bit_cast(uint64_t, o))
+                         : "memory");
+          }
+      }
+      stored = true;
+    } else {
+#pragma unroll
+      for (int q = 0; q < XW; ++q) {
+        const int m = m_base + q * 16;
+        if (m >= p.rows) continue;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const int n0 = wtile(tn, wf(i)) * 16 + 4 * grp;
+          *reinterpret_cast<uint2 *>(dst(m, n0)) = value(i, q, residual(m, n0));
+        }
+      }
     }
+    seq += per;
+    if (seq >= seq_end) break;
+    clear();
+  }
+  // The loads past the last tile still write this workgroup's LDS.
+  __builtin_amdgcn_s_waitcnt(kVmcnt0);
+}
+
+// ---- few rows
+constexpr int kPsFrags = 4 + 4;           // weight + activation fragments per k step
+constexpr int kPsSteps = 2, kPsRing = 3;  // k steps per stage, stage buffers
+constexpr int kPsStage = kPsSteps * kPsFrags;
+constexpr int kPsLoads = kPsStage / 4;    // loads per wave per stage
+
+template <uint32_t FLAGS>
+__global__ void __launch_bounds__(256, 1) pgemm_small_kernel(const PgemmParams p) {
+  constexpr bool GLU = (FLAGS & QDEC_GLU) != 0;
+  constexpr bool RES = (FLAGS & QDEC_RES_OUT) != 0;
+  __shared__ uint4 lds[kPsRing * kPsStage * 64];  // [ring slot][k step][fragment][lane]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, grp = lane >> 4;
+  const int wn = wave & 1, wm = wave >> 1;
+
+  // Tile order as in pgemm_kernel, one tile per workgroup.
+  int id = blockIdx.x;
+  const int G = gridDim.x;
+  if ((G & 7) == 0) id = (id & 7) * (G >> 3) + (id >> 3);
+  const int ntm = p.tiles / 4;
+  const int gsz = kPgGroupN * ntm;
+  const int g = id / gsz, r = id - g * gsz;
+  const int gn = min(kPgGroupN, p.wg_n - g * kPgGroupN);
+  const int tm = r / gn, tn = g * kPgGroupN + (r - (r / gn) * gn);
+
+  const int KS = p.k >> 5;
+  auto wtile = [&](int f) -> int {
+    if constexpr (GLU)
+      return f < 2 ? tn * 2 + f : p.up_tiles + tn * 2 + f - 2;
+    else
+      return tn * 4 + f;
+  };
+  const uint16_t *wb = p.w + (size_t)wtile(wave) * KS * 512 + lane * 8;
+  const uint16_t *xb = p.x + (size_t)(tm * 4 + wave) * 512 + lane * 8;
+  const size_t xks = (size_t)p.tiles * 512;  // elements per k step of x
+  const uint32_t lds0 = lds_addr(lds);
+  auto dma = [&](int s, int slot) {
+#pragma unroll
+    for (int j = 0; j < kPsSteps; ++j) {
+      const int ks = s * kPsSteps + j;
+      const uint32_t dst = lds0 + (uint32_t)(((slot * kPsSteps + j) * kPsFrags + wave) * 1024);
+      dma16(wb + (size_t)ks * 512, dst);
+      dma16(xb + ks * xks, dst + 4 * 1024);
+    }
+  };
+  // This wave's weight fragments (GLU: gate 0 pairs with up 1).
+  auto wf = [&](int i) -> int {
+    if constexpr (GLU)
+      return i < 1 ? wn + i : 2 + wn + i - 1;
+    else
+      return wn * 2 + i;
+  };
+
+  f32x4_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) acc[i][q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int nst = p.k / (32 * kPsSteps);
+#pragma unroll
+  for (int s = 0; s < kPsRing - 1; ++s)
+    if (s < nst) dma(s, s);
+  int slot = 0;
+  for (int s = 0; s < nst; ++s) {
+    // this wave's loads of stage s are done once at most the younger stage's
+    // are outstanding; the barrier makes every wave's visible and frees the
+    // slot of stage s-1 for stage s + 2
+    if (s + 1 < nst)
+      __builtin_amdgcn_s_waitcnt(vmcnt_enc(kPsLoads));
+    else
+      __builtin_amdgcn_s_waitcnt(kVmcnt0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + kPsRing - 1 < nst) dma(s + kPsRing - 1, slot == 0 ? kPsRing - 1 : slot - 1);
+#pragma unroll
+    for (int j = 0; j < kPsSteps; ++j) {
+      const uint4 *L = lds + (size_t)(slot * kPsSteps + j) * kPsFrags * 64 + lane;
+      uint4 a[2], bx[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) a[i] = L[wf(i) * 64];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) bx[q] = L[(4 + wm * 2 + q) * 64];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[i][q] = mfma16x16x32(a[i], bx[q], acc[i][q]);
+    }
+    slot = slot == kPsRing - 1 ? 0 : slot + 1;
   }
 
   // Epilogue: lane holds columns n0 .. n0+3 of row m for every fragment pair.
@@ -265,26 +435,19 @@ __global__ void __launch_bounds__(128 * NWM, 1) pgemm_kernel(const PgemmParams p
     uint16_t *dst = p.ofrag ? p.out + frag_off(m, n0, p.tiles) : p.out + (size_t)m * p.n_out + n0;
     *reinterpret_cast<uint2 *>(dst) = o;
   };
-  const int m_base = (tm * S::Xf + wm * XW) * 16 + col;
+  const int m_base = (tm * 4 + wm * 2) * 16 + col;
 #pragma unroll
-  for (int q = 0; q < XW; ++q) {
+  for (int q = 0; q < 2; ++q) {
     const int m = m_base + q * 16;
     if (m >= p.rows) continue;
     if constexpr (GLU) {
+      float o4[4];
 #pragma unroll
-      for (int i = 0; i < WN / 2; ++i) {
-        float o4[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float gv = rbf(acc[i][q][e]);
-          const float uv = rbf(acc[i + WN / 2][q][e]);
-          o4[e] = rbf(gv / (1.0f + expf(-gv))) * uv;
-        }
-        store(m, wtile(wf(i)) * 16 + 4 * grp, make_uint2(pack2(o4[0], o4[1]), pack2(o4[2], o4[3])));
-      }
+      for (int e = 0; e < 4; ++e) o4[e] = swiglu(rbf(acc[0][q][e]), rbf(acc[1][q][e]));
+      store(m, wtile(wf(0)) * 16 + 4 * grp, make_uint2(pack2(o4[0], o4[1]), pack2(o4[2], o4[3])));
     } else {
 #pragma unroll
-      for (int i = 0; i < WN; ++i) {
+      for (int i = 0; i < 2; ++i) {
         const int n0 = wtile(wf(i)) * 16 + 4 * grp;
         uint2 o;
         if constexpr (RES) {
@@ -714,22 +877,43 @@ __global__ void __launch_bounds__(64 * G * pa_wph(G), 1) pattn_kernel(const Patt
 
 }  // namespace
 
-template <int WN, int XW, int NWM>
+namespace {
+template <int WN>
 hipError_t launch_pgemm_tile(const PgemmParams &p, uint32_t flags, hipStream_t s) {
-  const dim3 grid(p.wg_n * (p.tiles / PgShape<WN, XW, NWM>::Xf)), block(128 * NWM);
+  const int T = p.wg_n * (p.tiles / PgTile<WN>::Xf);
+  const dim3 grid(T < kPgWorkgroups ? T : kPgWorkgroups), block(512);
   switch (flags) {
-    case 0u: hipLaunchKernelGGL((pgemm_kernel<0u, WN, XW, NWM>), grid, block, 0, s, p); break;
-    case QDEC_RES_OUT: hipLaunchKernelGGL((pgemm_kernel<QDEC_RES_OUT, WN, XW, NWM>), grid, block, 0, s, p); break;
-    case QDEC_GLU: hipLaunchKernelGGL((pgemm_kernel<QDEC_GLU, WN, XW, NWM>), grid, block, 0, s, p); break;
+    case 0u: hipLaunchKernelGGL((pgemm_kernel<0u, WN>), grid, block, 0, s, p); return hipSuccess;
+    case QDEC_RES_OUT: hipLaunchKernelGGL((pgemm_kernel<QDEC_RES_OUT, WN>), grid, block, 0, s, p); return hipSuccess;
+    case QDEC_GLU:
+      if constexpr (WN % 2 == 0) {
+        hipLaunchKernelGGL((pgemm_kernel<QDEC_GLU, WN>), grid, block, 0, s, p);
+        return hipSuccess;
+      }
+      return hipErrorInvalidValue;
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_pgemm_small(const PgemmParams &p, uint32_t flags, hipStream_t s) {
+  const dim3 grid(p.wg_n * (p.tiles / 4)), block(256);
+  switch (flags) {
+    case 0u: hipLaunchKernelGGL(pgemm_small_kernel<0u>, grid, block, 0, s, p); break;
+    case QDEC_RES_OUT: hipLaunchKernelGGL(pgemm_small_kernel<QDEC_RES_OUT>, grid, block, 0, s, p); break;
+    case QDEC_GLU: hipLaunchKernelGGL(pgemm_small_kernel<QDEC_GLU>, grid, block, 0, s, p); break;
     default: return hipErrorInvalidValue;
   }
   return hipSuccess;
 }
+}  // namespace
 
 hipError_t launch_pgemm(const PgemmParams &p, uint32_t flags, hipStream_t s) {
-  if (p.tile_rows == 64) return launch_pgemm_tile<2, 2, 2>(p, flags, s);
-  return p.tile_cols == 256 ? launch_pgemm_tile<8, kPg256Xw, 256 / (16 * kPg256Xw)>(p, flags, s)
-                            : launch_pgemm_tile<4, kPg128Xw, 256 / (16 * kPg128Xw)>(p, flags, s);
+  if (p.tile_rows == 64) return launch_pgemm_small(p, flags, s);
+  switch (p.tile_cols) {
+    case 256: return launch_pgemm_tile<8>(p, flags, s);
+    case 160: return launch_pgemm_tile<5>(p, flags, s);
+    default: return launch_pgemm_tile<4>(p, flags, s);
+  }
 }
 
 // Grouped row kernels from this many rows (below it one workgroup per row

@@ -190,13 +190,15 @@ size_t layer_attn_lds_bytes();
 
 // ---- prefill (prefill.hip)
 // Product tiles of a workgroup (activation rows x weight rows): 256 x 128,
-// 256 x 256 or 64 x 64; k a multiple of kPgStageK; the activation buffers
+// 256 x 160, 256 x 256 or 64 x 64; k a multiple of kPgStageK; the activation buffers
 // hold whole row tiles of the tile used: kPgRows rows, or kPgRowsSmall with
 // the 64 x 64 tile (the only one a call of fewer whole kPgRows tiles takes).
 constexpr int kPqMaxHeads = 80;  // query + key heads per row of qdec_prefill_qk (Qwen3-32B: 72)
 constexpr int kPgRows = 256;
 constexpr int kPgRowsSmall = 64;
 constexpr int kPgStageK = 64;
+// Workgroups of the 256-row tiles: one per CU, each walking its share of them.
+constexpr int kPgWorkgroups = 256;
 struct PgemmParams {
   const uint16_t *x;
   const uint16_t *w;
@@ -208,7 +210,7 @@ struct PgemmParams {
   int n_out;     // columns of out (n, or n/2 with GLU)
   int up_tiles;  // GLU: tile offset of the up half (n/32)
   int tile_rows; // activation rows per workgroup tile: 256 or 64
-  int tile_cols; // weight rows per workgroup tile: 128 or 256 (64 with 64 rows)
+  int tile_cols; // weight rows per workgroup tile: 128, 160 or 256 (64 with 64 rows)
   int wg_n;      // workgroup tiles along n
 };
 hipError_t launch_pgemm(const PgemmParams &p, uint32_t flags, hipStream_t s);

@@ -265,3 +265,28 @@ def test_prefill_qk_and_attention_vs_oracle(lib, B, T, pos0, cap):
     assert torch.isfinite(out).all()
     err = (out - ref).abs().max().item()
     assert err <= 0.02 * ref.abs().max().item(), err
+
+
+# The 256-row tiles run as one workgroup per CU walking several tiles: more
+# tiles than workgroups (a last round that is not full), fewer than eight
+# (fewer workgroups than XCDs), row counts that leave the last row tile
+# ragged, k of one and of an odd number of load rings, and 256 x 160 tiles
+# (picked for n = 2560 at 4096 rows), against the 64 x 64 tile bit for bit
+# (the tile changes no sum).
+@pytest.mark.parametrize("rows,n,k,tile", [
+    (256, 256, 64, (256, 256)), (300, 768, 64, (256, 128)), (513, 256, 704, (256, 256)),
+    (4096, 2560, 320, (0, 0)), (3900, 2560, 64, (0, 0)), (4100, 5120, 192, (256, 256)), (8192, 2560, 128, (256, 128)),
+])
+def test_prefill_gemm_walked_tiles_bitexact(lib, rows, n, k, tile):
+    from qdec import capi
+    x, w = rnd(rows, k, seed=rows + k), rnd(n, k, scale=0.05, seed=n + k)
+    tiles = round_up(rows, ROW_TILE) // 16
+    xf, wp, res = to_frag(lib, x, tiles), pack(lib, w), rnd(rows, n, seed=9)
+    for flags, frag in ((0, 0), (0, 1), (capi.RES_OUT, 0), (capi.GLU, 1), (capi.GLU, 0)):
+        kw = dict(flags=flags, res=res, out_frag=frag)
+        got = pgemm(lib, xf, wp, rows, n, k, tiles, tile=tile, **kw)
+        want = pgemm(lib, xf, wp, rows, n, k, tiles, tile=(64, 64), **kw)
+        if frag:
+            cols = n // 2 if flags == capi.GLU else n
+            got, want = frag_to_rows(got, rows, cols, tiles), frag_to_rows(want, rows, cols, tiles)
+        assert torch.equal(got, want), (flags, frag)
