@@ -49,6 +49,14 @@ __device__ __forceinline__ void dma16s(const char *base, uint32_t lane_off, uint
 }
 __device__ __forceinline__ uint32_t lds_addr(const void *p) { return (uint32_t)reinterpret_cast<uintptr_t>(p); }
 
+// Keeps the computation of v where it stands among other pins and volatile
+// assembly (the compiler moves plain arithmetic and MFMAs past scheduling
+// barriers before it schedules).
+template <class V>
+__device__ __forceinline__ void pin(V &v) {
+  asm volatile("" : "+v"(v));
+}
+
 // Maximum of v over the lane pairs (l, l ^ 16) and then (l, l ^ 32), with
 // gfx950's row swaps instead of LDS permutes: after v_permlane16_swap the two
 // outputs hold the odd / even 16-lane rows exchanged, after
@@ -639,46 +647,51 @@ __global__ void __launch_bounds__(256) pnorm_kernel(const uint16_t *__restrict__
 
 // ---------------------------------------------------------------- attention
 // A workgroup takes kPaRows positions of G = 2 or 4 query heads of one kv
-// head of one sequence; wave w takes head w % G of them and its share of
-// the positions, 2 M tiles of 16 rows (two waves per head: 4 or 8 waves).
-// Eight query heads per kv head run as two such workgroups.  Blocks of 32 cache slots
+// head of one sequence; wave w takes head w % G of them and half of the
+// positions, 2 M tiles of 16 rows (4 or 8 waves).  Blocks of 32 cache slots
 // go from global memory straight into LDS (global_load_lds_dwordx4 with
 // per-lane gather addresses, so every fragment lands in MFMA operand
-// order), three blocks in a ring, two ahead of the compute, shared by the
-// waves:
+// order), kPaRing blocks in a ring shared by the waves:
 //   K fragment (s, h): lane (c, g) holds slot 8*(c >> 2) + (c & 3) + 4h,
 //     channels 32s + 8g .. +8: the slot order that makes the score registers
 //     of S^T = K . Q^T exactly the B operand of O^T += V^T . P^T (each lane
 //     ends up with 8 consecutive slots of one query row);
 //   V fragment dt: lane (c, g) holds channel 16dt + c, slots 8g .. 8g+7 --
 //     16 contiguous bytes of the channel-major cache.
+// The loop is pipelined by hand: while block j's softmax runs on the vector
+// units, the matrix cores form block j + 1's scores (one MFMA every few
+// vector instructions), and block j's P.V product covers the LDS reads of
+// block j + 2's keys.  Before that every wave of a workgroup met at the
+// block's barrier, multiplied, then exponentiated, so the two units took
+// turns: 8 x 1024 rows after 3072 cached slots 572 -> 512 us (840 -> 940
+// TFLOP/s), and two heads per kv head, alone 540 -> 326 us.  What bounds it
+// now is shared: LDS reads (a wave's 32 rows take every K/V fragment for two
+// MFMAs), the vector units and the matrix cores each cost about a fifth of
+// the time when left out.
 // Online softmax in base 2 with fp32 state per row (running max kept in
 // score units, exp2(s * scale - m * scale) as one FMA), probabilities rounded
-// to bf16 for the P.V product, two tiles at a time in straight-line code
-// (independent MFMA chains and softmaxes interleave).  Only blocks that
-// cross some row's position are masked; the accumulators are rescaled only
-// when some row's max moved.
-// Slots past the block's last row are zeroed in V after the LDS read (the
-// cache may hold anything there, and 0 * NaN would poison the product).
+// to bf16 for the P.V product.  Each lane compares its own scores with the
+// running maximum; the cross-lane maximum and the rescaling of the
+// accumulators run only for a tile some row's maximum moves in.
+// Only blocks that cross some row's position are masked.  Slots past the
+// block's last row are zeroed in V after the LDS read (the cache may hold
+// anything there, and 0 * NaN would poison the product).
 constexpr int kPaKFrags = 8, kPaVFrags = 8;
 constexpr int kPaBlockVec = (kPaKFrags + kPaVFrags) * 64;  // uint4 per staged block
-constexpr int kPaRing = 3;
-// Waves per query head: two, each taking 2 M tiles (a workgroup of G = 2
-// or 4 query heads has 4 or 8 waves).
-constexpr int pa_wph(int G) { return 2; }
+constexpr int kPaRing = 4;
+// Waves per query head: two, each taking 2 M tiles.
+constexpr int kPaWph = 2;
 
-// G query heads per workgroup out of GS per kv head: GS = 8 (Qwen3-32B's
-// layout) runs as two workgroups of 4 heads per (kv head, row block), each
-// reading the kv head's K/V (8 heads in one workgroup would need 64
-// accumulator rows per wave and spill).
-template <int G, int GS = G>
-__global__ void __launch_bounds__(64 * G * pa_wph(G), 1) pattn_kernel(const PattnParams p) {
+// G query heads per workgroup out of GS per kv head: GS / G workgroups per
+// (kv head, row block), each reading the kv head's K/V (8 heads in one
+// workgroup would need 64 accumulator rows per wave and spill).
+template <int G, int GS>
+__global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnParams p) {
   constexpr int D = 128;
-  constexpr int WPH = pa_wph(G);
-  constexpr int MT = 4 / WPH;                  // M tiles of 16 positions per wave
-  constexpr int NWV = G * WPH;                 // waves
+  constexpr int MT = 4 / kPaWph;               // M tiles of 16 positions per wave
+  constexpr int NWV = G * kPaWph;              // waves
   constexpr int NSUB = GS / G;                 // workgroups per (kv head, row block)
-  static_assert(MT % 2 == 0 && (G == 2 || G == 4) && GS % G == 0, "tiles taken in pairs; 2 or 4 heads");
+  static_assert(MT == 2 && GS % G == 0 && 16 % NWV == 0, "two tiles per wave; whole fragments per wave");
   constexpr int FPW = (kPaKFrags + kPaVFrags) / NWV;  // fragments each wave loads per block
   __shared__ uint4 lds[kPaRing * kPaBlockVec];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -718,14 +731,14 @@ __global__ void __launch_bounds__(64 * G * pa_wph(G), 1) pattn_kernel(const Patt
     for (int s = 0; s < 4; ++s) qf[mt][s] = valid ? ld16(qrow + s * 32) : zero4();
   }
 
-  // Block j into ring slot `slot`: this wave gathers K fragments wave + NWV*i
+  // Block j into its ring slot: this wave gathers K fragments wave + NWV*i
   // (index 2s + h) and V fragments wave + NWV*i.
   const uint32_t lds0 = lds_addr(lds);
   const uint16_t *kg = kc + (size_t)(8 * (col >> 2) + (col & 3)) * D + 8 * grp;
   const uint16_t *vg = vc + (size_t)grp * D * 8 + col * 8;
-  auto dma_block = [&](int j, int slot) {
+  auto dma_block = [&](int j) {
     const int s0 = j * 32;
-    const uint32_t base = lds0 + (uint32_t)(slot * kPaBlockVec * 16);
+    const uint32_t base = lds0 + (uint32_t)((j & (kPaRing - 1)) * kPaBlockVec * 16);
 #pragma unroll
     for (int i = 0; i < FPW / 2; ++i) {
       const int f = wave + NWV * i;
@@ -742,41 +755,118 @@ __global__ void __launch_bounds__(64 * G * pa_wph(G), 1) pattn_kernel(const Patt
   float m_run[MT], l_run[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    m_run[mt] = NEG_INF;
+    m_run[mt] = -1e30f;
     l_run[mt] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) acc[mt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
+  uint4 kf[8];  // keys of the next block to score: fragment 2s + h
+  auto read_k = [&](int j) {
+    const uint4 *B = lds + (j & (kPaRing - 1)) * kPaBlockVec + lane;
+#pragma unroll
+    for (int f = 0; f < 8; ++f) kf[f] = B[f * 64];
+  };
+  struct Scores {
+    f32x4_t a[MT], b[MT];  // slots sb .. sb+3 and sb+4 .. sb+7 of a lane
+  };
+  // k step s of tile u's scores, slots sb .. +3 (h = 0) or sb+4 .. +7
+  auto score1 = [&](Scores &S, int s, int u, int h) {
+    f32x4_t &d = h ? S.b[u] : S.a[u];
+    d = mfma16x16x32(kf[2 * s + h], qf[u][s], s ? d : f32x4_t{0.f, 0.f, 0.f, 0.f});
+  };
+  // Waits until this wave's loads of block j are done (blocks up to `newest`
+  // have been issued), then meets the other waves: block j is in LDS, and
+  // every wave has read what it needs of the blocks before.
+  auto await = [&](int j, int newest) {
+    const int younger = min(newest, nb - 1) - j;
+    if (younger >= 2)
+      __builtin_amdgcn_s_waitcnt(vmcnt_enc(2 * FPW) & ~(15 << 8));
+    else if (younger == 1)
+      __builtin_amdgcn_s_waitcnt(vmcnt_enc(FPW) & ~(15 << 8));
+    else
+      __builtin_amdgcn_s_waitcnt(kVmcnt0 & ~(15 << 8));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
   // The query loads complete here, so no wait inside the loop (where it
   // would also wait for the blocks in flight) is needed for them.
   __builtin_amdgcn_s_waitcnt(kVmcnt0);
-  dma_block(0, 0);
-  if (nb > 1) dma_block(1, 1);
-  int slot = 0;
-  for (int j = 0; j < nb; ++j) {
-    // this wave's loads of block j are done once at most the next block's
-    // are outstanding; the barrier makes every wave's visible and frees the
-    // slot of block j-1 for block j+2
-    if (j + 1 < nb)
-      __builtin_amdgcn_s_waitcnt(vmcnt_enc(FPW));
-    else
-      __builtin_amdgcn_s_waitcnt(kVmcnt0);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (j + 2 < nb) dma_block(j + 2, slot == 0 ? kPaRing - 1 : slot - 1);
-    const uint4 *B = lds + slot * kPaBlockVec + lane;
-    uint4 ka[4], kb[4], vf[8];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      ka[s] = B[(s * 2) * 64];
-      kb[s] = B[(s * 2 + 1) * 64];
+  for (int j = 0; j < kPaRing - 1; ++j)
+    if (j < nb) dma_block(j);
+  await(0, kPaRing - 2);
+  read_k(0);
+  Scores s0, s1;
+#pragma unroll
+  for (int i = 0; i < 8 * MT; ++i) score1(s0, i >> 2, (i >> 1) & 1, i & 1);
+  await(min(1, nb - 1), kPaRing - 2);
+  if (kPaRing - 1 < nb) dma_block(kPaRing - 1);
+  read_k(1);
+
+  // Block j from its scores S; leaves block j + 1's in N (kf holds its keys;
+  // past the last block they are whatever the ring holds, and unused).
+  auto block = [&](int j, Scores &S, Scores &N) {
+    const int sb = j * 32 + 8 * grp;  // first of this lane's 8 slots
+    if (!(rows_full && j * 32 + 31 <= p.pos0 + t0)) {
+      // the block crosses some row's position (the diagonal, rows past the end)
+#pragma unroll
+      for (int u = 0; u < MT; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (sb + i > qpos[u]) S.a[u][i] = NEG_INF;
+          if (sb + 4 + i > qpos[u]) S.b[u][i] = NEG_INF;
+        }
     }
 #pragma unroll
+    for (int u = 0; u < MT; ++u) {
+      const float bmax = fmaxf(fmaxf(fmaxf(S.a[u][0], S.a[u][1]), fmaxf(S.a[u][2], S.a[u][3])),
+                               fmaxf(fmaxf(S.b[u][0], S.b[u][1]), fmaxf(S.b[u][2], S.b[u][3])));
+      if (!__any(bmax > m_run[u])) continue;  // no row's maximum moves
+      const float m_new = fmaxf(m_run[u], max_xor16_32(bmax));
+      const float alpha = __builtin_amdgcn_exp2f((m_run[u] - m_new) * scale);
+      l_run[u] *= alpha;
+      m_run[u] = m_new;
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) acc[u][dt] *= alpha;
+    }
+    uint4 vf[8];
+    const uint4 *B = lds + (j & (kPaRing - 1)) * kPaBlockVec + lane;
+#pragma unroll
     for (int dt = 0; dt < 8; ++dt) vf[dt] = B[(kPaKFrags + dt) * 64];
-    const int s0 = j * 32;
-    const int sb = s0 + 8 * grp;  // first of this lane's 8 slots
-    if (sb + 7 > last) {          // slots past the last row: zero V
+    // Block j + 1's scores between the exponentials of block j: one MFMA
+    // per probability, in this order.
+    uint4 pf[MT];
+    float pj[MT][8], mc[MT], psum[MT];
+#pragma unroll
+    for (int u = 0; u < MT; ++u) {
+      mc[u] = m_run[u] * scale;
+      psum[u] = 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < MT; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int i = u * 8 + e;  // MFMA i of the scores: k step i / 4, tile, slot half
+        float x = e < 4 ? S.a[u][e] : S.b[u][e - 4];
+        pin(x);
+        pj[u][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(x, scale, -mc[u]));
+        score1(N, i >> 2, (i >> 1) & 1, i & 1);
+        pin((i & 1) ? N.b[(i >> 1) & 1] : N.a[(i >> 1) & 1]);
+        if (i > 0) psum[(i - 1) >> 3] += pj[(i - 1) >> 3][(i - 1) & 7];
+        pin(pj[u][e]);
+      }
+    psum[MT - 1] += pj[MT - 1][7];
+#pragma unroll
+    for (int u = 0; u < MT; ++u) {
+      l_run[u] += psum[u];
+      pf[u] = pack8(pj[u]);
+    }
+    // Block j + 2 in LDS; slot j (whose V every wave holds) takes block j + kPaRing.
+    await(min(j + 2, nb - 1), j + kPaRing - 1);
+    if (j + kPaRing < nb) dma_block(j + kPaRing);
+    if (j * 32 + 31 > last) {  // slots past the last row: zero V
       uint32_t keep[4];
 #pragma unroll
       for (int d = 0; d < 4; ++d)
@@ -789,70 +879,15 @@ __global__ void __launch_bounds__(64 * G * pa_wph(G), 1) pattn_kernel(const Patt
         vf[dt].w &= keep[3];
       }
     }
-    // Online softmax of one tile's 8 scores per lane (masked ones -inf):
-    // updates the row state, returns the rescale factor and the bf16
-    // probabilities as the B operand of the P.V product.
-    auto softmax = [&](int mt, const float (&sc)[8], float &alpha, uint4 &pf) {
-      float bmax = sc[0];
+    read_k(j + 2);
 #pragma unroll
-      for (int e = 1; e < 8; ++e) bmax = fmaxf(bmax, sc[e]);
-      bmax = max_xor16_32(bmax);
-      const float m_new = fmaxf(m_run[mt], bmax);
-      alpha = (m_new == NEG_INF) ? 1.0f : __builtin_amdgcn_exp2f((m_run[mt] - m_new) * scale);
-      const float mc = m_new * scale;
-      float pj[8];
-      float psum = 0.f;
+    for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pj[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[e], scale, -mc));
-        psum += pj[e];
-      }
-      l_run[mt] = l_run[mt] * alpha + psum;
-      m_run[mt] = m_new;
-      pf = pack8(pj);
-    };
-    // Masks only where the block crosses some row's position (the diagonal,
-    // rows past the end); a tile that sees none of the block gets all -inf
-    // and leaves its rows unchanged (alpha 1, p 0).
-    const bool masked = !(rows_full && s0 + 31 <= p.pos0 + t0);
-#pragma unroll
-    for (int m2 = 0; m2 < MT; m2 += 2) {
-      f32x4_t sa[2], sbv[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) sa[u] = sbv[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          sa[u] = mfma16x16x32(ka[s], qf[m2 + u][s], sa[u]);
-          sbv[u] = mfma16x16x32(kb[s], qf[m2 + u][s], sbv[u]);
-        }
-      float alpha[2];
-      uint4 pf[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        float sc[8] = {sa[u][0], sa[u][1], sa[u][2], sa[u][3], sbv[u][0], sbv[u][1], sbv[u][2], sbv[u][3]};
-        if (masked) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if (sb + i > qpos[m2 + u]) sc[i] = NEG_INF;
-            if (sb + 4 + i > qpos[m2 + u]) sc[4 + i] = NEG_INF;
-          }
-        }
-        softmax(m2 + u, sc, alpha[u], pf[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-        if (__any(alpha[u] != 1.0f)) {
-#pragma unroll
-          for (int dt = 0; dt < 8; ++dt) acc[m2 + u][dt] *= alpha[u];
-        }
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) acc[m2 + u][dt] = mfma16x16x32(vf[dt], pf[u], acc[m2 + u][dt]);
-    }
-    slot = slot == kPaRing - 1 ? 0 : slot + 1;
+      for (int u = 0; u < MT; ++u) acc[u][dt] = mfma16x16x32(vf[dt], pf[u], acc[u][dt]);
+  };
+  for (int j = 0; j < nb; j += 2) {
+    block(j, s0, s1);
+    if (j + 1 < nb) block(j + 1, s1, s0);
   }
 
   // Rows in fragment order for the O projection: lane holds channels
@@ -942,13 +977,20 @@ hipError_t launch_pnorm(const void *x, const void *norm_w, void *out, float eps,
   return hipSuccess;
 }
 
+namespace {
+template <int G, int GS>
+void launch_pattn(const PattnParams &p, int blocks, hipStream_t s) {
+  hipLaunchKernelGGL((pattn_kernel<G, GS>), dim3(blocks * (GS / G)), dim3(64 * G * kPaWph), 0, s, p);
+}
+}  // namespace
+
 hipError_t launch_prefill_attn(const PattnParams &p, hipStream_t s) {
   const int nqb = (p.t_rows + kPaRows - 1) / kPaRows;
-  const dim3 grid(nqb * p.batch * p.nkv);
+  const int blocks = nqb * p.batch * p.nkv;
   switch (p.nq / p.nkv) {
-    case 2: hipLaunchKernelGGL(pattn_kernel<2>, grid, dim3(64 * 2 * pa_wph(2)), 0, s, p); break;
-    case 4: hipLaunchKernelGGL(pattn_kernel<4>, grid, dim3(64 * 4 * pa_wph(4)), 0, s, p); break;
-    case 8: hipLaunchKernelGGL((pattn_kernel<4, 8>), dim3(2 * grid.x), dim3(64 * 4 * pa_wph(4)), 0, s, p); break;
+    case 2: launch_pattn<2, 2>(p, blocks, s); break;
+    case 4: launch_pattn<4, 4>(p, blocks, s); break;
+    case 8: launch_pattn<4, 8>(p, blocks, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipSuccess;
