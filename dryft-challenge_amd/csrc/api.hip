@@ -62,13 +62,19 @@ static void gemm_scratch(const qdec_gemm_args *a, const GemmParams &p, size_t *p
   *xn_off = off;
 }
 
+// Whether gemm_wide.hip's 32-bit lane offsets reach the up half of w.
+static bool wide_offsets(const qdec_gemm_args *a) { return (uint64_t)a->n * a->k * 2 < (1ull << 32) - 4096; }
+
 // Derive the launch plan of a GEMM call; returns QDEC_OK or an error code.
-static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch) {
+// With `wide` the many-row plan or an error (qdec_gemm_wide).
+static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch, bool wide = false) {
   if (!a) return set_error(QDEC_EINVAL, "qdec_gemm: null args");
   *p = GemmParams{};
   const uint32_t f = a->flags;
   if (!gemm_flags_supported(f)) return set_error(QDEC_EUNSUPPORTED, "qdec_gemm: flags 0x%x not supported", f);
-  if (a->rows < 1 || a->rows > 64) return set_error(QDEC_EINVAL, "qdec_gemm: rows %d not in [1, 64]", a->rows);
+  const int row_min = wide ? kWideMinRows : 1, row_max = wide ? kWideMaxRows : 64;
+  if (a->rows < row_min || a->rows > row_max)
+    return set_error(QDEC_EINVAL, "qdec_gemm: rows %d not in [%d, %d]", a->rows, row_min, row_max);
   if (a->n <= 0 || a->n % 16) return set_error(QDEC_EINVAL, "qdec_gemm: n %d not a positive multiple of 16", a->n);
   if (a->k <= 0 || a->k % 32) return set_error(QDEC_EINVAL, "qdec_gemm: k %d not a positive multiple of 32", a->k);
   if (a->waves < 1 || a->waves > 8) return set_error(QDEC_EINVAL, "qdec_gemm: waves %d not in [1, 8]", a->waves);
@@ -253,6 +259,21 @@ static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch) 
     ring_d = gemm_ring_direct(mt, f, 1, p->ksw, a->tiles_per_wg);
   }
   const size_t lds_direct = head + red_bytes * tw;
+  // From 9 rows the direct path at four waves runs with every row tile of
+  // several output tiles in registers (gemm_wide.hip; the same bits).  MI355X,
+  // us per launch, direct / this, QKV, O, gate/up and down (k split 4): 13
+  // rows 9.7 / 7.9, 8.3 / 7.9, 20.3 / 19.3, 13.0 / 10.3; 32 rows 12.4 / 9.5,
+  // 10.2 / 9.2, 23.3 / 20.6, 16.2 / 11.3; 64 rows 16.9 / 11.4, 14.2 / 12.5,
+  // 30.7 / 22.5, 22.5 / 14.6; lm_head (16896 columns) at 64 rows 46.4 / 29.5.
+  // Below 9 rows the rows stay in LDS and are normalised there.
+  const bool many = a->rows >= kWideMinRows && a->waves == 4 && (arg || a->tiles_per_wg == 1) &&
+                    (a->ksplit == 1 || a->parts_out) && !a->next_norm_w && wide_offsets(a);
+  if (wide) {
+    if (!many || arg || xa || a->resident || (!a->x_frag && !(f & QDEC_NORM_IN)))
+      return set_error(QDEC_EUNSUPPORTED, "qdec_gemm_wide: needs 4 waves, one tile per workgroup, x_frag = 1 or NORM_IN, "
+                       "ksplit 1 or parts_out, no ARGMAX, x_attn, next_norm_w or resident");
+    if (!ring_d) ring_d = 1;  // its own ring
+  }
   // Past its register-staged rows a NORM_IN call does better on the direct
   // path: one normalisation pre-pass instead of every workgroup reading
   // whole rows for the statistics and then again for staging (gate/up at 8
@@ -335,6 +356,7 @@ static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch) 
   if (p->lds_bytes > (size_t)kGemmLdsX)
     return set_error(QDEC_EUNSUPPORTED, "qdec_gemm: rows %d x waves %d needs %zu B of LDS", a->rows, a->waves,
                      p->lds_bytes);
+  p->wide = p->xd && many;
   // Norm hand-over to the next NORM_IN call (gemm_dev.h hand_over_row).
   p->hnorm_w = nullptr;
   p->hxn = nullptr;
@@ -643,6 +665,23 @@ int qdec_gemm(const qdec_gemm_args *a, qdec_stream_t stream) {
   const int rc = plan_gemm(a, &p, true);
   if (rc != QDEC_OK) return rc;
   return launch_status(launch_gemm(p, a->flags, (hipStream_t)stream), "qdec_gemm");
+}
+
+int qdec_gemm_wide_workspace(const qdec_gemm_args *a, size_t *partial_bytes) {
+  GemmParams p;
+  const int rc = plan_gemm(a, &p, false, true);
+  if (rc != QDEC_OK) return rc;
+  size_t pb = 0, cb = 0, xn_off = 0;
+  gemm_scratch(a, p, &pb, &cb, &xn_off);
+  if (partial_bytes) *partial_bytes = pb;
+  return QDEC_OK;
+}
+
+int qdec_gemm_wide(const qdec_gemm_args *a, qdec_stream_t stream) {
+  GemmParams p;
+  const int rc = plan_gemm(a, &p, true, true);
+  if (rc != QDEC_OK) return rc;
+  return launch_status(launch_gemm(p, a->flags, (hipStream_t)stream), "qdec_gemm_wide");
 }
 
 int qdec_attn_workspace(const qdec_attn_args *a, size_t *partial_bytes, size_t *counter_bytes) {

@@ -310,6 +310,7 @@ hipError_t launch_gemm(const GemmParams &p, uint32_t flags, hipStream_t s) {
       if (e != hipSuccess) return e;
       q.x = p.xn;
     }
+    if (p.wide) return launch_wide(q, flags, s);
     if (p.tw == 2) return mt == 2 ? launch_direct_tw2(q, flags, grid, block, lds, s) : hipErrorInvalidValue;
     if (p.tw != 1) return hipErrorInvalidValue;
     switch (mt) {

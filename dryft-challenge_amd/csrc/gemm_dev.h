@@ -83,6 +83,33 @@ __device__ __forceinline__ void block_row_sums(float (&ss)[8], float *s_red, int
   __syncthreads();
 }
 
+// Row maxima of the argmax keys (gemm_body.inc: kArgSlots per row, folded by
+// every workgroup) by the workgroup that arrived last, nw waves: the picks to
+// ids_out, lens_inc (optional) up by one, and the keys zero again.  A wave
+// takes 4 rows per pass (16 lanes, one slot each), four passes' loads in
+// flight at once.
+__device__ __forceinline__ void argmax_finish(uint64_t *keys, int rows, int nw, int wave, int lane, int64_t *ids_out,
+                                              int32_t *lens_inc) {
+  for (int j0 = 0; j0 * nw * 4 < rows; j0 += 4) {
+    uint64_t kv[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int m = ((j0 + j) * nw + wave) * 4 + (lane >> 4);
+      kv[j] = m < rows ? ld64_dev(keys + (size_t)m * kArgSlots + (lane & 15)) : 0ull;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int m = ((j0 + j) * nw + wave) * 4 + (lane >> 4);
+      if (m < rows) st64_dev(keys + (size_t)m * kArgSlots + (lane & 15), 0ull);
+      const uint64_t best = row16_max(kv[j]);
+      if ((lane & 15) == 0 && m < rows) {
+        ids_out[m] = (int64_t)argmax_index(best);
+        if (lens_inc) lens_inc[m] += 1;
+      }
+    }
+  }
+}
+
 // Activation vector (8 consecutive elements from k index kk) of row m,
 // merged from the attention chunk partials the previous launch left with
 // out_partials (attn_dev.h: per (sequence, kv head, chunk) acc [R][128],

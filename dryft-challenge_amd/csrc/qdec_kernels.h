@@ -52,6 +52,12 @@ constexpr int kResLdsRing = 20;
 constexpr int kResSplitKSteps = 76;
 constexpr int kResSplitRing = 10;
 
+// Many rows in registers (gemm_wide.hip): kWideMinRows..kWideMaxRows rows,
+// one workgroup per CU in a round.
+constexpr int kWideMinRows = 9;
+constexpr int kWideMaxRows = 128;
+constexpr int kWideWorkgroups = 256;
+
 struct GemmParams {
   const void *x;
   const void *w;
@@ -105,6 +111,7 @@ struct GemmParams {
   uint32_t *hsync;
   int resident;  // gemm_resident.hip: 1 NORM_IN | GLU with the normalised rows in LDS, 2 RES_OUT with the rows in LDS,
                  // 3 RES_OUT split into k parts, each part's rows in LDS, 4 NORM_IN alone as 1
+  int wide;      // gemm_wide.hip: the direct path's sums with all rows' tiles in registers
   int res_waves;  // resident: waves per workgroup (set by the launcher)
   int res_half;   // resident GLU: the units are runs of half pairs (set by the launcher)
   size_t lds_bytes;
@@ -125,6 +132,7 @@ hipError_t launch_gemm(const GemmParams &p, uint32_t flags, hipStream_t s);
 hipError_t launch_glu_resident(const GemmParams &p, hipStream_t s);
 hipError_t launch_res_rows(const GemmParams &p, hipStream_t s);
 hipError_t launch_res_split(const GemmParams &p, hipStream_t s);
+hipError_t launch_wide(const GemmParams &p, uint32_t flags, hipStream_t s);
 
 struct AttnParams {
   const void *qkv;

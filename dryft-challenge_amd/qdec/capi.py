@@ -126,7 +126,7 @@ class Lib:
         so.qdec_pack_tiles.argtypes = [P, P, ctypes.c_int64, ctypes.c_int64, P]
         so.qdec_read_probe.argtypes = [P, ctypes.c_int64, P, I32, P]
         so.qdec_read_probe.restype = ctypes.c_int
-        for name, st in (("qdec_embed", EmbedArgs), ("qdec_gemm", GemmArgs), ("qdec_attn", AttnArgs),
+        for name, st in (("qdec_embed", EmbedArgs), ("qdec_gemm", GemmArgs), ("qdec_gemm_wide", GemmArgs), ("qdec_attn", AttnArgs),
                          ("qdec_attn_noalloc", AttnArgs),
                          ("qdec_ngram_draft", DraftArgs), ("qdec_spec_accept", AcceptArgs),
                          ("qdec_rownorm", RownormArgs), ("qdec_prefill_gemm", PgemmArgs),
@@ -143,6 +143,8 @@ class Lib:
             fn.argtypes = [ctypes.POINTER(st), ctypes.POINTER(ctypes.c_size_t),
                            ctypes.POINTER(ctypes.c_size_t)]
             fn.restype = ctypes.c_int
+        so.qdec_gemm_wide_workspace.argtypes = [ctypes.POINTER(GemmArgs), ctypes.POINTER(ctypes.c_size_t)]
+        so.qdec_gemm_wide_workspace.restype = ctypes.c_int
         so.qdec_gemm_prepass.argtypes = [ctypes.POINTER(GemmArgs), ctypes.POINTER(I32)]
         so.qdec_gemm_prepass.restype = ctypes.c_int
 
@@ -173,6 +175,14 @@ class Lib:
 
     def gemm(self, args, stream):
         self._check("qdec_gemm", self.so.qdec_gemm(ctypes.byref(args), stream))
+
+    def gemm_wide(self, args, stream):
+        self._check("qdec_gemm_wide", self.so.qdec_gemm_wide(ctypes.byref(args), stream))
+
+    def gemm_wide_workspace(self, args):
+        pb = ctypes.c_size_t()
+        self._check("qdec_gemm_wide_workspace", self.so.qdec_gemm_wide_workspace(ctypes.byref(args), ctypes.byref(pb)))
+        return pb.value
 
     def attn(self, args, stream):
         self._check("qdec_attn", self.so.qdec_attn(ctypes.byref(args), stream))

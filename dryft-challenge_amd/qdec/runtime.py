@@ -47,9 +47,9 @@ PREFILL_ROWS = 32768
 PREFILL_ROW_TILE = 256
 PREFILL_ROW_TILE_SMALL = 64
 # A prompt of at most this many rows in all (batch x length) runs its layer
-# products through the decode GEMMs (qdec_gemm) instead of the matrix-core
-# prefill products, which make too few workgroups at so few rows.
-PREFILL_SKINNY_ROWS = GEMM_MAX_ROWS
+# products through qdec_gemm_wide instead of the matrix-core prefill products,
+# which make too few workgroups at so few rows.
+PREFILL_SKINNY_ROWS = 128
 # lm_head output tiles per workgroup from 2 rows (the role plan's 4 stays at
 # 1 row).  Grouping changes no sum and the argmax partials are scanned
 # lowest index first, so tokens and logits do not depend on it (MI355X,
@@ -102,11 +102,19 @@ O_FOUR_WAVES_MIN_BATCH = 9
 O_SPLIT = 2
 O_SPLIT_MIN_BATCH = 17
 O_SPLIT_MAX_BATCH = 32
-# Output tiles per workgroup of QKV and down at two M tiles (WIDE_MIN_ROWS..32
-# rows).  Paired tiles run two per wave, so each activation fragment a wave
-# loads feeds both (the sums do not change).  MI355X, 32 rows, us per launch
-# (one tile / two): QKV 18.6 / 15.3 with 8 waves (pre-pass included), down
-# 16.1 / 15.0; gate/up (28.4 / 30.4) and O (10.5 / 13.5) keep one.
+# From MANY_ROWS_MIN_BATCH sequences (no speculation there) a step's plans are
+# those of qdec_gemm's many-row kernel (step_plan): O and down split k and
+# leave fp32 partials to the next NORM_IN call's pre-pass at every batch,
+# since their 160 output tiles alone leave a third of the CUs idle.  Same-box
+# A/B, us per launch unsplit / split: down at 13 rows 18.7 / 11.4, O 8.8 /
+# 7.4; four layers (1024-token prompts), per-tile kernels and role_plan
+# against the many-row kernel and step_plan: batch 9 381 / 329 us, 13 390 /
+# 338, 33 592 / 507, 64 684 / 573.  At batch 8 and below the merge costs as
+# much as the split gains (batch 8 3.01 -> 3.09 ms per step, batch 1 2.145 ->
+# 2.155).
+MANY_ROWS_MIN_BATCH = 9
+# Output tiles per workgroup of qdec_gemm's two-tiles-per-wave plan (17..32
+# rows); the runtime's own calls take the many-row kernel there.
 WIDE_TILES = 2
 WIDE_MIN_ROWS = 17
 # gate/up at RESIDENT_ROWS rows runs with its rows resident in LDS
@@ -274,6 +282,22 @@ def role_plan(n, k, role, batch=1):
                 tiles = cand
                 break
     return ksplit, waves, tiles
+
+
+def step_plan(n, k, role, batch, split_o=True):
+    """(ksplit, waves, tiles_per_wg) of ``role`` in a state of ``batch``
+    sequences: role_plan's, and from MANY_ROWS_MIN_BATCH that of the many-row
+    kernel -- 4 waves, O (``split_o``) and down in O_SPLIT and DOWN_SPLIT k
+    splits where their widths allow."""
+    ksplit, waves, tiles = role_plan(n, k, role, batch)
+    if batch < MANY_ROWS_MIN_BATCH or role not in ("qkv", "o", "down"):
+        return ksplit, waves, tiles
+    ks = k // 32
+    want = {"qkv": 1, "o": O_SPLIT if split_o else 1, "down": DOWN_SPLIT}[role]
+    for split in (want, 1):
+        if ks % (split * 4) == 0 and (split == 1 or n // 16 <= 256):
+            return split, 4, tiles
+    return 1, waves, tiles
 
 
 # From this batch the attention runs 8 waves per workgroup with the
@@ -491,17 +515,18 @@ class DecodeState:
         self.hbuf = torch.zeros((2, R, H), dtype=bf, device=dev)
         self.h = self.hbuf[0]
         self.plans = dict(model.plans)
-        self.plans["down"] = role_plan(H, c.inter, "down", batch)
-        self.plans["qkv"] = role_plan(c.n_qkv, H, "qkv", batch)
-        self.plans["o"] = role_plan(H, c.nq * c.head_dim, "o", batch)
+        self.plans["down"] = step_plan(H, c.inter, "down", batch)
+        self.plans["qkv"] = step_plan(c.n_qkv, H, "qkv", batch)
         ks, _, _ = self.plans["down"]
+        # O splits only where down does: the residual then always moves by
+        # merges (_residual_in).
+        self.plans["o"] = step_plan(H, c.nq * c.head_dim, "o", batch, split_o=ks > 1)
         self.down_parts = torch.zeros((ks, R, H), dtype=torch.float32, device=dev) if ks > 1 else None
         # A split O projection leaves its update as partials too (o_parts);
         # the gate/up call's pre-pass merges them into hpost, the residual
         # after the attention, to which the down projection's partials then
         # belong.
         ko, _, _ = self.plans["o"]
-        assert ko == 1 or ks > 1, "a split O needs a split down (the residual then always moves by merges)"
         self.o_parts = torch.zeros((ko, R, H), dtype=torch.float32, device=dev) if ko > 1 else None
         self.hpost = torch.zeros((R, H), dtype=bf, device=dev) if ko > 1 else None
         self.qkv = torch.zeros((R, c.n_qkv), dtype=bf, device=dev)
@@ -681,31 +706,20 @@ class DecodeState:
             a.w = m.lm_w.data_ptr()
             a.norm_w = m.norm_w.data_ptr()
             a.n, a.k, a.flags = c.vocab, c.hidden, capi.NORM_IN | capi.ARGMAX
-            # 8 tiles per workgroup from 2 rows; past two M tiles (33+ rows,
-            # verify passes only) one, so the direct path's ring fits the
-            # workgroup's k range (the grouping changes no sum).
+            # 8 tiles per workgroup from 2 rows; from 9 the many-row kernel
+            # groups them itself (the grouping changes no sum).
             if rows == 1:
                 a.tiles_per_wg = tiles
-            elif rows <= 32 and (c.vocab // 16) % LM_TILES_BATCHED == 0:
+            elif rows <= 8 and (c.vocab // 16) % LM_TILES_BATCHED == 0:
                 a.tiles_per_wg = LM_TILES_BATCHED
-            else:
-                a.tiles_per_wg = 1
             a.out = self.logits.data_ptr() if self.logits is not None else None
             a.ids_out = (ids_out if ids_out is not None else self.ids).data_ptr()
             a.lens_inc = lens_inc.data_ptr() if lens_inc is not None else None
-        # two output tiles per workgroup for QKV and down at two M tiles
-        if role in ("qkv", "down") and WIDE_MIN_ROWS <= rows <= 32 and (a.n // 16) % WIDE_TILES == 0:
-            a.tiles_per_wg = WIDE_TILES
         if hasattr(self, "gemm_partial"):
             a.partial = self.gemm_partial.data_ptr()
             a.counters = self.gemm_counters.data_ptr()
         if role in ("gate_up", "qkv") + RESIDENT_RES_ROLES:
-            wide = a.tiles_per_wg
-            if role == "qkv":
-                a.tiles_per_wg = 1  # the resident plan takes one tile per workgroup
             a.resident = 1 if self._resident(a, role) else 0
-            if not a.resident:
-                a.tiles_per_wg = wide
         if hand:
             L = c.n_layers
             if role in ("o", "down"):
@@ -929,9 +943,8 @@ class Prefill:
     attention over the cache -> O product + residual -> rownorm -> gate/up
     product with SwiGLU -> down product + residual, the products on the
     matrix cores (qdec_prefill_gemm).  A prompt of at most
-    PREFILL_SKINNY_ROWS rows runs its products as the decode GEMMs instead
-    (qdec_gemm over all its rows, each weight read once; MI355X, one
-    sequence: see DecodeState.prefill).  After the last chunk the final row
+    PREFILL_SKINNY_ROWS rows runs its products as qdec_gemm_wide instead (each
+    weight streamed once for all rows).  After the last chunk the final row
     of each sequence goes through the decode lm_head + argmax.
 
     Replaces engine/engine.py:448-490 (``_layers_forward`` over the whole
@@ -944,7 +957,7 @@ class Prefill:
         self.max_chunk = max(1, rows // B)
         self.chunk = min(prompt_len, self.max_chunk)
         # The whole prompt in one chunk of at most PREFILL_SKINNY_ROWS rows:
-        # the decode GEMMs (see _skinny_args).
+        # the weight-streaming products (_skinny_layers).
         self.skinny = B * prompt_len <= min(PREFILL_SKINNY_ROWS, B * self.max_chunk)
         rows = prefill_tiles(B * self.chunk) * 16
         dev, bf = state.model.device, torch.bfloat16
@@ -954,53 +967,74 @@ class Prefill:
         self.att = torch.zeros((rows * c.nq * c.head_dim,), dtype=bf, device=dev)
         self.act = torch.zeros((rows * c.inter,), dtype=bf, device=dev)
         self.ids = torch.zeros((rows,), dtype=torch.int64, device=dev)
-        self.partial = self.counters = None
+        self._skinny_bufs, self._skinny_calls = None, {}
 
-    def _skinny_args(self, role, layer, R):
-        """qdec_gemm arguments of one layer product over all R prompt rows
-        (row b*S + t): x of QKV and gate/up is the residual h (row-major,
-        NORM_IN), the attention output comes in fragment order, and gate/up
-        hands its SwiGLU rows to down in fragment order from FRAG_ROWS rows,
-        as the decode step does.  Plans as the decode step's for R rows
-        (two tiles per wave at 17-32 rows), without a k split."""
+    def _skinny_layers(self, R):
+        """Every layer's four products over all R prompt rows (row b*S + t)
+        as qdec_gemm_wide calls, and the buffer that holds the residual after
+        the last one.  O and down split k as step_plan splits them and leave
+        their partials to the next NORM_IN call's pre-pass, which merges them
+        into the other of two residual buffers; the last layer's down, which
+        no call follows, does not split.  Built once per row count."""
+        if R in self._skinny_calls:
+            return self._skinny_calls[R]
         st, m, c = self.state, self.state.model, self.state.model.cfg
-        ksplit, waves, _ = m.plans[role]
-        if role == "qkv" and R >= WIDE_MIN_ROWS:
-            waves = 8
-        a = capi.GemmArgs()
-        a.eps, a.rows, a.ksplit, a.waves, a.tiles_per_wg = c.eps, R, 1, waves, 1
-        frag = 1 if R >= FRAG_ROWS else 0
-        if role == "qkv":
-            a.x, a.w, a.out, a.norm_w = self.h.data_ptr(), m.w_qkv[layer].data_ptr(), self.qkv.data_ptr(), \
-                m.in_w[layer].data_ptr()
-            a.n, a.k, a.flags = c.n_qkv, c.hidden, capi.NORM_IN
-        elif role == "o":
-            a.x, a.w, a.res = self.att.data_ptr(), m.w_o[layer].data_ptr(), self.h.data_ptr()
-            a.n, a.k, a.flags, a.x_frag = c.hidden, c.nq * c.head_dim, capi.RES_OUT, 1
-        elif role == "gate_up":
-            a.x, a.w, a.out, a.norm_w = self.h.data_ptr(), m.w_gu[layer].data_ptr(), self.act.data_ptr(), \
-                m.post_w[layer].data_ptr()
-            a.n, a.k, a.flags, a.out_frag = c.inter, c.hidden, capi.NORM_IN | capi.GLU, frag
-        else:
-            a.x, a.w, a.res = self.act.data_ptr(), m.w_down[layer].data_ptr(), self.h.data_ptr()
-            a.n, a.k, a.flags, a.x_frag = c.hidden, c.inter, capi.RES_OUT, frag
-        if role in ("qkv", "down") and WIDE_MIN_ROWS <= R <= 32 and (a.n // 16) % WIDE_TILES == 0:
-            a.tiles_per_wg = WIDE_TILES
-        if self.partial is not None:
-            a.partial, a.counters = self.partial.data_ptr(), self.counters.data_ptr()
-        return a
+        dev, H, nqd = m.device, c.hidden, c.nq * c.head_dim
+        split = {role: step_plan(H, k, role, MANY_ROWS_MIN_BATCH)[0] for role, k in (("o", nqd), ("down", c.inter))}
+        rows = self.state.batch * self.chunk  # the most this Prefill runs
+        if self._skinny_bufs is None:
+            xn = -(-rows // 16) * 16 * H  # the pre-pass's rows (qdec_gemm_wide_workspace)
+            self._skinny_bufs = (torch.zeros_like(self.h),
+                                 torch.zeros((max(split.values()) * rows * H,), dtype=torch.float32, device=dev),
+                                 torch.zeros((xn + 128,), dtype=torch.bfloat16, device=dev))
+        other, parts, partial = self._skinny_bufs
+        bufs = (self.h, other)
 
-    def _skinny_workspace(self, R):
-        """Scratch of the decode GEMMs over R rows (the plan, and so its
-        scratch, depends on the row count); grown, never shrunk."""
-        pb = cb = 16
-        for role in ("qkv", "o", "gate_up", "down"):
-            p_, c_ = self.state.lib.gemm_workspace(self._skinny_args(role, 0, R))
-            pb, cb = max(pb, p_), max(cb, c_)
-        if self.partial is None or self.partial.numel() * 4 < pb or self.counters.numel() * 4 < cb:
-            dev = self.state.model.device
-            self.partial = torch.zeros((pb // 4 + 4,), dtype=torch.float32, device=dev)
-            self.counters = torch.zeros((cb // 4 + 4,), dtype=torch.int32, device=dev)
+        def args(role, i, n, k, flags, w):
+            a = capi.GemmArgs()
+            a.eps, a.rows, a.n, a.k, a.flags, a.w = c.eps, R, n, k, flags, w[i].data_ptr()
+            a.ksplit, a.waves, a.tiles_per_wg, a.partial = 1, 4, 1, partial.data_ptr()
+            return a
+
+        cur, pending, layers = 0, 0, []  # pending: partials the residual still owes
+
+        def norm_in(a, norm_w):
+            nonlocal cur, pending
+            a.x, a.norm_w = bufs[cur].data_ptr(), norm_w.data_ptr()
+            if pending:
+                cur = 1 - cur
+                a.x_parts, a.x_nparts, a.x_merged = parts.data_ptr(), pending, bufs[cur].data_ptr()
+                pending = 0
+
+        def res_out(a, x, ks):
+            nonlocal pending
+            a.x, a.x_frag, a.res = x.data_ptr(), 1, bufs[cur].data_ptr()
+            if ks > 1:
+                a.ksplit, a.parts_out, pending = ks, parts.data_ptr(), ks
+
+        for i in range(c.n_layers):
+            qkv = args("qkv", i, c.n_qkv, H, capi.NORM_IN, m.w_qkv)
+            qkv.out = self.qkv.data_ptr()
+            norm_in(qkv, m.in_w[i])
+            o = args("o", i, H, nqd, capi.RES_OUT, m.w_o)
+            res_out(o, self.att, split["o"])
+            gu = args("gate_up", i, c.inter, H, capi.NORM_IN | capi.GLU, m.w_gu)
+            gu.out, gu.out_frag = self.act.data_ptr(), 1
+            norm_in(gu, m.post_w[i])
+            down = args("down", i, H, c.inter, capi.RES_OUT, m.w_down)
+            res_out(down, self.act, split["down"] if i + 1 < c.n_layers else 1)
+            layers.append((qkv, o, gu, down))
+        for a in layers[0]:
+            if st.lib.gemm_wide_workspace(a) > partial.numel() * 2:
+                raise RuntimeError(f"prefill: {R} rows need {st.lib.gemm_wide_workspace(a)} bytes of scratch")
+        self._skinny_calls[R] = (layers, bufs[cur])
+        return self._skinny_calls[R]
+
+    def _skinny_fits(self, R):
+        """Whether qdec_gemm_wide takes this model's products (k / 128 whole
+        in every role)."""
+        c = self.state.model.cfg
+        return R >= 9 and all(k % 128 == 0 for k in (c.hidden, c.nq * c.head_dim, c.inter))
 
     def _gemm(self, x, w, out, n, k, rows, tiles, flags=0, res=None, out_frag=0):
         a = capi.PgemmArgs()
@@ -1013,9 +1047,12 @@ class Prefill:
         st = self.state
         m, c, lib = st.model, st.model.cfg, st.lib
         B, S = prompt.shape
+        if self.skinny and B * S <= GEMM_MAX_ROWS and not self._skinny_fits(B * S):
+            st.prefill_steps(prompt, stream=stream)
+            return
         s = (stream or torch.cuda.current_stream(m.device)).cuda_stream
         H, D = c.hidden, c.head_dim
-        T = self.chunk
+        T, last = self.chunk, self.h
         for c0 in range(0, S, self.chunk):
             T = min(self.chunk, S - c0)
             R = B * T
@@ -1036,18 +1073,19 @@ class Prefill:
             at.qkv, at.out, at.sm_scale = self.qkv.data_ptr(), self.att.data_ptr(), D ** -0.5
             at.batch, at.t_rows, at.pos0, at.nq, at.nkv = B, T, c0, c.nq, c.nkv
             at.head_dim, at.cap, at.tiles = D, st.cap, tiles
-            if self.skinny:
-                self._skinny_workspace(R)
-                at.tiles = -(-R // 16)  # the fragment order of the decode GEMMs
-                for i in range(c.n_layers):
-                    lib.gemm(self._skinny_args("qkv", i, R), s)
+            if self.skinny and self._skinny_fits(R):
+                at.tiles = -(-R // 16)  # the fragment order of qdec_gemm
+                layers, last = self._skinny_layers(R)
+                for i, (g_qkv, g_o, g_gu, g_dn) in enumerate(layers):
+                    lib.gemm_wide(g_qkv, s)
                     qk.q_norm_w, qk.k_norm_w = m.q_norm[i].data_ptr(), m.k_norm[i].data_ptr()
                     qk.k_cache, qk.v_cache = st.k_cache[i].data_ptr(), st.v_cache[i].data_ptr()
                     lib.prefill_qk(qk, s)
                     at.k_cache, at.v_cache = qk.k_cache, qk.v_cache
                     lib.prefill_attn(at, s)
-                    for role in ("o", "gate_up", "down"):
-                        lib.gemm(self._skinny_args(role, i, R), s)
+                    lib.gemm_wide(g_o, s)
+                    lib.gemm_wide(g_gu, s)
+                    lib.gemm_wide(g_dn, s)
                 continue
             g_qkv = self._gemm(self.xn, m.w_qkv[0], self.qkv, c.n_qkv, H, R, tiles)
             g_o = self._gemm(self.att, m.w_o[0], self.h, H, c.nq * D, R, tiles, capi.RES_OUT, res=self.h)
@@ -1072,6 +1110,6 @@ class Prefill:
                 g_dn.w = m.w_down[i].data_ptr()
                 lib.prefill_gemm(g_dn, s)
         # The last position of every sequence: final norm, lm_head, argmax.
-        st.h[:B].copy_(self.h[:B * T].view(B, T, H)[:, T - 1])
+        st.h[:B].copy_(last[:B * T].view(B, T, H)[:, T - 1])
         lib.gemm(st._gemm_args("lm", 0, B, ids_out=st.ids, pending=False), s)
         st.lens.fill_(S)

@@ -267,6 +267,19 @@ int qdec_gemm_workspace(const qdec_gemm_args *a, size_t *partial_bytes,
  * arguments are invalid (the error of qdec_gemm). */
 int qdec_gemm_prepass(const qdec_gemm_args *a, int32_t *threads);
 
+/* qdec_gemm at 9..128 rows on the many-row kernel that qdec_gemm itself takes
+ * from 9 to 64 rows at four waves: the same arguments and results, with
+ * flags 0, NORM_IN, RES_OUT, GLU or NORM_IN | GLU, waves 4, tiles_per_wg 1, k / 32
+ * / ksplit a multiple of 4, x_frag = 1 or NORM_IN (whose pre-pass writes the
+ * normalised rows to the partial workspace), ksplit > 1 only with parts_out,
+ * and no x_attn, next_norm_w or resident; n (2n with GLU) x k below 2 Gi
+ * elements.  QDEC_EUNSUPPORTED otherwise.  For the products of a short prompt,
+ * whose weights are read once for all rows.
+ * Replaces F.linear as the prefill forward uses it (engine/engine.py:448-461). */
+int qdec_gemm_wide(const qdec_gemm_args *a, qdec_stream_t stream);
+/* Bytes of `partial` a qdec_gemm_wide call with these arguments needs. */
+int qdec_gemm_wide_workspace(const qdec_gemm_args *a, size_t *partial_bytes);
+
 /* --------------------------------------------------- GQA decode attention */
 
 /* For every sequence b and query row t < t_rows (absolute position

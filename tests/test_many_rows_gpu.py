@@ -1,0 +1,183 @@
+"""The many-row product (qdec_gemm from 9 rows at four waves, qdec_gemm_wide up
+to 128) against the calls of at most 8 rows, bit for bit: every role's
+epilogue, row counts at the edges of the row tiles, widths that leave a
+workgroup short of output units and k ranges shorter than, equal to and past
+its load ring."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def lib():
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a HIP device")
+    from qdec import capi
+    return capi.lib()
+
+
+def stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+def rnd(*shape, scale=1.0, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=g) * scale).to(torch.bfloat16).to(DEV)
+
+
+def pack(lib, w):
+    dst = torch.empty(w.numel(), dtype=torch.bfloat16, device=DEV)
+    lib.pack_tiles(w.data_ptr(), dst.data_ptr(), w.shape[0], w.shape[1], stream())
+    return dst
+
+
+def to_frag(x):
+    """[rows, k] in fragment order, rows past the last NaN (they must not matter)."""
+    rows, k = x.shape
+    mt = -(-rows // 16)
+    full = torch.full((mt * 16, k), float("nan"), dtype=torch.bfloat16, device=DEV)
+    full[:rows] = x
+    return full.view(mt, 16, k // 32, 4, 8).permute(2, 0, 3, 1, 4).contiguous()
+
+
+def from_frag(buf, rows, cols):
+    mt = -(-rows // 16)
+    return buf.view(cols // 32, mt, 4, 16, 8).permute(1, 3, 0, 2, 4).reshape(mt * 16, cols)[:rows]
+
+
+class Call:
+    """One product in every form: kind -> the outputs of the rows given."""
+
+    def __init__(self, lib, kind, n, k, ksplit, seed):
+        from qdec import capi
+        self.lib, self.capi, self.kind, self.n, self.k, self.ksplit = lib, capi, kind, n, k, ksplit
+        glu = kind == "glu"
+        self.w = pack(lib, rnd(2 * n if glu else n, k, scale=0.05, seed=seed))
+        self.norm_w = rnd(k, scale=0.2, seed=seed + 1)
+        self.scratch = torch.zeros(4 << 20, dtype=torch.float32, device=DEV)
+        self.counters = torch.zeros(8192, dtype=torch.int32, device=DEV)
+
+    def __call__(self, x, res, wide):
+        c, rows, n = self.capi, x.shape[0], self.n
+        a = c.GemmArgs()
+        flags = {"norm": c.NORM_IN, "glu": c.NORM_IN | c.GLU, "plain": 0, "res": c.RES_OUT, "parts": c.RES_OUT,
+                 "argmax": c.NORM_IN | c.ARGMAX}[self.kind]
+        a.w, a.eps, a.rows, a.n, a.k, a.flags = self.w.data_ptr(), 1e-6, rows, n, self.k, flags
+        a.ksplit, a.waves, a.tiles_per_wg = self.ksplit, 4, 1
+        a.partial, a.counters = self.scratch.data_ptr(), self.counters.data_ptr()
+        if flags & c.NORM_IN:
+            a.x, a.norm_w = x.data_ptr(), self.norm_w.data_ptr()
+        else:
+            xf = to_frag(x)
+            a.x, a.x_frag = xf.data_ptr(), 1
+        mt = -(-rows // 16)
+        out = torch.full((mt * 16, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+        r = res.clone()
+        parts = torch.full((self.ksplit, rows, n), float("nan"), device=DEV)
+        ids = torch.full((rows,), -1, dtype=torch.int64, device=DEV)
+        lens = torch.zeros(rows, dtype=torch.int32, device=DEV)
+        frag = self.kind == "glu" and n % 32 == 0
+        if self.kind in ("norm", "glu", "plain", "argmax"):
+            a.out, a.out_frag = out.data_ptr(), int(frag)
+        else:
+            a.res = r.data_ptr()
+        if self.kind == "parts":
+            a.parts_out = parts.data_ptr()
+        if self.kind == "argmax":
+            a.ids_out, a.lens_inc = ids.data_ptr(), lens.data_ptr()
+        need = self.lib.gemm_wide_workspace(a) if wide else self.lib.gemm_workspace(a)[0]
+        assert need <= self.scratch.numel() * 4
+        (self.lib.gemm_wide if wide else self.lib.gemm)(a, stream())
+        torch.cuda.synchronize()
+        assert int(self.counters.abs().sum()) == 0
+        if self.kind == "argmax":
+            assert (lens == 1).all()
+            return [out[:rows], ids]
+        if self.kind == "parts":
+            assert torch.equal(r, res)
+            return list(parts)
+        if self.kind == "res":
+            return [r]
+        return [from_frag(out, rows, n) if frag else out[:rows]]
+
+
+# (kind, n, k, ksplit): one output unit and one k step per wave; units that do
+# not divide among workgroups; more units than one round of three; k splits.
+SHAPES = [("norm", 16, 128, 1), ("norm", 272, 640, 1), ("norm", 12304, 256, 1), ("plain", 272, 1152, 1),
+          ("glu", 16, 128, 1), ("glu", 304, 2560, 1), ("glu", 9728, 384, 1), ("res", 48, 1536, 1),
+          ("res", 2560, 4096, 1), ("parts", 2560, 4096, 2), ("parts", 2560, 9728, 4), ("parts", 1040, 512, 4)]
+
+
+@pytest.mark.parametrize("kind,n,k,ksplit", SHAPES)
+@pytest.mark.parametrize("rows", [9, 16, 17, 31, 33, 48, 64, 65, 100, 128])
+def test_many_rows_bitexact(lib, kind, n, k, ksplit, rows):
+    call = Call(lib, kind, n, k, ksplit, seed=n + k)
+    x, res = rnd(rows, k, scale=2.0, seed=rows), rnd(rows, n, seed=rows + 1)
+    want = [call(x[i:i + 8].contiguous(), res[i:i + 8].contiguous(), False) for i in range(0, rows, 8)]
+    for wide in (True,) if rows > 64 else (True, False):
+        got = call(x, res, wide)
+        for j, g in enumerate(got):
+            w = torch.cat([o[j] for o in want])
+            assert torch.isfinite(w).all()
+            kindint = torch.int16 if g.dtype == torch.bfloat16 else torch.int32
+            assert torch.equal(g.contiguous().view(kindint), w.view(kindint)), (wide, j)
+
+
+@pytest.mark.parametrize("rows,n", [(9, 16), (16, 4112), (33, 784), (64, 16896)])
+def test_many_rows_argmax(lib, rows, n):
+    """The lm_head's logits and picks; equal weight rows plant exact ties, so
+    the lowest of equal indices has to win across units and workgroups."""
+    call = Call(lib, "argmax", n, 256, 1, seed=n)
+    w = rnd(n, 256, scale=0.05, seed=n)
+    w[n // 2] = w[3] = w[n - 1] = 4 * w[3]
+    call.w = pack(lib, w)
+    x, res = rnd(rows, 256, scale=2.0, seed=rows), rnd(rows, n, seed=1)
+    logits, ids = call(x, res, False)
+    want = [call(x[i:i + 8].contiguous(), res[i:i + 8], False) for i in range(0, rows, 8)]
+    assert torch.equal(logits, torch.cat([o[0] for o in want]))
+    assert torch.equal(ids, torch.cat([o[1] for o in want]))
+    top = logits.float().amax(1, keepdim=True)
+    first = torch.where(logits.float() == top, torch.arange(n, device=DEV), n).amin(1)
+    assert torch.equal(ids, first)
+
+
+def test_wide_refusals(lib):
+    from qdec import capi
+    x, out = rnd(128, 256), torch.zeros(128, 64, dtype=torch.bfloat16, device=DEV)
+    good = dict(x=x.data_ptr(), w=x.data_ptr(), out=out.data_ptr(), eps=1e-6, rows=100, n=64, k=256, flags=0, ksplit=1,
+                waves=4, tiles_per_wg=1, x_frag=1)
+    lib.gemm_wide_workspace(capi.GemmArgs(**good))
+    for bad in (dict(rows=8), dict(rows=129), dict(waves=8), dict(waves=2), dict(tiles_per_wg=2), dict(x_frag=0),
+                dict(ksplit=2), dict(flags=capi.ARGMAX), dict(resident=1), dict(k=192)):
+        with pytest.raises(capi.QdecError):
+            lib.gemm_wide_workspace(capi.GemmArgs(**{**good, **bad}))
+    with pytest.raises(capi.QdecError):  # qdec_gemm itself still ends at 64 rows
+        lib.gemm_workspace(capi.GemmArgs(**good))
+
+
+def test_short_prompts_of_several_lengths_in_one_state(lib):
+    """One state prefills prompts of different lengths one after the other:
+    each leaves what a fresh state leaves."""
+    from qdec.checkpoint import generate_tensors, qwen3_config
+    from qdec.runtime import DecodeState, DeviceModel
+    cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024)
+    model = DeviceModel(cfg, dict(generate_tensors(cfg, seed=3, norm_jitter=0.05)), DEV)
+    shared = DecodeState(model, 2, 160, max_t=16, keep_logits=True)
+    for S in (60, 25, 64, 40, 130, 33):
+        prompt = torch.randint(0, 1024, (2, S), generator=torch.Generator().manual_seed(S)).to(DEV)
+        fresh = DecodeState(model, 2, 160, max_t=16, keep_logits=True)
+        for st in (shared, fresh):
+            st.prefill(prompt)
+        torch.cuda.synchronize()
+        if S <= 64:  # past a longer prompt the shared state keeps its products, whose sums differ
+            same = shared._prefill.skinny == fresh._prefill.skinny
+        if same:
+            assert torch.equal(shared.logits[:2], fresh.logits[:2]), S
+            assert torch.equal(shared.k_cache[:, :, :, :S], fresh.k_cache[:, :, :, :S]), S
+        else:
+            d = (shared.logits[:2].float() - fresh.logits[:2].float()).abs().max()
+            assert d <= 2e-2 * fresh.logits[:2].float().abs().max(), S
