@@ -187,10 +187,13 @@ bool gemm_fast_path(const GemmParams &p, uint32_t flags) {
 }
 
 int gemm_ring(int ksw, uint32_t flags) {
-  if (flags & QDEC_GLU) return ksw % 10 == 0 ? 10 : 0;
   // 20 and 16 measured faster than passes on MI355X; a 19-register ring
-  // (k = 9728 with 4 waves) was slower than 20-block passes.
-  for (const int rw : {20, 16})
+  // (k = 9728 with 4 waves) was slower than 20-block passes.  8 (8 gate|up
+  // pairs with GLU) for the widths those do not divide (Qwen3-1.7B's k =
+  // 2048): staged rows and a short ring beat the normalisation pre-pass and
+  // the direct path, us at one row QKV 12.6 -> 6.3, gate/up 17.1 -> 11.7.
+  if (flags & QDEC_GLU) return ksw % 10 == 0 ? 10 : ksw % 8 == 0 ? 8 : 0;
+  for (const int rw : {20, 16, 8})
     if (ksw % rw == 0) return rw;
   return 0;
 }
@@ -333,6 +336,10 @@ hipError_t launch_gemm(const GemmParams &p, uint32_t flags, hipStream_t s) {
         hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN | QDEC_ARGMAX, 20, false, 1, true>), grid, block, lds, s, p);
       else if (flags == (QDEC_NORM_IN | QDEC_ARGMAX) && p.rw == 16)
         hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN | QDEC_ARGMAX, 16, false, 1, true>), grid, block, lds, s, p);
+      else if (flags == QDEC_NORM_IN && p.rw == 8)
+        hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN, 8, false, 1, true>), grid, block, lds, s, p);
+      else if (flags == (QDEC_NORM_IN | QDEC_ARGMAX) && p.rw == 8)
+        hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN | QDEC_ARGMAX, 8, false, 1, true>), grid, block, lds, s, p);
       else
         return hipErrorInvalidValue;
       return hipSuccess;
@@ -347,16 +354,25 @@ hipError_t launch_gemm(const GemmParams &p, uint32_t flags, hipStream_t s) {
         hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN | QDEC_ARGMAX, 20, false, R8>), grid, block, lds, s, p);
       else if (flags == (QDEC_NORM_IN | QDEC_ARGMAX) && p.rw == 16)
         hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN | QDEC_ARGMAX, 16, false, R8>), grid, block, lds, s, p);
+      else if (flags == QDEC_NORM_IN && p.rw == 8)
+        hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN, 8, false, R8>), grid, block, lds, s, p);
+      else if (flags == (QDEC_NORM_IN | QDEC_ARGMAX) && p.rw == 8)
+        hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN | QDEC_ARGMAX, 8, false, R8>), grid, block, lds, s, p);
       else
         return hipErrorInvalidValue;
       return hipSuccess;
     }
     if (flags == (QDEC_NORM_IN | QDEC_GLU)) {
-      if (p.rw != 10) return hipErrorInvalidValue;
-      hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN | QDEC_GLU, 10, false>), grid, block, lds, s, p);
+      if (p.rw == 10)
+        hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN | QDEC_GLU, 10, false>), grid, block, lds, s, p);
+      else if (p.rw == 8)
+        hipLaunchKernelGGL((gemm_kernel<1, QDEC_NORM_IN | QDEC_GLU, 8, false>), grid, block, lds, s, p);
+      else
+        return hipErrorInvalidValue;
       return hipSuccess;
     }
     switch (p.rw) {
+      case 8: return launch_flags<1, 8>(p, flags, grid, block, lds, s);
       case 16: return launch_flags<1, 16>(p, flags, grid, block, lds, s);
       case 20: return launch_flags<1, 20>(p, flags, grid, block, lds, s);
       default: return hipErrorInvalidValue;

@@ -60,6 +60,7 @@ class Call:
         self.norm_w = rnd(k, scale=0.2, seed=seed + 1)
         self.scratch = torch.zeros(4 << 20, dtype=torch.float32, device=DEV)
         self.counters = torch.zeros(8192, dtype=torch.int32, device=DEV)
+        self.waves, self.row_major = 4, False
 
     def __call__(self, x, res, wide):
         c, rows, n = self.capi, x.shape[0], self.n
@@ -67,10 +68,12 @@ class Call:
         flags = {"norm": c.NORM_IN, "glu": c.NORM_IN | c.GLU, "plain": 0, "res": c.RES_OUT, "parts": c.RES_OUT,
                  "argmax": c.NORM_IN | c.ARGMAX}[self.kind]
         a.w, a.eps, a.rows, a.n, a.k, a.flags = self.w.data_ptr(), 1e-6, rows, n, self.k, flags
-        a.ksplit, a.waves, a.tiles_per_wg = self.ksplit, 4, 1
+        a.ksplit, a.waves, a.tiles_per_wg = self.ksplit, self.waves, 1
         a.partial, a.counters = self.scratch.data_ptr(), self.counters.data_ptr()
         if flags & c.NORM_IN:
             a.x, a.norm_w = x.data_ptr(), self.norm_w.data_ptr()
+        elif self.row_major:
+            a.x = x.data_ptr()
         else:
             xf = to_frag(x)
             a.x, a.x_frag = xf.data_ptr(), 1
@@ -143,6 +146,23 @@ def test_many_rows_argmax(lib, rows, n):
     top = logits.float().amax(1, keepdim=True)
     first = torch.where(logits.float() == top, torch.arange(n, device=DEV), n).amin(1)
     assert torch.equal(ids, first)
+
+
+@pytest.mark.parametrize("kind,n,k,waves", [("norm", 4096, 2048, 8), ("norm", 304, 1024, 4), ("glu", 6144, 2048, 4),
+                                            ("glu", 48, 1024, 4), ("res", 304, 2048, 8)])
+def test_short_ring_bitexact(lib, kind, n, k, waves):
+    """Widths whose k range per wave is a multiple of 8 but not of the longer
+    load rings (rows staged in LDS, a ring of 8): 1, 3, 5 and 8 rows give the
+    bits that a call of 12 rows, which reads them directly, gives."""
+    call = Call(lib, kind, n, k, 1, seed=n + k)
+    call.waves = waves
+    x, res = rnd(12, k, scale=2.0, seed=5), rnd(12, n, seed=6)
+    want = call(x, res, False)[0]
+    for rows in ([3], [0, 1, 2], [7, 8, 9, 10, 11], list(range(8))):
+        call.row_major = True
+        got = call(x[rows].contiguous(), res[rows].contiguous(), False)[0]
+        call.row_major = False
+        assert torch.equal(got.contiguous().view(torch.int16), want[rows].view(torch.int16)), rows
 
 
 def test_wide_refusals(lib):
