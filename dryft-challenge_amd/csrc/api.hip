@@ -770,20 +770,30 @@ int qdec_spec_accept(const qdec_accept_args *a, qdec_stream_t stream) {
 }
 
 // ------------------------------------------------------------- prefill
-int qdec_rownorm(const qdec_rownorm_args *a, qdec_stream_t stream) {
+static int rownorm(const qdec_rownorm_args *a, const float *parts, int nparts, void *merged, qdec_stream_t stream) {
   if (!a || !a->x || !a->out) return set_error(QDEC_EINVAL, "qdec_rownorm: null pointer");
   if (a->rows < 1 || a->k < 32 || a->k % 32 || a->tiles < (a->rows + 15) / 16)
     return set_error(QDEC_EINVAL, "qdec_rownorm: rows %d k %d tiles %d", a->rows, a->k, a->tiles);
-  if (!aligned16(a->x) || !aligned16(a->out) || (a->norm_w && !aligned16(a->norm_w)))
+  if (!aligned16(a->x) || !aligned16(a->out) || (a->norm_w && !aligned16(a->norm_w)) || !aligned16(parts) || !aligned16(merged))
     return set_error(QDEC_EALIGN, "qdec_rownorm: pointers must be 16-byte aligned");
-  const hipError_t e = pnorm_fits(a->k, a->rows)
+  const hipError_t e = !parts && pnorm_fits(a->k, a->rows)
                           ? launch_pnorm(a->x, a->norm_w, a->out, a->eps, a->rows, a->k, a->tiles, (hipStream_t)stream)
-                          : launch_rownorm_rows(a->x, a->norm_w, a->out, a->eps, a->rows, a->k, a->tiles,
-                                                (hipStream_t)stream);
+                          : launch_rownorm_rows(a->x, a->norm_w, a->out, a->eps, a->rows, a->k, a->tiles, parts, nparts,
+                                                merged, (hipStream_t)stream);
   return launch_status(e, "qdec_rownorm");
 }
 
-int qdec_prefill_gemm(const qdec_pgemm_args *a, qdec_stream_t stream) {
+int qdec_rownorm(const qdec_rownorm_args *a, qdec_stream_t stream) { return rownorm(a, nullptr, 0, nullptr, stream); }
+
+int qdec_rownorm_merge(const qdec_rownorm_args *a, const float *parts, int32_t nparts, void *merged,
+                       qdec_stream_t stream) {
+  if (!a || !parts || !merged || merged == a->x) return set_error(QDEC_EINVAL, "qdec_rownorm_merge: null pointer, or merged is x");
+  if (nparts < 1 || nparts > 8) return set_error(QDEC_EINVAL, "qdec_rownorm_merge: nparts %d not in [1, 8]", nparts);
+  return rownorm(a, parts, nparts, merged, stream);
+}
+
+// parts != NULL: RES_OUT with k in ksplit parts left to qdec_rownorm_merge.
+static int prefill_gemm(const qdec_pgemm_args *a, float *parts, int ksplit, qdec_stream_t stream) {
   if (!a || !a->x || !a->w || !a->out) return set_error(QDEC_EINVAL, "qdec_prefill_gemm: null pointer");
   const uint32_t f = a->flags;
   if (f != 0u && f != QDEC_RES_OUT && f != QDEC_GLU)
@@ -800,6 +810,7 @@ int qdec_prefill_gemm(const qdec_pgemm_args *a, qdec_stream_t stream) {
   // prompt padded to 64 rows) take the 64 x 64 tile only.
   const bool whole256 = a->tiles % (kPgRows / 16) == 0;
   if (trows == 0 && !whole256) trows = 64, tcols = 64;
+  if (parts) trows = 256, tcols = 128;  // few row tiles (the caller's rule): the narrow tile, many parts
   if (trows == 0) {
     // The least of the tiles' costs, in rounds of 256 x 256 tiles: the
     // 256-row tiles run one per CU, so ceil(tiles / 256) rounds, a round of
@@ -848,7 +859,21 @@ int qdec_prefill_gemm(const qdec_pgemm_args *a, qdec_stream_t stream) {
   p.tile_rows = trows;
   p.tile_cols = tcols;
   p.wg_n = glu ? (a->n / 2) / (tcols / 2) : a->n / tcols;
+  p.ksplit = ksplit;
+  p.parts = parts;
   return launch_status(launch_pgemm(p, f, (hipStream_t)stream), "qdec_prefill_gemm");
+}
+
+int qdec_prefill_gemm(const qdec_pgemm_args *a, qdec_stream_t stream) { return prefill_gemm(a, nullptr, 1, stream); }
+
+int qdec_prefill_gemm_split(const qdec_pgemm_args *a, float *parts, int32_t ksplit, qdec_stream_t stream) {
+  if (!a || !parts || !aligned16(parts)) return set_error(QDEC_EINVAL, "qdec_prefill_gemm_split: parts null or unaligned");
+  if (a->flags != QDEC_RES_OUT || a->tile_rows || a->tile_cols || a->tiles % (kPgRows / 16))
+    return set_error(QDEC_EUNSUPPORTED, "qdec_prefill_gemm_split: RES_OUT, tile 0 x 0, whole 256-row tiles");
+  if (ksplit < 1 || ksplit > 8 || a->k % (kPgStageK * ksplit))
+    return set_error(QDEC_EINVAL, "qdec_prefill_gemm_split: ksplit %d (1..8, k %d in parts of a multiple of %d)", ksplit,
+                     a->k, kPgStageK);
+  return prefill_gemm(a, parts, ksplit, stream);
 }
 
 int qdec_prefill_qk(const qdec_prefill_qk_args *a, qdec_stream_t stream) {

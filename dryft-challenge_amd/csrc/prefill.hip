@@ -107,36 +107,42 @@ struct PgTile {
   static constexpr int PRE = (3 * WN) / 8;        // MFMA groups ahead of the barrier
 };
 
+constexpr uint32_t kPgParts = 1u << 8;  // template flag beside the QDEC_* ones
+
 template <uint32_t FLAGS, int WN>
 __global__ void __launch_bounds__(512, 2) pgemm_kernel(const PgemmParams p) {
   using S = PgTile<WN>;
   constexpr bool GLU = (FLAGS & QDEC_GLU) != 0;
   constexpr bool RES = (FLAGS & QDEC_RES_OUT) != 0;
+  constexpr bool PARTS = (FLAGS & kPgParts) != 0;  // k parts, their sums left in p.parts
   constexpr int XW = S::XW, RING = S::RING;
   static_assert(!GLU || WN % 2 == 0, "gate and up fragments pair up within a wave");
   __shared__ uint4 lds[RING * S::Frags * 64];  // [ring slot][fragment][lane]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
   const int wn = wave & 1, wm = wave >> 1;
-  const int KS = p.k >> 5;  // even
+  const int KSW = p.k >> 5, KS = PARTS ? KSW / p.ksplit : KSW;  // k steps of the weights and of a part (even)
 
   // Tile order: workgroup i runs on XCD i % 8, so each XCD gets a contiguous
   // range of the sequence, dealt to its workgroups in turn; the sequence
   // walks groups of kPgGroupN column tiles across all row tiles (the group's
   // weights stay in L2, each row tile of x is read by the group's workgroups
   // together).
-  const int ntm = p.tiles / S::Xf, T = ntm * p.wg_n;
-  const int nx = min(8, (int)gridDim.x), xcd = blockIdx.x & 7;
-  const int seq_end = (int)((int64_t)T * (xcd + 1) / nx);
-  const int per = ((int)gridDim.x + 7 - xcd) >> 3;  // workgroups on this XCD
-  int seq = (int)((int64_t)T * xcd / nx) + (blockIdx.x >> 3);
+  const int ntm = p.tiles / S::Xf, T1 = ntm * p.wg_n, T = PARTS ? T1 * p.ksplit : T1;
+  const int G = gridDim.x, xcd = blockIdx.x & 7;
+  const int per = G >> 3;  // workgroups on this XCD (the grid is a multiple of 8)
+  const int seq_end = (int)((int64_t)T * (xcd + 1) / 8);
+  int seq = (int)((int64_t)T * xcd / 8) + (blockIdx.x >> 3);
   if (seq >= seq_end) return;
-  auto place = [&](int id, int &tm, int &tn) {
+  auto place = [&](int id, int &tm, int &tn) -> int {  // and the k part
+    const int part = PARTS ? __builtin_amdgcn_readfirstlane(id / T1) : 0;
+    id -= part * T1;
     const int gsz = kPgGroupN * ntm;
-    const int g = id / gsz, r = id - g * gsz;
+    const int g = __builtin_amdgcn_readfirstlane(id / gsz), r = id - g * gsz;
     const int gn = min(kPgGroupN, p.wg_n - g * kPgGroupN);
-    tm = r / gn;
+    tm = __builtin_amdgcn_readfirstlane(r / gn);
     tn = g * kPgGroupN + (r - tm * gn);
+    return part;
   };
   // Weight tile of workgroup fragment f (GLU: WN gate tiles, then the WN
   // matching up tiles).
@@ -164,12 +170,12 @@ __global__ void __launch_bounds__(512, 2) pgemm_kernel(const PgemmParams p) {
   const char *src[S::LoadsMax];
   auto aim = [&](int id) {
     int tm, tn;
-    place(id, tm, tn);
+    const size_t k0 = (size_t)place(id, tm, tn) * KS;
 #pragma unroll
     for (int q = 0; q < S::LoadsMax; ++q) {
       const int f = min(wave + S::NW * q, S::Frags - 1);
-      src[q] = f < S::Wf ? reinterpret_cast<const char *>(p.w) + (size_t)wtile(tn, f) * KS * 1024
-                         : reinterpret_cast<const char *>(p.x) + (size_t)(tm * S::Xf + f - S::Wf) * 1024;
+      src[q] = f < S::Wf ? reinterpret_cast<const char *>(p.w) + ((size_t)wtile(tn, f) * KSW + k0) * 1024
+                         : reinterpret_cast<const char *>(p.x) + k0 * xks + (size_t)(tm * S::Xf + f - S::Wf) * 1024;
     }
   };
   auto load = [&](int q, uint32_t slot_base) {
@@ -285,7 +291,7 @@ __global__ void __launch_bounds__(512, 2) pgemm_kernel(const PgemmParams p) {
     // pair.  A tile whose rows are all real stores through inline assembly,
     // so the number of stores the next tile's first waits let pass is known.
     int tm, tn;
-    place(seq, tm, tn);
+    const int part = place(seq, tm, tn);
     auto residual = [&](int m, int n0) -> uint2 {
       if constexpr (RES) return *reinterpret_cast<const uint2 *>(p.res + (size_t)m * p.n_out + n0);
       return make_uint2(0u, 0u);
@@ -308,7 +314,18 @@ __global__ void __launch_bounds__(512, 2) pgemm_kernel(const PgemmParams p) {
     };
     constexpr int NI = GLU ? WN / 2 : WN;
     const int m_base = (tm * S::Xf + wm * XW) * 16 + col;
-    if ((tm + 1) * S::Xf * 16 <= p.rows) {
+    if constexpr (PARTS) {
+      // a k part's sums, merged by the row norm that reads the residual next
+#pragma unroll
+      for (int q = 0; q < XW; ++q) {
+        const int m = m_base + q * 16;
+        if (m >= p.rows) continue;
+#pragma unroll
+        for (int i = 0; i < WN; ++i)
+          *reinterpret_cast<f32x4_t *>(p.parts + ((size_t)part * p.rows + m) * p.n_out + wtile(tn, wf(i)) * 16 + 4 * grp) =
+              acc[i][q];
+      }
+    } else if ((tm + 1) * S::Xf * 16 <= p.rows) {
 #pragma unroll
       for (int q0 = 0; q0 < XW; q0 += 2) {
         uint2 rv[2][NI];  // residuals of two row fragments, loaded together
@@ -915,11 +932,19 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
 namespace {
 template <int WN>
 hipError_t launch_pgemm_tile(const PgemmParams &p, uint32_t flags, hipStream_t s) {
-  const int T = p.wg_n * (p.tiles / PgTile<WN>::Xf);
-  const dim3 grid(T < kPgWorkgroups ? T : kPgWorkgroups), block(512);
+  const int T = p.wg_n * (p.tiles / PgTile<WN>::Xf) * p.ksplit;
+  // A whole number per XCD: an XCD's tiles never outnumber its workgroups
+  // while the launch has fewer tiles than CUs.
+  const dim3 grid(T < kPgWorkgroups ? (T + 7) / 8 * 8 : kPgWorkgroups), block(512);
   switch (flags) {
     case 0u: hipLaunchKernelGGL((pgemm_kernel<0u, WN>), grid, block, 0, s, p); return hipSuccess;
     case QDEC_RES_OUT: hipLaunchKernelGGL((pgemm_kernel<QDEC_RES_OUT, WN>), grid, block, 0, s, p); return hipSuccess;
+    case kPgParts:
+      if constexpr (WN == 4) {
+        hipLaunchKernelGGL((pgemm_kernel<kPgParts, WN>), grid, block, 0, s, p);
+        return hipSuccess;
+      }
+      return hipErrorInvalidValue;
     case QDEC_GLU:
       if constexpr (WN % 2 == 0) {
         hipLaunchKernelGGL((pgemm_kernel<QDEC_GLU, WN>), grid, block, 0, s, p);
@@ -944,6 +969,7 @@ hipError_t launch_pgemm_small(const PgemmParams &p, uint32_t flags, hipStream_t 
 
 hipError_t launch_pgemm(const PgemmParams &p, uint32_t flags, hipStream_t s) {
   if (p.tile_rows == 64) return launch_pgemm_small(p, flags, s);
+  if (p.parts) flags = kPgParts;
   switch (p.tile_cols) {
     case 256: return launch_pgemm_tile<8>(p, flags, s);
     case 160: return launch_pgemm_tile<5>(p, flags, s);

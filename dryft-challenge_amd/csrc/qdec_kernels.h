@@ -220,6 +220,8 @@ struct PgemmParams {
   int tile_rows; // activation rows per workgroup tile: 256 or 64
   int tile_cols; // weight rows per workgroup tile: 128, 160 or 256 (64 with 64 rows)
   int wg_n;      // workgroup tiles along n
+  int ksplit;    // 256-row tiles: k parts, each its own tiles
+  float *parts;  // RES_OUT: [ksplit][rows][n] sums left instead of the update
 };
 hipError_t launch_pgemm(const PgemmParams &p, uint32_t flags, hipStream_t s);
 
@@ -244,7 +246,7 @@ struct PattnParams {
 hipError_t launch_prefill_attn(const PattnParams &p, hipStream_t s);
 
 hipError_t launch_rownorm_rows(const void *x, const void *norm_w, void *out, float eps, int rows, int k,
-                               int tiles, hipStream_t s);
+                               int tiles, const float *parts, int nparts, void *merged, hipStream_t s);
 // One workgroup per 16-row tile (prefill.hip): for k up to 4096 and enough
 // rows to fill the GPU.
 bool pnorm_fits(int k, int rows);

@@ -145,6 +145,10 @@ class Lib:
             fn.restype = ctypes.c_int
         so.qdec_gemm_wide_workspace.argtypes = [ctypes.POINTER(GemmArgs), ctypes.POINTER(ctypes.c_size_t)]
         so.qdec_gemm_wide_workspace.restype = ctypes.c_int
+        so.qdec_rownorm_merge.argtypes = [ctypes.POINTER(RownormArgs), P, I32, P, P]
+        so.qdec_rownorm_merge.restype = ctypes.c_int
+        so.qdec_prefill_gemm_split.argtypes = [ctypes.POINTER(PgemmArgs), P, I32, P]
+        so.qdec_prefill_gemm_split.restype = ctypes.c_int
         so.qdec_gemm_prepass.argtypes = [ctypes.POINTER(GemmArgs), ctypes.POINTER(I32)]
         so.qdec_gemm_prepass.restype = ctypes.c_int
 
@@ -204,6 +208,13 @@ class Lib:
 
     def rownorm(self, args, stream):
         self._check("qdec_rownorm", self.so.qdec_rownorm(ctypes.byref(args), stream))
+
+    def rownorm_merge(self, args, parts, nparts, merged, stream):
+        self._check("qdec_rownorm_merge", self.so.qdec_rownorm_merge(ctypes.byref(args), parts, nparts, merged, stream))
+
+    def prefill_gemm_split(self, args, parts, ksplit, stream):
+        self._check("qdec_prefill_gemm_split",
+                    self.so.qdec_prefill_gemm_split(ctypes.byref(args), parts, ksplit, stream))
 
     def prefill_gemm(self, args, stream):
         self._check("qdec_prefill_gemm", self.so.qdec_prefill_gemm(ctypes.byref(args), stream))

@@ -41,15 +41,19 @@ ATTN_MAX_T = 16
 # the 256 x 256 product tile (32 x 4096 prompts: 1.33 s at 16K rows, 1.27 s
 # at 32K, 1.29 s at 64K; the tokens are the same for any chunking).
 PREFILL_ROWS = 32768
-# Row tile of the prefill product (kPgRows of qdec_kernels.h); a chunk of
-# fewer rows is padded to PREFILL_ROW_TILE_SMALL instead (kPgRowsSmall, the
-# 64 x 64 tile), see prefill_tiles.
+# Row tile of the prefill product (kPgRows of qdec_kernels.h); a chunk of at
+# most PREFILL_WIDE_ROWS rows is padded to PREFILL_ROW_TILE_SMALL instead
+# (kPgRowsSmall, the 64 x 64 tile), see prefill_tiles.
 PREFILL_ROW_TILE = 256
 PREFILL_ROW_TILE_SMALL = 64
-# A prompt of at most this many rows in all (batch x length) runs its layer
-# products through qdec_gemm_wide instead of the matrix-core prefill products,
-# which make too few workgroups at so few rows.
-PREFILL_SKINNY_ROWS = 128
+# A prompt of at most PREFILL_SKINNY_ROWS rows in all (batch x length), in one
+# chunk, leaves most CUs idle in the prefill products: up to PREFILL_WIDE_ROWS
+# it runs through qdec_gemm_wide, which streams each weight once for all rows,
+# and above that O and down split k (prefill_split).  The sums then depend on
+# the row count; larger prompts, and any prompt in several chunks, take the
+# unsplit products, whose sums do not.
+PREFILL_WIDE_ROWS = 128
+PREFILL_SKINNY_ROWS = 2048
 # lm_head output tiles per workgroup from 2 rows (the role plan's 4 stays at
 # 1 row).  Grouping changes no sum and the argmax partials are scanned
 # lowest index first, so tokens and logits do not depend on it (MI355X,
@@ -157,11 +161,27 @@ def round_up(x, m):
 
 def prefill_tiles(rows):
     """16-row tiles of a prefill chunk of ``rows`` rows: rows rounded up to
-    PREFILL_ROW_TILE_SMALL below PREFILL_ROW_TILE, else to PREFILL_ROW_TILE.
-    So a short prompt's products run over its rows rounded up to 64, not to
-    a whole 256-row tile."""
-    g = PREFILL_ROW_TILE_SMALL if rows < PREFILL_ROW_TILE else PREFILL_ROW_TILE
+    PREFILL_ROW_TILE_SMALL up to PREFILL_WIDE_ROWS, else to PREFILL_ROW_TILE.
+    So a short chunk's products run over its rows rounded up to 64, not to
+    a whole 256-row tile (which at 140 to 255 rows pays: gate/up 43 -> 40 us
+    on 256 x 128 tiles, and O and down split k on them)."""
+    g = PREFILL_ROW_TILE_SMALL if rows <= PREFILL_WIDE_ROWS else PREFILL_ROW_TILE
     return round_up(rows, g) // 16
+
+
+def prefill_split(rows, n, k):
+    """k parts of O and down of a whole prompt of ``rows`` rows: the most, up
+    to 8, whose 256 x 128 tiles still run in one round of the 256 CUs.
+    MI355X, us with the row norm behind it, unsplit / split: down at 140 rows
+    49 / 28.5 (8 parts), 512 62 / 41.5 (4), 1024 96 / 68 (2), 1500 137 / 85
+    (2), 2048 (1 part fills the CUs; 2 would take 132) 126; O at 140 26 / 23,
+    512 32 / 28.6, 1024 45 / 39, 1500 63 / 48."""
+    tiles, parts = round_up(rows, PREFILL_ROW_TILE) // PREFILL_ROW_TILE * (n // 128), 1
+    if n % 128:
+        return 1
+    while parts < 8 and 2 * parts * tiles <= 256 and k % (64 * 2 * parts) == 0:
+        parts *= 2
+    return parts
 
 
 class ModelConfig:
@@ -956,8 +976,7 @@ class Prefill:
         self.state = state
         self.max_chunk = max(1, rows // B)
         self.chunk = min(prompt_len, self.max_chunk)
-        # The whole prompt in one chunk of at most PREFILL_SKINNY_ROWS rows:
-        # the weight-streaming products (_skinny_layers).
+        # The whole prompt in one chunk of at most PREFILL_SKINNY_ROWS rows.
         self.skinny = B * prompt_len <= min(PREFILL_SKINNY_ROWS, B * self.max_chunk)
         rows = prefill_tiles(B * self.chunk) * 16
         dev, bf = state.model.device, torch.bfloat16
@@ -968,6 +987,7 @@ class Prefill:
         self.act = torch.zeros((rows * c.inter,), dtype=bf, device=dev)
         self.ids = torch.zeros((rows,), dtype=torch.int64, device=dev)
         self._skinny_bufs, self._skinny_calls = None, {}
+        self._split_bufs = None
 
     def _skinny_layers(self, R):
         """Every layer's four products over all R prompt rows (row b*S + t)
@@ -981,7 +1001,7 @@ class Prefill:
         st, m, c = self.state, self.state.model, self.state.model.cfg
         dev, H, nqd = m.device, c.hidden, c.nq * c.head_dim
         split = {role: step_plan(H, k, role, MANY_ROWS_MIN_BATCH)[0] for role, k in (("o", nqd), ("down", c.inter))}
-        rows = self.state.batch * self.chunk  # the most this Prefill runs
+        rows = min(self.state.batch * self.chunk, PREFILL_WIDE_ROWS)  # the most this path runs
         if self._skinny_bufs is None:
             xn = -(-rows // 16) * 16 * H  # the pre-pass's rows (qdec_gemm_wide_workspace)
             self._skinny_bufs = (torch.zeros_like(self.h),
@@ -1034,7 +1054,7 @@ class Prefill:
         """Whether qdec_gemm_wide takes this model's products (k / 128 whole
         in every role)."""
         c = self.state.model.cfg
-        return R >= 9 and all(k % 128 == 0 for k in (c.hidden, c.nq * c.head_dim, c.inter))
+        return 9 <= R <= PREFILL_WIDE_ROWS and all(k % 128 == 0 for k in (c.hidden, c.nq * c.head_dim, c.inter))
 
     def _gemm(self, x, w, out, n, k, rows, tiles, flags=0, res=None, out_frag=0):
         a = capi.PgemmArgs()
@@ -1087,13 +1107,44 @@ class Prefill:
                     lib.gemm_wide(g_gu, s)
                     lib.gemm_wide(g_dn, s)
                 continue
+            # O and down of a short whole prompt leave k parts of their update
+            # (pending) to the next row norm, which merges them into the
+            # other of two residual buffers.
+            sp_o = prefill_split(R, H, c.nq * D) if self.skinny and R > PREFILL_WIDE_ROWS else 1
+            sp_dn = prefill_split(R, H, c.inter) if self.skinny and R > PREFILL_WIDE_ROWS else 1
+            res, other, parts = self.h, None, None
+            if sp_o > 1 or sp_dn > 1:
+                if self._split_bufs is None:  # prefill_split bounds parts x rows x n
+                    self._split_bufs = (torch.zeros_like(self.h), torch.zeros((256 * PREFILL_ROW_TILE * 128,),
+                                                                              dtype=torch.float32, device=m.device))
+                other, parts = self._split_bufs
+            pending = 0
+
+            def norm_rows(norm_w):
+                nonlocal res, other, pending
+                norm.x, norm.norm_w = res.data_ptr(), norm_w.data_ptr() if norm_w is not None else None
+                if pending:
+                    lib.rownorm_merge(norm, parts.data_ptr(), pending, other.data_ptr(), s)
+                    res, other, pending = other, res, 0
+                else:
+                    lib.rownorm(norm, s)
+
+            def res_product(g, w, split):
+                nonlocal pending
+                g.w = w.data_ptr()
+                g.out = g.res = res.data_ptr()
+                if split > 1:
+                    lib.prefill_gemm_split(g, parts.data_ptr(), split, s)
+                    pending = split
+                else:
+                    lib.prefill_gemm(g, s)
+
             g_qkv = self._gemm(self.xn, m.w_qkv[0], self.qkv, c.n_qkv, H, R, tiles)
             g_o = self._gemm(self.att, m.w_o[0], self.h, H, c.nq * D, R, tiles, capi.RES_OUT, res=self.h)
             g_gu = self._gemm(self.xn, m.w_gu[0], self.act, 2 * c.inter, H, R, tiles, capi.GLU, out_frag=1)
             g_dn = self._gemm(self.act, m.w_down[0], self.h, H, c.inter, R, tiles, capi.RES_OUT, res=self.h)
             for i in range(c.n_layers):
-                norm.norm_w = m.in_w[i].data_ptr()
-                lib.rownorm(norm, s)
+                norm_rows(m.in_w[i])
                 g_qkv.w = m.w_qkv[i].data_ptr()
                 lib.prefill_gemm(g_qkv, s)
                 qk.q_norm_w, qk.k_norm_w = m.q_norm[i].data_ptr(), m.k_norm[i].data_ptr()
@@ -1101,14 +1152,14 @@ class Prefill:
                 lib.prefill_qk(qk, s)
                 at.k_cache, at.v_cache = qk.k_cache, qk.v_cache
                 lib.prefill_attn(at, s)
-                g_o.w = m.w_o[i].data_ptr()
-                lib.prefill_gemm(g_o, s)
-                norm.norm_w = m.post_w[i].data_ptr()
-                lib.rownorm(norm, s)
+                res_product(g_o, m.w_o[i], sp_o)
+                norm_rows(m.post_w[i])
                 g_gu.w = m.w_gu[i].data_ptr()
                 lib.prefill_gemm(g_gu, s)
-                g_dn.w = m.w_down[i].data_ptr()
-                lib.prefill_gemm(g_dn, s)
+                res_product(g_dn, m.w_down[i], sp_dn)
+            if pending:
+                norm_rows(None)  # only the merge is needed
+            last = res
         # The last position of every sequence: final norm, lm_head, argmax.
         st.h[:B].copy_(last[:B * T].view(B, T, H)[:, T - 1])
         lib.gemm(st._gemm_args("lm", 0, B, ids_out=st.ids, pending=False), s)

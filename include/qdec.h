@@ -473,6 +473,11 @@ typedef struct {
   int32_t tiles;      /* >= ceil(rows / 16) */
 } qdec_rownorm_args;
 int qdec_rownorm(const qdec_rownorm_args *a, qdec_stream_t stream);
+/* The same of rows that still owe a split residual update: first
+ * x = bf16(x + bf16(((p0 + p1) + p2) + ...)) over parts[j][rows][k], j < nparts
+ * (1..8), written to merged ([rows, k] bf16, not x itself). */
+int qdec_rownorm_merge(const qdec_rownorm_args *a, const float *parts, int32_t nparts, void *merged,
+                       qdec_stream_t stream);
 
 /* out = x @ W^T on the matrix cores for x in fragment order (`tiles` M
  * tiles, a multiple of 16), W tiled [n, k].  A workgroup computes tile_rows
@@ -503,6 +508,12 @@ typedef struct {
   int32_t tile_cols; /* 0, 128 or 256 (with 256 rows), 64 (with 64 rows) */
 } qdec_pgemm_args;
 int qdec_prefill_gemm(const qdec_pgemm_args *a, qdec_stream_t stream);
+/* QDEC_RES_OUT with k in ksplit parts (1..8, each a multiple of 64): the sums
+ * of part j are left in parts[j][rows][n] (16-byte aligned) and neither res nor
+ * out is touched; qdec_rownorm_merge applies the update.  On 256 x 128 tiles
+ * (tile 0 x 0, `tiles` a multiple of 16).  For row counts whose output tiles
+ * alone leave most CUs idle. */
+int qdec_prefill_gemm_split(const qdec_pgemm_args *a, float *parts, int32_t ksplit, qdec_stream_t stream);
 
 /* Per-head RMSNorm (q_norm / k_norm) and RoPE of every row's query and key
  * heads, with the arithmetic of qdec_attn; the rotated keys and the raw

@@ -290,3 +290,65 @@ def test_prefill_gemm_walked_tiles_bitexact(lib, rows, n, k, tile):
             cols = n // 2 if flags == capi.GLU else n
             got, want = frag_to_rows(got, rows, cols, tiles), frag_to_rows(want, rows, cols, tiles)
         assert torch.equal(got, want), (flags, frag)
+
+
+@pytest.mark.parametrize("rows,n,k,parts", [(1, 128, 128, 2), (140, 2560, 4096, 8), (300, 512, 1536, 4), (513, 256, 448, 7),
+                                            (256, 384, 64, 1)])
+def test_prefill_gemm_split_and_merge(lib, rows, n, k, parts):
+    """k parts left by the product and merged by the row norm: each part's
+    sums exact on small integers; the merged residual and the normalised rows
+    those of a plain row norm over the residual with the parts added in
+    order."""
+    from qdec import capi
+    x, w = small_ints(rows, k, seed=rows), small_ints(n, k, seed=n + k)
+    tiles = round_up(rows, ROW_TILE) // 16
+    xf, wp = to_frag(lib, x, tiles), pack(lib, w)
+    res = small_ints(rows, n, lo=-8, hi=8, seed=3)
+    rd = res.to(DEV)
+    ps = torch.full((parts, rows, n), float("nan"), device=DEV)
+    a = capi.PgemmArgs(x=xf.data_ptr(), w=wp.data_ptr(), out=rd.data_ptr(), res=rd.data_ptr(), flags=capi.RES_OUT,
+                       rows=rows, n=n, k=k, tiles=tiles)
+    lib.prefill_gemm_split(a, ps.data_ptr(), parts, stream())
+    torch.cuda.synchronize()
+    kp = k // parts
+    for j in range(parts):
+        ref = x[:, j * kp:(j + 1) * kp].float() @ w[:, j * kp:(j + 1) * kp].float().T
+        assert torch.equal(ps[j].cpu(), ref), j
+    assert torch.equal(rd.cpu(), res)
+    nw = rnd(n, seed=8).to(DEV)
+    merged = torch.zeros(rows, n, dtype=torch.bfloat16, device=DEV)
+    out = torch.zeros(tiles * 16 * n, dtype=torch.bfloat16, device=DEV)
+    r = capi.RownormArgs(x=rd.data_ptr(), norm_w=nw.data_ptr(), out=out.data_ptr(), eps=1e-6, rows=rows, k=n, tiles=tiles)
+    lib.rownorm_merge(r, ps.data_ptr(), parts, merged.data_ptr(), stream())
+    torch.cuda.synchronize()
+    want = bf16(res.float() + bf16(x.float() @ w.float().T)).to(torch.bfloat16)
+    assert torch.equal(merged.cpu(), want)
+    assert torch.equal(out.cpu(), to_frag(lib, want, tiles, norm_w=nw.cpu()).cpu())
+    with pytest.raises(capi.QdecError):
+        lib.prefill_gemm_split(a, ps.data_ptr(), 9, stream())
+    with pytest.raises(capi.QdecError):
+        lib.rownorm_merge(r, ps.data_ptr(), parts, rd.data_ptr(), stream())
+
+
+def test_long_prompt_chunking_bitexact(lib):
+    """Past PREFILL_SKINNY_ROWS no product splits k, so position chunks of any
+    length leave the same bits (their attention reads the earlier chunks from
+    the cache)."""
+    from qdec.checkpoint import generate_tensors, qwen3_config
+    from qdec.runtime import PREFILL_SKINNY_ROWS, DecodeState, DeviceModel, Prefill
+    cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024)
+    model = DeviceModel(cfg, dict(generate_tensors(cfg, seed=3, norm_jitter=0.05)), DEV)
+    B, S = 3, 701
+    assert B * S > PREFILL_SKINNY_ROWS
+    prompt = torch.randint(0, 1024, (B, S), generator=torch.Generator().manual_seed(1)).to(DEV)
+    states = []
+    for rows in (None, 50 * B, 300 * B):
+        st = DecodeState(model, B, S + 18, max_t=16, keep_logits=True)
+        if rows:
+            st._prefill = Prefill(st, S, rows=rows)
+        st.prefill(prompt)
+        states.append(st)
+    torch.cuda.synchronize()
+    for st in states[1:]:
+        assert torch.equal(st.k_cache, states[0].k_cache) and torch.equal(st.v_cache, states[0].v_cache)
+        assert torch.equal(st.logits[:B], states[0].logits[:B])
