@@ -702,20 +702,20 @@ constexpr int kPaWph = 2;
 // G query heads per workgroup out of GS per kv head: GS / G workgroups per
 // (kv head, row block), each reading the kv head's K/V (8 heads in one
 // workgroup would need 64 accumulator rows per wave and spill).
-template <int G, int GS>
+template <int G, int GS, int MT>
 __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnParams p) {
   constexpr int D = 128;
-  constexpr int MT = 4 / kPaWph;               // M tiles of 16 positions per wave
+  constexpr int ROWS = 16 * MT * kPaWph;       // positions per workgroup
   constexpr int NWV = G * kPaWph;              // waves
   constexpr int NSUB = GS / G;                 // workgroups per (kv head, row block)
-  static_assert(MT == 2 && GS % G == 0 && 16 % NWV == 0, "two tiles per wave; whole fragments per wave");
+  static_assert((MT == 1 || MT == 2) && GS % G == 0 && 16 % NWV == 0, "whole fragments per wave");
   constexpr int FPW = (kPaKFrags + kPaVFrags) / NWV;  // fragments each wave loads per block
   __shared__ uint4 lds[kPaRing * kPaBlockVec];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, grp = lane >> 4;
   const int head = wave % G, half = wave / G;  // query head of the group, which 16*MT positions
   const int T = p.t_rows;
-  const int nqb = (T + kPaRows - 1) / kPaRows;
+  const int nqb = (T + ROWS - 1) / ROWS;
   const int cells = p.batch * p.nkv * NSUB;
   const int qb = nqb - 1 - (int)(blockIdx.x / cells);  // longest rows first
   const int cell = (int)(blockIdx.x % cells);
@@ -723,9 +723,9 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
   const int b = bk / p.nkv, kvh = bk - b * p.nkv;
   const int hq = kvh * GS + sub * G + head;
   const int width = (p.nq + 2 * p.nkv) * D;
-  const int t0 = qb * kPaRows;
+  const int t0 = qb * ROWS;
   const int tw = t0 + half * 16 * MT;  // this wave's first position
-  const int tlast = min(T, t0 + kPaRows) - 1;
+  const int tlast = min(T, t0 + ROWS) - 1;
   const int last = p.pos0 + tlast;  // highest slot any row of the block sees
   const int nb = last / 32 + 1;
   const size_t slab = ((size_t)b * p.nkv + kvh) * (size_t)p.cap * D;
@@ -733,7 +733,7 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
   const uint16_t *vc = p.v_cache + slab;
   const float NEG_INF = -__builtin_huge_valf();
   const float scale = p.scale_log2;
-  const bool rows_full = t0 + kPaRows - 1 <= tlast;  // all 64 rows are real
+  const bool rows_full = t0 + ROWS - 1 <= tlast;  // all rows are real
 
   // Queries as B operands: row col of M tile mt, channels 32s + 8*grp.
   uint4 qf[MT][4];
@@ -817,7 +817,7 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
   read_k(0);
   Scores s0, s1;
 #pragma unroll
-  for (int i = 0; i < 8 * MT; ++i) score1(s0, i >> 2, (i >> 1) & 1, i & 1);
+  for (int i = 0; i < 8 * MT; ++i) score1(s0, i / (2 * MT), (i >> 1) % MT, i & 1);
   await(min(1, nb - 1), kPaRing - 2);
   if (kPaRing - 1 < nb) dma_block(kPaRing - 1);
   read_k(1);
@@ -865,12 +865,12 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
     for (int u = 0; u < MT; ++u)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const int i = u * 8 + e;  // MFMA i of the scores: k step i / 4, tile, slot half
+        const int i = u * 8 + e;  // MFMA i of the scores: k step, tile, slot half
         float x = e < 4 ? S.a[u][e] : S.b[u][e - 4];
         pin(x);
         pj[u][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(x, scale, -mc[u]));
-        score1(N, i >> 2, (i >> 1) & 1, i & 1);
-        pin((i & 1) ? N.b[(i >> 1) & 1] : N.a[(i >> 1) & 1]);
+        score1(N, i / (2 * MT), (i >> 1) % MT, i & 1);
+        pin((i & 1) ? N.b[(i >> 1) % MT] : N.a[(i >> 1) % MT]);
         if (i > 0) psum[(i - 1) >> 3] += pj[(i - 1) >> 3][(i - 1) & 7];
         pin(pj[u][e]);
       }
@@ -1004,19 +1004,28 @@ hipError_t launch_pnorm(const void *x, const void *norm_w, void *out, float eps,
 }
 
 namespace {
+// Short prompts: one M tile per wave (32 positions per workgroup) while 64
+// positions leave more than half of the CUs idle -- a block takes a wave
+// about as long as its latencies, however few rows it carries.  MI355X, us
+// (64 positions / 32): one sequence of 300 tokens 19.2 / 12.3, 512 28.2 / 18.0,
+// 1024 49.5 / 31.7; 128 positions after 2000 cached 88 / 52; 8 x 128 13.6 /
+// 10.4.
 template <int G, int GS>
-void launch_pattn(const PattnParams &p, int blocks, hipStream_t s) {
-  hipLaunchKernelGGL((pattn_kernel<G, GS>), dim3(blocks * (GS / G)), dim3(64 * G * kPaWph), 0, s, p);
+void launch_pattn(const PattnParams &p, hipStream_t s) {
+  const int cells = p.batch * p.nkv * (GS / G);
+  const int b64 = (p.t_rows + kPaRows - 1) / kPaRows * cells, b32 = (p.t_rows + kPaRows / 2 - 1) / (kPaRows / 2) * cells;
+  if (b64 <= 128)
+    hipLaunchKernelGGL((pattn_kernel<G, GS, 1>), dim3(b32), dim3(64 * G * kPaWph), 0, s, p);
+  else
+    hipLaunchKernelGGL((pattn_kernel<G, GS, 2>), dim3(b64), dim3(64 * G * kPaWph), 0, s, p);
 }
 }  // namespace
 
 hipError_t launch_prefill_attn(const PattnParams &p, hipStream_t s) {
-  const int nqb = (p.t_rows + kPaRows - 1) / kPaRows;
-  const int blocks = nqb * p.batch * p.nkv;
   switch (p.nq / p.nkv) {
-    case 2: launch_pattn<2, 2>(p, blocks, s); break;
-    case 4: launch_pattn<4, 4>(p, blocks, s); break;
-    case 8: launch_pattn<4, 8>(p, blocks, s); break;
+    case 2: launch_pattn<2, 2>(p, s); break;
+    case 4: launch_pattn<4, 4>(p, s); break;
+    case 8: launch_pattn<4, 8>(p, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipSuccess;
