@@ -331,6 +331,15 @@ def step_plan(n, k, role, batch, split_o=True):
 # is mixed (1024 tokens 2.195 / 2.228, 2048 2.404 / 2.283: ten chunks to
 # merge), and batch 1 (2.089 / 2.077) stays on 4.
 ATTN8_MIN_BATCH = 3
+# Above this batch (8 kv heads: more than one workgroup per CU) a state of at
+# least ATTN4_MIN_CAP slots runs 4 waves again: two workgroups share a CU, and
+# one's prologue and merge run beside the other's stream instead of in a round
+# of their own (four layers, us, 8 / 4 waves: 33 sequences at 1000 tokens 500
+# / 486, 48 at 500 452 / 438, 64 at 500 477 / 471, 64 at 1500 643 / 632; 32 at
+# 4096 652 / 658).  No speculation runs there, so the count may depend on the
+# capacity.
+ATTN8_MAX_BATCH = 32
+ATTN4_MIN_CAP = 512
 # Rows per sequence an 8-wave attention workgroup takes (two M tiles of
 # query rows per kv head).
 ATTN8_MAX_T = 8
@@ -521,6 +530,8 @@ class DecodeState:
         # head_dim 64 (the tiny test configurations): four 16-channel output
         # tiles, one per wave of a 4-wave workgroup
         self.attn_waves = attn_waves(batch) if c.head_dim == 128 else 4
+        if batch > ATTN8_MAX_BATCH and self.cap >= ATTN4_MIN_CAP:
+            self.attn_waves = 4
         assert self.attn_waves == 4 or self.max_t <= 8
         cache_shape = (L, batch, c.nkv, self.cap, D)
         self.k_cache = torch.zeros(cache_shape, dtype=bf, device=dev)
@@ -995,7 +1006,8 @@ class Prefill:
         the last one.  O and down split k as step_plan splits them and leave
         their partials to the next NORM_IN call's pre-pass, which merges them
         into the other of two residual buffers; the last layer's down, which
-        no call follows, does not split.  Built once per row count."""
+        no call follows, leaves its parts to the merge that ``run`` adds.
+        Built once per row count."""
         if R in self._skinny_calls:
             return self._skinny_calls[R]
         st, m, c = self.state, self.state.model, self.state.model.cfg
@@ -1042,12 +1054,18 @@ class Prefill:
             gu.out, gu.out_frag = self.act.data_ptr(), 1
             norm_in(gu, m.post_w[i])
             down = args("down", i, H, c.inter, capi.RES_OUT, m.w_down)
-            res_out(down, self.act, split["down"] if i + 1 < c.n_layers else 1)
+            res_out(down, self.act, split["down"])
             layers.append((qkv, o, gu, down))
         for a in layers[0]:
             if st.lib.gemm_wide_workspace(a) > partial.numel() * 2:
                 raise RuntimeError(f"prefill: {R} rows need {st.lib.gemm_wide_workspace(a)} bytes of scratch")
-        self._skinny_calls[R] = (layers, bufs[cur])
+        merge = None
+        if pending:
+            merge = capi.RownormArgs()
+            merge.x, merge.out, merge.rows, merge.k, merge.tiles = (bufs[cur].data_ptr(), self.xn.data_ptr(), R, H,
+                                                                    -(-R // 16))
+            cur = 1 - cur
+        self._skinny_calls[R] = (layers, merge, pending, bufs[cur])
         return self._skinny_calls[R]
 
     def _skinny_fits(self, R):
@@ -1095,7 +1113,7 @@ class Prefill:
             at.head_dim, at.cap, at.tiles = D, st.cap, tiles
             if self.skinny and self._skinny_fits(R):
                 at.tiles = -(-R // 16)  # the fragment order of qdec_gemm
-                layers, last = self._skinny_layers(R)
+                layers, merge, pending, last = self._skinny_layers(R)
                 for i, (g_qkv, g_o, g_gu, g_dn) in enumerate(layers):
                     lib.gemm_wide(g_qkv, s)
                     qk.q_norm_w, qk.k_norm_w = m.q_norm[i].data_ptr(), m.k_norm[i].data_ptr()
@@ -1106,6 +1124,8 @@ class Prefill:
                     lib.gemm_wide(g_o, s)
                     lib.gemm_wide(g_gu, s)
                     lib.gemm_wide(g_dn, s)
+                if merge is not None:
+                    lib.rownorm_merge(merge, self._skinny_bufs[1].data_ptr(), pending, last.data_ptr(), s)
                 continue
             # O and down of a short whole prompt leave k parts of their update
             # (pending) to the next row norm, which merges them into the
