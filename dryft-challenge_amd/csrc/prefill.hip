@@ -490,119 +490,131 @@ __global__ void __launch_bounds__(256, 1) pgemm_small_kernel(const PgemmParams p
 }
 
 // ------------------------------------------------------- head norm + RoPE
-constexpr int kPqHeadsPerWave = kPqMaxHeads / 4;  // per wave of the per-row kernel
+// 16 lanes hold a head, 8 channels each, so a wave normalises and rotates 4
+// heads at once with one reciprocal square root for all of them: the sum of
+// squares is 3 additions in a lane, then the 16 lanes of a DPP row (the
+// pairing of the full butterfly over 2-channel lanes that the decode kernels
+// use, so the bits are theirs), and RoPE's partner channel i +- 64 is the
+// lane 8 further round the row.  With 2 channels per lane the vector units
+// bounded it: 8192 rows of 32 + 8 heads took 75 us.
+constexpr int kPqBatch = 5;  // heads per lane loaded before the first is reduced
+typedef uint32_t u32x4a4_t __attribute__((ext_vector_type(4), aligned(4)));
 
-// Few rows: one workgroup per row, wave w normalising and rotating heads w,
-// w+4, ...  The values move in groups of 8 slots, the channel-major V
-// cache's 16-byte cells: the row that starts a group (its slot a multiple of
-// 8, or the call's first row) writes every row of the group that the call
-// holds, one vector per (kv head, channel) when all 8 are there, element by
-// element at the call's ragged ends.
-__global__ void __launch_bounds__(256) pqk_row_kernel(const PqkParams p) {
-  constexpr int D = 128;
-  const int m = blockIdx.x;
-  const int b = m / p.t_rows, t = m - b * p.t_rows;
-  const int pos = p.pos0 + t;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int width = (p.nq + 2 * p.nkv) * D;
-  uint16_t *row = p.qkv + (size_t)m * width;
-  const uint32_t cw = *reinterpret_cast<const uint32_t *>(p.cos_tab + (size_t)pos * D + 2 * lane);
-  const uint32_t sw = *reinterpret_cast<const uint32_t *>(p.sin_tab + (size_t)pos * D + 2 * lane);
-  const uint32_t qw = *reinterpret_cast<const uint32_t *>(p.q_norm_w + 2 * lane);
-  const uint32_t kw = *reinterpret_cast<const uint32_t *>(p.k_norm_w + 2 * lane);
-  // Every head of this wave loaded before the first is reduced, so their
-  // latencies overlap (the host admits at most 4 * kPqHeadsPerWave heads).
-  const int nh = p.nq + p.nkv;
-  uint32_t raw[kPqHeadsPerWave];
-#pragma unroll
-  for (int j = 0; j < kPqHeadsPerWave; ++j) {
-    const int h = wave + 4 * j;
-    raw[j] = h < nh ? *reinterpret_cast<const uint32_t *>(row + (size_t)h * D + 2 * lane) : 0u;
-  }
-#pragma unroll
-  for (int j = 0; j < kPqHeadsPerWave; ++j) {
-    const int h = wave + 4 * j;
-    if (h >= nh) break;
-    const uint32_t o = head_norm_rope2(raw[j], h < p.nq ? qw : kw, cw, sw, p.eps);
-    if (h < p.nq)
-      *reinterpret_cast<uint32_t *>(row + (size_t)h * D + 2 * lane) = o;
-    else
-      *reinterpret_cast<uint32_t *>(p.k_cache + (((size_t)b * p.nkv + (h - p.nq)) * p.cap + pos) * D + 2 * lane) = o;
-  }
-  if ((pos & 7) != 0 && t != 0) return;  // another row writes this group
-  const int n = min(8 - (pos & 7), p.t_rows - t);  // rows of the group in this call
-  for (int i = threadIdx.x; i < p.nkv * D; i += blockDim.x) {
-    const int kvh = i >> 7, ch = i & 127;
-    const uint16_t *src = row + (size_t)(p.nq + p.nkv + kvh) * D + ch;
-    uint16_t *vb = p.v_cache + ((size_t)b * p.nkv + kvh) * p.cap * D + ((size_t)(pos >> 3) * D + ch) * 8;
-    if (n == 8) {
-      uint16_t v[8];
-#pragma unroll
-      for (int r = 0; r < 8; ++r) v[r] = src[(size_t)r * width];
-      *reinterpret_cast<uint4 *>(vb) = make_uint4(v[0] | ((uint32_t)v[1] << 16), v[2] | ((uint32_t)v[3] << 16),
-                                                  v[4] | ((uint32_t)v[5] << 16), v[6] | ((uint32_t)v[7] << 16));
-    } else {
-      for (int r = 0; r < n; ++r) vb[(pos & 7) + r] = src[(size_t)r * width];
-    }
-  }
+// Tables and norm weights are only promised to be aligned to 4 bytes.
+__device__ __forceinline__ uint4 ld16a4(const uint16_t *p) {
+  const u32x4a4_t v = *reinterpret_cast<const u32x4a4_t *>(p);
+  return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-// Many rows: a workgroup takes 8 consecutive positions of one sequence.  Wave w
-// normalises and rotates the 40 heads of rows 2w and 2w+1 (queries back into
-// qkv, keys into the K cache); then each thread moves the raw values of 4
-// (kv head, channel) pairs: 8 positions of one channel are one 16-byte
-// vector of the channel-major V cache when the group starts on a multiple of
-// 8 slots and is complete (element stores otherwise).
-constexpr int kPqRows = 8;
+__device__ __forceinline__ uint4 head_norm_rope8(const uint4 &raw, const uint4 &w, const uint4 &cw, const uint4 &sw,
+                                                 bool first_half, float eps) {
+  float x[8], g[8], c[8], s[8], y[8], o[8];
+  unpack8(raw, x);
+  unpack8(w, g);
+  unpack8(cw, c);
+  unpack8(sw, s);
+  float q[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    q[e] = x[2 * e] * x[2 * e] + x[2 * e + 1] * x[2 * e + 1];
+    pin(q[e]);
+  }
+  float ss = (q[0] + q[1]) + (q[2] + q[3]);
+  ss += dpp_f<0xB1>(ss);   // quad_perm [1,0,3,2]
+  ss += dpp_f<0x4E>(ss);   // quad_perm [2,3,0,1]
+  ss += dpp_f<0x141>(ss);  // row_half_mirror
+  ss += dpp_f<0x140>(ss);  // row_mirror
+  const float rstd = 1.0f / sqrtf(ss / 128.0f + eps);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] = rbf(g[e] * rbf(x[e] * rstd));
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float r = dpp_f<0x128>(y[e]);  // row_ror:8
+    o[e] = rbf(y[e] * c[e]) + rbf((first_half ? -r : r) * s[e]);
+  }
+  return pack8(o);
+}
 
+// ROWS = 1: a workgroup per row, its waves taking 4 heads each in turn.
+// ROWS = 8: a workgroup takes the positions of one sequence that share a
+// group of 8 slots, each wave two of them.  The values move in groups of 8 slots, the channel-major
+// V cache's 16-byte cells: two channels of a kv head per thread, 4 bytes of
+// each of the group's rows, element by element at the call's ragged ends.
+// With ROWS = 1 the row that starts a group (its slot a multiple of 8, or
+// the call's first row) writes every row of the group that the call holds.
+template <int ROWS>
 __global__ void __launch_bounds__(256) pqk_kernel(const PqkParams p) {
   constexpr int D = 128;
   const int T = p.t_rows;
-  const int ngrp = (T + kPqRows - 1) / kPqRows;
-  const int b = blockIdx.x / ngrp, t0 = (blockIdx.x - b * ngrp) * kPqRows;
-  const int nrow = min(kPqRows, T - t0);
+  const int off = p.pos0 & (ROWS - 1);  // groups start on multiples of 8 slots
+  const int ngrp = (T + off + ROWS - 1) / ROWS;
+  const int b = blockIdx.x / ngrp, g0 = (blockIdx.x - b * ngrp) * ROWS - off;
+  const int t0 = max(g0, 0);
+  const int nrow = min(g0 + ROWS, T) - t0;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ch8 = (lane & 15) * 8;
+  const bool first_half = (lane & 15) < 8;
   const int width = (p.nq + 2 * p.nkv) * D;
   uint16_t *rows = p.qkv + (size_t)(b * T + t0) * width;
-  const uint32_t qw = *reinterpret_cast<const uint32_t *>(p.q_norm_w + 2 * lane);
-  const uint32_t kw = *reinterpret_cast<const uint32_t *>(p.k_norm_w + 2 * lane);
-#pragma unroll
-  for (int i = 0; i < kPqRows / 4; ++i) {
-    const int r = wave * (kPqRows / 4) + i;
+  const uint4 qw = ld16a4(p.q_norm_w + ch8), kw = ld16a4(p.k_norm_w + ch8);
+  constexpr int RW = ROWS == 1 ? 1 : ROWS / 4;  // rows of a wave
+  constexpr int HS = ROWS == 1 ? 16 : 4;        // heads normalised at once on a row
+  const int h0 = (lane >> 4) + (ROWS == 1 ? 4 * wave : 0);
+  const int nh = p.nq + p.nkv;
+  for (int i = 0; i < RW; ++i) {
+    const int r = ROWS == 1 ? 0 : wave * RW + i;
     if (r >= nrow) break;
     const int pos = p.pos0 + t0 + r;
-    uint16_t *row = rows + (size_t)r * width;
-    const uint32_t cw = *reinterpret_cast<const uint32_t *>(p.cos_tab + (size_t)pos * D + 2 * lane);
-    const uint32_t sw = *reinterpret_cast<const uint32_t *>(p.sin_tab + (size_t)pos * D + 2 * lane);
-    for (int h = 0; h < p.nq + p.nkv; ++h) {
-      uint32_t *cell = reinterpret_cast<uint32_t *>(row + (size_t)h * D + 2 * lane);
-      const uint32_t o = head_norm_rope2(*cell, h < p.nq ? qw : kw, cw, sw, p.eps);
-      if (h < p.nq)
-        *cell = o;
-      else
-        *reinterpret_cast<uint32_t *>(p.k_cache + (((size_t)b * p.nkv + (h - p.nq)) * p.cap + pos) * D + 2 * lane) = o;
+    uint16_t *row = rows + (size_t)r * width + ch8;
+    uint16_t *kc = p.k_cache + ((size_t)b * p.nkv * p.cap + pos) * D + ch8;
+    const uint4 cw = ld16a4(p.cos_tab + (size_t)pos * D + ch8), sw = ld16a4(p.sin_tab + (size_t)pos * D + ch8);
+    for (int hb = 0; hb < nh; hb += HS * kPqBatch) {
+      uint4 raw[kPqBatch];
+#pragma unroll
+      for (int j = 0; j < kPqBatch; ++j) {
+        const int h = hb + h0 + HS * j;
+        raw[j] = h < nh ? ld16(row + (size_t)h * D) : zero4();
+      }
+#pragma unroll
+      for (int j = 0; j < kPqBatch; ++j) {
+        const int h = hb + h0 + HS * j;
+        const uint4 o = head_norm_rope8(raw[j], h < p.nq ? qw : kw, cw, sw, first_half, p.eps);
+        if (h < nh)
+          *reinterpret_cast<uint4 *>(h < p.nq ? row + (size_t)h * D : kc + (size_t)(h - p.nq) * p.cap * D) = o;
+      }
     }
   }
   const int slot0 = p.pos0 + t0;
-  const bool whole = nrow == kPqRows && (slot0 & 7) == 0;
-  for (int i = threadIdx.x; i < p.nkv * D; i += blockDim.x) {
-    const int kvh = i >> 7, ch = i & 127;
+  int n = nrow;  // rows to move, from slot0
+  if (ROWS == 1) {
+    if ((slot0 & 7) != 0 && t0 != 0) return;  // another row writes this group
+    n = min(8 - (slot0 & 7), T - t0);
+  }
+  const bool whole = n == 8 && (slot0 & 7) == 0;
+  for (int i = threadIdx.x; i < p.nkv * (D / 2); i += blockDim.x) {
+    const int kvh = i >> 6, ch = (i & 63) * 2;
     const uint16_t *src = rows + (size_t)(p.nq + p.nkv + kvh) * D + ch;
     uint16_t *vb = p.v_cache + ((size_t)b * p.nkv + kvh) * p.cap * D;
     if (whole) {
-      uint16_t v[kPqRows];
+      uint32_t v[8];
 #pragma unroll
-      for (int r = 0; r < kPqRows; ++r) v[r] = src[(size_t)r * width];
-      uint4 o;
-      o.x = v[0] | ((uint32_t)v[1] << 16);
-      o.y = v[2] | ((uint32_t)v[3] << 16);
-      o.z = v[4] | ((uint32_t)v[5] << 16);
-      o.w = v[6] | ((uint32_t)v[7] << 16);
-      *reinterpret_cast<uint4 *>(vb + ((size_t)(slot0 >> 3) * D + ch) * 8) = o;
+      for (int r = 0; r < 8; ++r) v[r] = *reinterpret_cast<const uint32_t *>(src + (size_t)r * width);
+      uint32_t lo[4], hi[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        lo[r] = (v[2 * r] & 0xffffu) | (v[2 * r + 1] << 16);
+        hi[r] = (v[2 * r] >> 16) | (v[2 * r + 1] & 0xffff0000u);
+      }
+      uint4 *dst = reinterpret_cast<uint4 *>(vb + ((size_t)(slot0 >> 3) * D + ch) * 8);
+      dst[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+      dst[1] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
     } else {
-      for (int r = 0; r < nrow; ++r) {
+      for (int r = 0; r < n; ++r) {
         const int slot = slot0 + r;
-        vb[((size_t)(slot >> 3) * D + ch) * 8 + (slot & 7)] = src[(size_t)r * width];
+        const uint32_t v = *reinterpret_cast<const uint32_t *>(src + (size_t)r * width);
+        uint16_t *cell = vb + ((size_t)(slot >> 3) * D + ch) * 8 + (slot & 7);
+        cell[0] = (uint16_t)v;
+        cell[8] = (uint16_t)(v >> 16);
       }
     }
   }
@@ -977,19 +989,25 @@ hipError_t launch_pgemm(const PgemmParams &p, uint32_t flags, hipStream_t s) {
   }
 }
 
-// Grouped row kernels from this many rows (below it one workgroup per row
-// or per 16-row tile leaves the GPU short of workgroups: a 512-token prompt
-// measured 10.0 ms with the per-row kernels and 11.8 with the grouped ones;
-// 32 x 1024-row chunks 5% faster with the grouped ones).
+// Row norms by whole 16-row tiles from this many rows (below it the tiles
+// leave the GPU short of workgroups: a 512-token prompt measured 10.0 ms with
+// the per-row kernels and 11.8 with the grouped ones; 32 x 1024-row chunks 5%
+// faster with the grouped ones).
 constexpr int kGroupedRows = 4096;
+// Head norms and RoPE by groups of 8 slots from this many rows: us grouped /
+// per row with 32 + 8 heads: 512 rows 12.6 / 6.9, 1000 14.0 / 11.6, 1500
+// 14.2 / 15.4, 4096 23.7 / 30.2, 8192 38 / 54, 32768 162 / 239.  (A lane per
+// 2 channels, and groups aligned to the call instead of the cache: 512 rows
+// 8.3, 8192 62, 32768 225, and 3000 rows from slot 1 the V cache element by
+// element.)
+constexpr int kPqGroupedRows = 1280;
 
 hipError_t launch_prefill_qk(const PqkParams &p, hipStream_t s) {
-  if (p.batch * p.t_rows < kGroupedRows) {
-    hipLaunchKernelGGL(pqk_row_kernel, dim3(p.batch * p.t_rows), dim3(256), 0, s, p);
+  if (p.batch * p.t_rows < kPqGroupedRows) {
+    hipLaunchKernelGGL(pqk_kernel<1>, dim3(p.batch * p.t_rows), dim3(256), 0, s, p);
     return hipSuccess;
   }
-  const int ngrp = (p.t_rows + kPqRows - 1) / kPqRows;
-  hipLaunchKernelGGL(pqk_kernel, dim3(p.batch * ngrp), dim3(256), 0, s, p);
+  hipLaunchKernelGGL(pqk_kernel<8>, dim3(p.batch * (((p.pos0 & 7) + p.t_rows + 7) / 8)), dim3(256), 0, s, p);
   return hipSuccess;
 }
 

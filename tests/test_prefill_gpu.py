@@ -267,6 +267,35 @@ def test_prefill_qk_and_attention_vs_oracle(lib, B, T, pos0, cap):
     assert err <= 0.02 * ref.abs().max().item(), err
 
 
+# Calls of 1280 rows or more work on groups of 8 slots, smaller ones row by
+# row: the same sequences in one grouped call and one call each, bit for bit,
+# with groups cut at the front, at the end and at both.
+@pytest.mark.parametrize("B,T,pos0,nq,nkv", [(1300, 1, 7, 4, 2), (400, 5, 6, 6, 2), (3, 517, 3, 64, 8), (2, 641, 8, 17, 3)])
+def test_prefill_qk_grouped_rows_bitexact(lib, B, T, pos0, nq, nkv):
+    from qdec import capi
+    cap = round_up(pos0 + T, 32)
+    qkv0 = rnd(B * T, (nq + 2 * nkv) * D, seed=B).to(DEV)
+    qn, kn, cos, sin = (rnd(*shape, seed=i).to(DEV) for i, shape in enumerate([(D,), (D,), (cap, D), (cap, D)]))
+    got = []
+    for step in (B, 1):
+        qkv = qkv0.clone()
+        kc = torch.zeros(B, nkv, cap, D, dtype=torch.bfloat16, device=DEV)
+        vc = torch.zeros(B, nkv, cap // 8, D, 8, dtype=torch.bfloat16, device=DEV)
+        for b in range(0, B, step):
+            q = capi.PrefillQkArgs()
+            q.qkv, q.q_norm_w, q.k_norm_w, q.cos_tab, q.sin_tab = (qkv[b * T:].data_ptr(), qn.data_ptr(), kn.data_ptr(),
+                                                                  cos.data_ptr(), sin.data_ptr())
+            q.k_cache, q.v_cache, q.eps = kc[b:].data_ptr(), vc[b:].data_ptr(), 1e-6
+            q.batch, q.t_rows, q.pos0, q.nq, q.nkv, q.head_dim, q.cap = step, T, pos0, nq, nkv, D, cap
+            lib.prefill_qk(q, stream())
+        torch.cuda.synchronize()
+        got.append((qkv, kc, vc))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    v = qkv0.view(B, T, nq + 2 * nkv, D)[:, :, nq + nkv:].transpose(1, 2)
+    assert torch.equal(got[0][2].transpose(-1, -2).reshape(B, nkv, cap, D)[:, :, pos0:pos0 + T], v)
+
+
 # The 256-row tiles run as one workgroup per CU walking several tiles: more
 # tiles than workgroups (a last round that is not full), fewer than eight
 # (fewer workgroups than XCDs), row counts that leave the last row tile
