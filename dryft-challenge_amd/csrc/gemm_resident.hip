@@ -326,12 +326,7 @@ __global__ void __launch_bounds__(64 * 4 * (GLU ? kResMaxPairs : kResMaxTiles1))
   if constexpr (GLU) {
     float o4[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float g = rbf(ag[i]);
-      const float u = rbf(au[i]);
-      const float sg = rbf(g / (1.0f + expf(-g)));
-      o4[i] = sg * u;
-    }
+    for (int i = 0; i < 4; ++i) o4[i] = swiglu(rbf(ag[i]), rbf(au[i]));
     o.x = pack2(o4[0], o4[1]);
     o.y = pack2(o4[2], o4[3]);
   } else {
@@ -526,12 +521,7 @@ __global__ void __launch_bounds__(64 * 4 * kResMaxPairs) glu_resident2_kernel(co
     if constexpr (GLU) {
       float o4[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float g = rbf(ag[mt][i]);
-        const float u = rbf(au[mt][i]);
-        const float sg = rbf(g / (1.0f + expf(-g)));
-        o4[i] = sg * u;
-      }
+      for (int i = 0; i < 4; ++i) o4[i] = swiglu(rbf(ag[mt][i]), rbf(au[mt][i]));
       o.x = pack2(o4[0], o4[1]);
       o.y = pack2(o4[2], o4[3]);
     } else {

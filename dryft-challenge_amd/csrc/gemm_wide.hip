@@ -147,7 +147,7 @@ __global__ void __launch_bounds__(256, (FLAGS & QDEC_ARGMAX) ? 2 : 1) wide_kerne
       const float g4[4] = {rbf(s.x), rbf(s.y), rbf(s.z), rbf(s.w)}, u4[4] = {rbf(up.x), rbf(up.y), rbf(up.z), rbf(up.w)};
       float o4[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o4[e] = rbf(g4[e] / (1.0f + expf(-g4[e]))) * u4[e];
+      for (int e = 0; e < 4; ++e) o4[e] = swiglu(g4[e], u4[e]);
       const int n0 = unit * 8 + grp * 4;
       uint16_t *out = reinterpret_cast<uint16_t *>(p.out);
       *reinterpret_cast<uint2 *>(p.ofrag ? out + frag_off(m, n0, p.ofrag) : out + (size_t)m * p.n + n0) =

@@ -79,9 +79,6 @@ struct Int {
   static constexpr int value = V;
 };
 
-// SwiGLU of one gate / up pair, both already rounded: bf16(silu(g)) * u.
-__device__ __forceinline__ float swiglu(float g, float u) { return rbf(g / (1.0f + expf(-g))) * u; }
-
 // Tiles of 256 rows x (32 WN) columns, eight waves as 2 (columns) x 4 (rows),
 // each WN weight x 4 activation fragments: 256 x 256 (WN 8, 32 KiB stages,
 // RING 5), 256 x 160 (WN 5, 26 KiB, RING 6) and 256 x 128 (WN 4, 24 KiB,

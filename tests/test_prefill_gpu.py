@@ -381,3 +381,27 @@ def test_long_prompt_chunking_bitexact(lib):
     for st in states[1:]:
         assert torch.equal(st.k_cache, states[0].k_cache) and torch.equal(st.v_cache, states[0].v_cache)
         assert torch.equal(st.logits[:B], states[0].logits[:B])
+
+
+@pytest.mark.parametrize("tile", [(64, 64), (256, 256)])
+def test_prefill_gemm_silu_of_every_gate_value(lib, tile):
+    """One-hot rows pick each finite bf16 value as a gate, with an up value
+    of 1: silu in 64 bits rounded to bf16, at most one unit in the last place
+    away where an fp32 result rounds the other way (fewer than 1 in 1000),
+    and nothing but flushed values below the normal range."""
+    from qdec import capi
+    k = 256
+    g = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    g = torch.where(torch.isfinite(g), g, torch.zeros_like(g)).view(256, k)
+    w = torch.cat([g, torch.ones(256, k, dtype=torch.bfloat16)])
+    x = torch.eye(k, dtype=torch.bfloat16)
+    tiles = k // 16
+    out = pgemm(lib, to_frag(lib, x, tiles), pack(lib, w), k, 512, k, tiles, flags=capi.GLU, tile=tile).cpu()
+    gd = g.T.double()
+    ref = (gd / (1 + torch.exp(-gd))).to(torch.bfloat16)
+    normal = gd.abs() >= 2.0 ** -125
+    ulps = (out.view(torch.int16).int() - ref.view(torch.int16).int()).abs()
+    deep = ref.abs().float() < 2.0 ** -120
+    assert ulps[normal & ~deep].max() <= 1
+    assert (ulps[normal & ~deep] == 0).float().mean() >= 0.999
+    assert (out[deep | ~normal].float().abs() < 2.0 ** -119).all()
