@@ -119,6 +119,25 @@ def test_rownorm_layout_and_norm(lib, rows):
     assert exact >= 0.99
 
 
+@pytest.mark.parametrize("k", [96, 1024, 1056, 2048, 2080, 2560, 2592, 4096])
+@pytest.mark.parametrize("norm", [True, False])
+def test_rownorm_tiles_bitexact(lib, k, norm):
+    """4096 rows or more go by 16-row tiles, each width's form at its edges:
+    the per-row kernel's bits, and zeros past the last row."""
+    rows = 4101
+    x = rnd(rows, k, scale=3, seed=k)
+    x[5] *= 1e-4  # eps counts
+    w = rnd(k, seed=1) if norm else None
+    tiles = round_up(rows, ROW_TILE) // 16
+    got = frag_to_rows(to_frag(lib, x, tiles, norm_w=w), tiles * 16, k, tiles).cpu()
+    for i in (0, 2048, 4096):
+        part = x[i:i + 2048]
+        pt = round_up(part.shape[0], 16) // 16
+        want = frag_to_rows(to_frag(lib, part, pt, norm_w=w), part.shape[0], k, pt).cpu()
+        assert torch.equal(got[i:i + part.shape[0]].view(torch.int16), want.view(torch.int16))
+    assert (got[rows:] == 0).all()
+
+
 TILES = [(256, 128), (256, 256), (64, 64)]
 
 
