@@ -356,7 +356,9 @@ static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch, 
   if (p->lds_bytes > (size_t)kGemmLdsX)
     return set_error(QDEC_EUNSUPPORTED, "qdec_gemm: rows %d x waves %d needs %zu B of LDS", a->rows, a->waves,
                      p->lds_bytes);
-  p->wide = p->xd && many;
+  // (The many-row kernel reads fragment order only: 9 to 16 row-major rows
+  // that no LDS plan holds stay on the direct path.)
+  p->wide = p->xd && p->xt && many;
   // Norm hand-over to the next NORM_IN call (gemm_dev.h hand_over_row).
   p->hnorm_w = nullptr;
   p->hxn = nullptr;

@@ -165,6 +165,19 @@ def test_short_ring_bitexact(lib, kind, n, k, waves):
         assert torch.equal(got.contiguous().view(torch.int16), want[rows].view(torch.int16)), rows
 
 
+@pytest.mark.parametrize("kind,n,k", [("res", 48, 9728), ("plain", 48, 1152)])
+def test_row_major_rows_bitexact(lib, kind, n, k):
+    """9 to 16 row-major rows that do not fit LDS (k = 9728), or whose k range
+    no load ring divides, take the direct path: the bits of fragment order."""
+    call = Call(lib, kind, n, k, 1, seed=n + k)
+    x, res = rnd(16, k, scale=2.0, seed=5), rnd(16, n, seed=6)
+    want = call(x, res, False)[0]
+    call.row_major = True
+    for rows in (9, 13, 16):
+        got = call(x[:rows].contiguous(), res[:rows].contiguous(), False)[0]
+        assert torch.equal(got.contiguous().view(torch.int16), want[:rows].contiguous().view(torch.int16)), rows
+
+
 def test_wide_refusals(lib):
     from qdec import capi
     x, out = rnd(128, 256), torch.zeros(128, 64, dtype=torch.bfloat16, device=DEV)
