@@ -215,6 +215,12 @@ class ModelConfig:
         (DecodeState.prefill_steps)."""
         return self.head_dim == 128 and self.group in (2, 4, 8) and self.nq + self.nkv <= 80
 
+    @property
+    def wide_widths(self):
+        """Whether qdec_gemm_wide takes this model's products (k / 128 whole
+        in every role)."""
+        return all(k % 128 == 0 for k in (self.hidden, self.nq * self.head_dim, self.inter))
+
     def check_supported(self):
         problems = []
         if self.head_dim not in (128, 64):
@@ -925,7 +931,9 @@ class DecodeState:
             raise ValueError(f"prompt batch {B} != state batch {self.batch}")
         if S < 1 or S >= self.cap:
             raise ValueError(f"prompt length {S} must be in [1, {self.cap})")
-        if S <= max_rows_per_seq(B, group=self.model.cfg.group) or not self.model.cfg.prefill_kernels:
+        c = self.model.cfg
+        if (S <= max_rows_per_seq(B, group=c.group) or not c.prefill_kernels
+                or (B * S <= GEMM_MAX_ROWS and not c.wide_widths)):
             # A prompt one decode step holds goes through the decode kernels:
             # with few rows the prefill products have too few workgroups
             # (MI355X, time to the first token, 16 tokens: 3.08 ms against
@@ -1068,12 +1076,6 @@ class Prefill:
         self._skinny_calls[R] = (layers, merge, pending, bufs[cur])
         return self._skinny_calls[R]
 
-    def _skinny_fits(self, R):
-        """Whether qdec_gemm_wide takes this model's products (k / 128 whole
-        in every role)."""
-        c = self.state.model.cfg
-        return 9 <= R <= PREFILL_WIDE_ROWS and all(k % 128 == 0 for k in (c.hidden, c.nq * c.head_dim, c.inter))
-
     def _gemm(self, x, w, out, n, k, rows, tiles, flags=0, res=None, out_frag=0):
         a = capi.PgemmArgs()
         a.x, a.w, a.out = x.data_ptr(), w.data_ptr(), out.data_ptr()
@@ -1085,9 +1087,6 @@ class Prefill:
         st = self.state
         m, c, lib = st.model, st.model.cfg, st.lib
         B, S = prompt.shape
-        if self.skinny and B * S <= GEMM_MAX_ROWS and not self._skinny_fits(B * S):
-            st.prefill_steps(prompt, stream=stream)
-            return
         s = (stream or torch.cuda.current_stream(m.device)).cuda_stream
         H, D = c.hidden, c.head_dim
         T, last = self.chunk, self.h
@@ -1111,7 +1110,7 @@ class Prefill:
             at.qkv, at.out, at.sm_scale = self.qkv.data_ptr(), self.att.data_ptr(), D ** -0.5
             at.batch, at.t_rows, at.pos0, at.nq, at.nkv = B, T, c0, c.nq, c.nkv
             at.head_dim, at.cap, at.tiles = D, st.cap, tiles
-            if self.skinny and self._skinny_fits(R):
+            if self.skinny and 9 <= R <= PREFILL_WIDE_ROWS and c.wide_widths:
                 at.tiles = -(-R // 16)  # the fragment order of qdec_gemm
                 layers, merge, pending, last = self._skinny_layers(R)
                 for i, (g_qkv, g_o, g_gu, g_dn) in enumerate(layers):
