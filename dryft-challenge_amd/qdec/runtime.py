@@ -995,8 +995,6 @@ class Prefill:
         self.state = state
         self.max_chunk = max(1, rows // B)
         self.chunk = min(prompt_len, self.max_chunk)
-        # The whole prompt in one chunk of at most PREFILL_SKINNY_ROWS rows.
-        self.skinny = B * prompt_len <= min(PREFILL_SKINNY_ROWS, B * self.max_chunk)
         rows = prefill_tiles(B * self.chunk) * 16
         dev, bf = state.model.device, torch.bfloat16
         self.h = torch.zeros((rows, c.hidden), dtype=bf, device=dev)
@@ -1024,9 +1022,9 @@ class Prefill:
         rows = min(self.state.batch * self.chunk, PREFILL_WIDE_ROWS)  # the most this path runs
         if self._skinny_bufs is None:
             xn = -(-rows // 16) * 16 * H  # the pre-pass's rows (qdec_gemm_wide_workspace)
-            self._skinny_bufs = (torch.zeros_like(self.h),
-                                 torch.zeros((max(split.values()) * rows * H,), dtype=torch.float32, device=dev),
-                                 torch.zeros((xn + 128,), dtype=torch.bfloat16, device=dev))
+            self._skinny_bufs = (torch.empty((rows, H), dtype=torch.bfloat16, device=dev),
+                                 torch.empty((max(split.values()) * rows * H,), dtype=torch.float32, device=dev),
+                                 torch.empty((xn + 128,), dtype=torch.bfloat16, device=dev))
         other, parts, partial = self._skinny_bufs
         bufs = (self.h, other)
 
@@ -1087,6 +1085,10 @@ class Prefill:
         st = self.state
         m, c, lib = st.model, st.model.cfg, st.lib
         B, S = prompt.shape
+        # The whole prompt in one chunk of at most PREFILL_SKINNY_ROWS rows.
+        # Decided by the prompt, not by the first one this object saw, so a
+        # short prompt gives the same bits whatever ran before it.
+        self.skinny = S <= self.chunk and B * S <= PREFILL_SKINNY_ROWS
         s = (stream or torch.cuda.current_stream(m.device)).cuda_stream
         H, D = c.hidden, c.head_dim
         T, last = self.chunk, self.h
@@ -1134,8 +1136,10 @@ class Prefill:
             res, other, parts = self.h, None, None
             if sp_o > 1 or sp_dn > 1:
                 if self._split_bufs is None:  # prefill_split bounds parts x rows x n
-                    self._split_bufs = (torch.zeros_like(self.h), torch.zeros((256 * PREFILL_ROW_TILE * 128,),
-                                                                              dtype=torch.float32, device=m.device))
+                    self._split_bufs = (torch.empty((min(len(self.h), PREFILL_SKINNY_ROWS), H), dtype=torch.bfloat16,
+                                                    device=m.device),
+                                        torch.empty((256 * PREFILL_ROW_TILE * 128,), dtype=torch.float32,
+                                                    device=m.device))
                 other, parts = self._split_bufs
             pending = 0
 

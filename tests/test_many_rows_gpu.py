@@ -194,15 +194,16 @@ def test_wide_refusals(lib):
 
 def test_short_prompts_of_several_lengths_in_one_state(lib):
     """One state prefills prompts of different lengths one after the other:
-    each leaves what a fresh state leaves."""
+    each leaves what a fresh state leaves, a short one after a long one
+    (unsplit products) too."""
     from qdec.checkpoint import generate_tensors, qwen3_config
     from qdec.runtime import DecodeState, DeviceModel
     cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024)
     model = DeviceModel(cfg, dict(generate_tensors(cfg, seed=3, norm_jitter=0.05)), DEV)
-    shared = DecodeState(model, 2, 160, max_t=16, keep_logits=True)
-    for S in (60, 25, 64, 40, 130, 33):
+    shared = DecodeState(model, 2, 1120, max_t=16, keep_logits=True)
+    for S in (60, 25, 64, 40, 130, 33, 1100, 33, 400, 64):
         prompt = torch.randint(0, 1024, (2, S), generator=torch.Generator().manual_seed(S)).to(DEV)
-        fresh = DecodeState(model, 2, 160, max_t=16, keep_logits=True)
+        fresh = DecodeState(model, 2, 1120, max_t=16, keep_logits=True)
         for st in (shared, fresh):
             st.prefill(prompt)
         torch.cuda.synchronize()
