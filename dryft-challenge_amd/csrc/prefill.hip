@@ -791,7 +791,7 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
   float m_run[MT], l_run[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    m_run[mt] = -1e30f;
+    m_run[mt] = NEG_INF;
     l_run[mt] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) acc[mt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};

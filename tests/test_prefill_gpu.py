@@ -286,6 +286,32 @@ def test_prefill_qk_and_attention_vs_oracle(lib, B, T, pos0, cap):
     assert err <= 0.02 * ref.abs().max().item(), err
 
 
+@pytest.mark.parametrize("T,pos0", [(1, 0), (40, 0), (70, 33), (300, 5)])
+def test_prefill_attention_of_very_low_scores(lib, T, pos0):
+    """Every score the same -2^112 (powers of two: exact), far below any
+    finite start of the running maximum: the probabilities are equal, so a
+    row is the mean of the values it sees (bf16 rounds it once; sums of small
+    integers are exact)."""
+    from qdec import capi
+    nkv, cap = 2, round_up(pos0 + T, 32)
+    nq = 4 * nkv
+    qkv = torch.full((T, (nq + 2 * nkv) * D), 2.0 ** 55, dtype=torch.bfloat16, device=DEV)
+    kc = torch.full((1, nkv, cap, D), -2.0 ** 50, dtype=torch.bfloat16, device=DEV)
+    v = small_ints(1, nkv, cap, D, lo=-8, hi=8, seed=T)
+    vc = v_layout(v).to(DEV)
+    tiles = round_up(T, 16) // 16
+    out = torch.full((tiles * 16 * nq * D,), float("nan"), dtype=torch.bfloat16, device=DEV)
+    a = capi.PrefillAttnArgs(qkv=qkv.data_ptr(), k_cache=kc.data_ptr(), v_cache=vc.data_ptr(), out=out.data_ptr(),
+                             sm_scale=0.125 / 1.4426950408889634, batch=1, t_rows=T, pos0=pos0, nq=nq, nkv=nkv,
+                             head_dim=D, cap=cap, tiles=tiles)  # in base 2 the scale is 2^-3
+    lib.prefill_attn(a, stream())
+    torch.cuda.synchronize()
+    got = frag_to_rows(out, T, nq * D, tiles).cpu().double().view(T, nkv, 4, D)
+    seen = torch.arange(pos0 + 1, pos0 + T + 1).double()[:, None, None]
+    want = (v[0].double().cumsum(1)[:, pos0:pos0 + T].transpose(0, 1) / seen)[:, :, None].expand_as(got)
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs()).all()
+
+
 # Calls of 1280 rows or more work on groups of 8 slots, smaller ones row by
 # row: the same sequences in one grouped call and one call each, bit for bit,
 # with groups cut at the front, at the end and at both.
