@@ -65,9 +65,15 @@ static void gemm_scratch(const qdec_gemm_args *a, const GemmParams &p, size_t *p
 // Whether gemm_wide.hip's 32-bit lane offsets reach the up half of w.
 static bool wide_offsets(const qdec_gemm_args *a) { return (uint64_t)a->n * a->k * 2 < (1ull << 32) - 4096; }
 
+// What a GEMM plan is for: a qdec_gemm call; qdec_gemm_wide (the many-row plan
+// or an error); a stage of qdec_layer, whose kernel has no ring of 8 (a down
+// whose k range only that ring divides keeps the direct path it is compiled
+// for).
+enum class PlanFor { kCall, kWide, kLayer };
+
 // Derive the launch plan of a GEMM call; returns QDEC_OK or an error code.
-// With `wide` the many-row plan or an error (qdec_gemm_wide).
-static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch, bool wide = false) {
+static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch, PlanFor what = PlanFor::kCall) {
+  const bool wide = what == PlanFor::kWide;
   if (!a) return set_error(QDEC_EINVAL, "qdec_gemm: null args");
   *p = GemmParams{};
   const uint32_t f = a->flags;
@@ -247,7 +253,8 @@ static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch, 
   p->xd = 0;
   p->tw = 1;
   p->xn = nullptr;
-  const int ring = gemm_ring(p->ksw, f);
+  int ring = gemm_ring(p->ksw, f);
+  if (ring == 8 && what == PlanFor::kLayer) ring = 0;
   // Direct path: two tiles per wave at two M tiles when the workgroup's
   // tiles pair up, without GLU (sums unchanged: every tile keeps its own
   // MFMA chain).  gate/up stays at one: at 32 rows its four weight streams
@@ -534,7 +541,7 @@ int plan_layer(const qdec_layer_args *a, LayerParams *L, int *workgroups, size_t
   static const uint32_t flags[4] = {QDEC_NORM_IN, QDEC_RES_OUT, QDEC_NORM_IN | QDEC_GLU, QDEC_RES_OUT};
   static const int rings[4] = {20, 16, 10, 20};
   for (int i = 0; i < 4; ++i) {
-    const int rc = plan_gemm(ga[i], &L->g[i], true);
+    const int rc = plan_gemm(ga[i], &L->g[i], true, PlanFor::kLayer);
     if (rc != QDEC_OK) return rc;
     const GemmParams &p = L->g[i];
     const bool direct = i == 3;
@@ -671,7 +678,7 @@ int qdec_gemm(const qdec_gemm_args *a, qdec_stream_t stream) {
 
 int qdec_gemm_wide_workspace(const qdec_gemm_args *a, size_t *partial_bytes) {
   GemmParams p;
-  const int rc = plan_gemm(a, &p, false, true);
+  const int rc = plan_gemm(a, &p, false, PlanFor::kWide);
   if (rc != QDEC_OK) return rc;
   size_t pb = 0, cb = 0, xn_off = 0;
   gemm_scratch(a, p, &pb, &cb, &xn_off);
@@ -681,7 +688,7 @@ int qdec_gemm_wide_workspace(const qdec_gemm_args *a, size_t *partial_bytes) {
 
 int qdec_gemm_wide(const qdec_gemm_args *a, qdec_stream_t stream) {
   GemmParams p;
-  const int rc = plan_gemm(a, &p, true, true);
+  const int rc = plan_gemm(a, &p, true, PlanFor::kWide);
   if (rc != QDEC_OK) return rc;
   return launch_status(launch_gemm(p, a->flags, (hipStream_t)stream), "qdec_gemm_wide");
 }

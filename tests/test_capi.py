@@ -337,10 +337,16 @@ def _set(obj, **kw):
     (dict(fix=_set("down", ksplit=4)), -3, "down plan"),
     (dict(fix=_set("gate_up", flags=capi.NORM_IN)), -3, "gate_up plan"),
     (dict(fix=_set("qkv", rows=2)), -3, "qkv plan"),
+    # a down whose k / 128 a ring of 8 divides, but not the longer ones, keeps
+    # the layer kernel's plan (the attention stage after it is what is refused)
+    (dict(fix=_set("down", k=9216), cap=100), -1, "cap"),
 ])
 def test_layer_validation(qlib, kw, code, needle):
-    fix = kw.pop("fix", None)
+    kw = dict(kw)
+    fix, cap = kw.pop("fix", None), kw.pop("cap", None)
     la = _layer(**kw) if fix is None else _layer(fix=fix)
+    if cap is not None:
+        la.attn.contents.cap = cap
     assert qlib.so.qdec_layer(ctypes.byref(la), None) == code
     assert needle in qlib.last_error()
     assert qlib.so.qdec_layer_prepare(ctypes.byref(la)) == code

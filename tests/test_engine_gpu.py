@@ -327,6 +327,30 @@ def test_layer_launch_equals_its_stage_launches(engine, B, S, seed):
     assert not torch.equal(snap[0], got[0])  # the step did something
 
 
+@pytest.mark.parametrize("B", [1, 4])
+def test_layer_launch_of_a_down_on_the_short_ring(B):
+    """An intermediate width of 9216: its down projection's own call stages
+    its rows with a ring of 8, which the layer kernel does not have; the
+    layer launch takes the shape all the same and gives those bits."""
+    from qdec.checkpoint import generate_tensors
+    from qdec.runtime import DecodeState, DeviceModel
+    cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024, intermediate_size=9216)
+    model = DeviceModel(cfg, dict(generate_tensors(cfg, seed=3, norm_jitter=0.05)), "cuda:0")
+    st = DecodeState(model, B, 80, max_t=1)
+    st.prefill(prompts(B, 50, 44, vocab=1024).to(model.device))
+    st.enable_layer_launch()
+    snap = _snapshot(st)
+    _stage_launches(st)
+    torch.cuda.synchronize()
+    want = _snapshot(st)
+    _restore(st, snap)
+    st.run_step(t_rows=1, lm_head=False, advance=False)
+    torch.cuda.synchronize()
+    assert st.layer_error() == 0
+    assert all(_same(g, w) for g, w in zip(_snapshot(st), want))
+    assert not torch.equal(snap[0], want[0])
+
+
 @pytest.mark.parametrize("B,S,n,seed", [(1, 60, 8, 51), (4, 45, 6, 52)])
 def test_layer_launch_vs_oracle(engine, oracle, B, S, n, seed):
     """Plain decode with one launch per layer, teacher-forced against the
