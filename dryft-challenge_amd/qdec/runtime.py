@@ -932,8 +932,7 @@ class DecodeState:
         if S < 1 or S >= self.cap:
             raise ValueError(f"prompt length {S} must be in [1, {self.cap})")
         c = self.model.cfg
-        if (S <= max_rows_per_seq(B, group=c.group) or not c.prefill_kernels
-                or (B * S <= GEMM_MAX_ROWS and not c.wide_widths)):
+        if S <= max_rows_per_seq(B, group=c.group) or not c.prefill_kernels:
             # A prompt one decode step holds goes through the decode kernels:
             # with few rows the prefill products have too few workgroups
             # (MI355X, time to the first token, 16 tokens: 3.08 ms against
@@ -982,8 +981,9 @@ class Prefill:
     attention over the cache -> O product + residual -> rownorm -> gate/up
     product with SwiGLU -> down product + residual, the products on the
     matrix cores (qdec_prefill_gemm).  A prompt of at most
-    PREFILL_SKINNY_ROWS rows runs its products as qdec_gemm_wide instead (each
-    weight streamed once for all rows).  After the last chunk the final row
+    PREFILL_WIDE_ROWS rows runs its products as qdec_gemm_wide instead (each
+    weight streamed once for all rows), or as qdec_gemm (up to GEMM_MAX_ROWS
+    rows) where a width is no multiple of 128.  After the last chunk the final row
     of each sequence goes through the decode lm_head + argmax.
 
     Replaces engine/engine.py:448-490 (``_layers_forward`` over the whole
@@ -1005,6 +1005,7 @@ class Prefill:
         self.ids = torch.zeros((rows,), dtype=torch.int64, device=dev)
         self._skinny_bufs, self._skinny_calls = None, {}
         self._split_bufs = None
+        self._gemm_scratch = None
 
     def _skinny_layers(self, R):
         """Every layer's four products over all R prompt rows (row b*S + t)
@@ -1074,6 +1075,52 @@ class Prefill:
         self._skinny_calls[R] = (layers, merge, pending, bufs[cur])
         return self._skinny_calls[R]
 
+    def _gemm_args(self, role, layer, R):
+        """qdec_gemm arguments of one layer product over all R prompt rows
+        (row b*S + t), for widths that qdec_gemm_wide does not take: x of QKV
+        and gate/up is the residual h (row-major, NORM_IN), the attention
+        output comes in fragment order, and gate/up hands its SwiGLU rows to
+        down in fragment order from FRAG_ROWS rows, as the decode step does.
+        Plans as the decode step's (two tiles per wave at 17-32 rows),
+        without a k split."""
+        m, c = self.state.model, self.state.model.cfg
+        a = capi.GemmArgs()
+        a.eps, a.rows, a.ksplit, a.waves, a.tiles_per_wg = c.eps, R, 1, m.plans[role][1], 1
+        frag = 1 if R >= FRAG_ROWS else 0
+        if role == "qkv":
+            a.x, a.w, a.out, a.norm_w = (self.h.data_ptr(), m.w_qkv[layer].data_ptr(), self.qkv.data_ptr(),
+                                         m.in_w[layer].data_ptr())
+            a.n, a.k, a.flags = c.n_qkv, c.hidden, capi.NORM_IN
+            if R >= WIDE_MIN_ROWS and c.hidden % 256 == 0:
+                a.waves = 8
+        elif role == "o":
+            a.x, a.w, a.res = self.att.data_ptr(), m.w_o[layer].data_ptr(), self.h.data_ptr()
+            a.n, a.k, a.flags, a.x_frag = c.hidden, c.nq * c.head_dim, capi.RES_OUT, 1
+        elif role == "gate_up":
+            a.x, a.w, a.out, a.norm_w = (self.h.data_ptr(), m.w_gu[layer].data_ptr(), self.act.data_ptr(),
+                                         m.post_w[layer].data_ptr())
+            a.n, a.k, a.flags, a.out_frag = c.inter, c.hidden, capi.NORM_IN | capi.GLU, frag
+        else:
+            a.x, a.w, a.res = self.act.data_ptr(), m.w_down[layer].data_ptr(), self.h.data_ptr()
+            a.n, a.k, a.flags, a.x_frag = c.hidden, c.inter, capi.RES_OUT, frag
+        if role in ("qkv", "down") and WIDE_MIN_ROWS <= R <= 32 and (a.n // 16) % WIDE_TILES == 0:
+            a.tiles_per_wg = WIDE_TILES
+        if self._gemm_scratch is not None:
+            a.partial, a.counters = (t.data_ptr() for t in self._gemm_scratch)
+        return a
+
+    def _gemm_layers(self, R):
+        """Every layer's four qdec_gemm calls (_gemm_args), their scratch
+        grown to what R rows need (the plan depends on the row count)."""
+        roles = ("qkv", "o", "gate_up", "down")
+        need = [self.state.lib.gemm_workspace(self._gemm_args(role, 0, R)) for role in roles]
+        pb, cb = (max(16, *b) // 4 + 4 for b in zip(*need))
+        if self._gemm_scratch is None or any(t.numel() < n for t, n in zip(self._gemm_scratch, (pb, cb))):
+            dev = self.state.model.device
+            self._gemm_scratch = (torch.zeros((pb,), dtype=torch.float32, device=dev),
+                                  torch.zeros((cb,), dtype=torch.int32, device=dev))
+        return [[self._gemm_args(role, i, R) for role in roles] for i in range(self.state.model.cfg.n_layers)]
+
     def _gemm(self, x, w, out, n, k, rows, tiles, flags=0, res=None, out_frag=0):
         a = capi.PgemmArgs()
         a.x, a.w, a.out = x.data_ptr(), w.data_ptr(), out.data_ptr()
@@ -1112,19 +1159,22 @@ class Prefill:
             at.qkv, at.out, at.sm_scale = self.qkv.data_ptr(), self.att.data_ptr(), D ** -0.5
             at.batch, at.t_rows, at.pos0, at.nq, at.nkv = B, T, c0, c.nq, c.nkv
             at.head_dim, at.cap, at.tiles = D, st.cap, tiles
-            if self.skinny and 9 <= R <= PREFILL_WIDE_ROWS and c.wide_widths:
+            wide = c.wide_widths and 9 <= R <= PREFILL_WIDE_ROWS
+            if self.skinny and (wide or (not c.wide_widths and R <= GEMM_MAX_ROWS)):
                 at.tiles = -(-R // 16)  # the fragment order of qdec_gemm
-                layers, merge, pending, last = self._skinny_layers(R)
+                product = lib.gemm_wide if wide else lib.gemm
+                layers, merge, pending, last = (self._skinny_layers(R) if wide
+                                                else (self._gemm_layers(R), None, 0, self.h))
                 for i, (g_qkv, g_o, g_gu, g_dn) in enumerate(layers):
-                    lib.gemm_wide(g_qkv, s)
+                    product(g_qkv, s)
                     qk.q_norm_w, qk.k_norm_w = m.q_norm[i].data_ptr(), m.k_norm[i].data_ptr()
                     qk.k_cache, qk.v_cache = st.k_cache[i].data_ptr(), st.v_cache[i].data_ptr()
                     lib.prefill_qk(qk, s)
                     at.k_cache, at.v_cache = qk.k_cache, qk.v_cache
                     lib.prefill_attn(at, s)
-                    lib.gemm_wide(g_o, s)
-                    lib.gemm_wide(g_gu, s)
-                    lib.gemm_wide(g_dn, s)
+                    product(g_o, s)
+                    product(g_gu, s)
+                    product(g_dn, s)
                 if merge is not None:
                     lib.rownorm_merge(merge, self._skinny_bufs[1].data_ptr(), pending, last.data_ptr(), s)
                 continue

@@ -211,20 +211,29 @@ def test_short_prompts_of_several_lengths_in_one_state(lib):
         assert torch.equal(shared.k_cache[:, :, :, :S], fresh.k_cache[:, :, :, :S]), S
 
 
-@pytest.mark.parametrize("B,S", [(1, 37), (3, 20)])
-def test_short_prompt_of_widths_the_wide_product_refuses(lib, B, S):
-    """Widths of 64 but not 128: a prompt of up to 64 rows goes through the
-    decode steps, and the logits are those of the last position."""
+@pytest.mark.parametrize("B,S,hidden", [(1, 37, 320), (3, 20, 320), (1, 64, 512), (2, 20, 512)])
+def test_short_prompt_of_widths_the_wide_product_refuses(lib, monkeypatch, B, S, hidden):
+    """Widths that are not all multiples of 128: a prompt of up to 64 rows is
+    one pass over the weights (qdec_gemm), not one per decode step, and its
+    logits, cache and picks agree with the decode steps' (bf16 sums in another
+    order: 2e-2 of the largest, as every end-to-end comparison here)."""
     from qdec.checkpoint import generate_tensors, qwen3_config
     from qdec.runtime import DecodeState, DeviceModel
-    cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024, hidden_size=320, intermediate_size=704,
+    cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024, hidden_size=hidden, intermediate_size=704,
                        num_attention_heads=4, num_key_value_heads=2)
     model = DeviceModel(cfg, dict(generate_tensors(cfg, seed=3, norm_jitter=0.05)), DEV)
     prompt = torch.randint(0, 1024, (B, S), generator=torch.Generator().manual_seed(S)).to(DEV)
     st, ref = (DecodeState(model, B, 160, max_t=4, keep_logits=True) for _ in range(2))
+    passes, embed = [], st.lib.embed
+    monkeypatch.setattr(st.lib, "embed", lambda e, s: (passes.append(e.rows), embed(e, s)))
     st.prefill(prompt)
+    monkeypatch.undo()
+    assert passes == [B * S]
     ref.prefill_steps(prompt)
     torch.cuda.synchronize()
     t = (S - 1) % ref.max_t + 1
-    assert torch.equal(st.logits[:B], ref.logits[:B * t].view(B, t, -1)[:, t - 1])
-    assert torch.equal(st.ids[:B], ref.ids[:B]) and torch.equal(st.k_cache, ref.k_cache)
+    logits = ref.logits[:B * t].view(B, t, -1)[:, t - 1].float()
+    assert (st.logits[:B].float() - logits).abs().max() <= 2e-2 * logits.abs().max()
+    for got, want in ((st.k_cache, ref.k_cache), (st.v_cache, ref.v_cache)):
+        assert (got.float() - want.float()).abs().max() <= 2e-2 * want.float().abs().max()
+    assert st.lens.tolist() == [S] * B
