@@ -35,6 +35,7 @@ import torch
 from . import capi
 
 GEMM_MAX_ROWS = 64
+GEMM_WIDE_MIN_ROWS = 9  # of qdec_gemm_wide
 ATTN_MAX_T = 16
 # Rows (sequences x positions) of one prefill chunk: activations of 32K rows
 # take about 2.2 GB; at that size O and down still make 1280 workgroups of
@@ -46,12 +47,12 @@ PREFILL_ROWS = 32768
 # (kPgRowsSmall, the 64 x 64 tile), see prefill_tiles.
 PREFILL_ROW_TILE = 256
 PREFILL_ROW_TILE_SMALL = 64
-# A prompt of at most PREFILL_SKINNY_ROWS rows in all (batch x length), in one
-# chunk, leaves most CUs idle in the prefill products: up to PREFILL_WIDE_ROWS
-# it runs through qdec_gemm_wide, which streams each weight once for all rows,
-# and above that O and down split k (prefill_split).  The sums then depend on
-# the row count; larger prompts, and any prompt in several chunks, take the
-# unsplit products, whose sums do not.
+# A prompt of at most PREFILL_SKINNY_ROWS rows in all (batch x length) leaves
+# most CUs idle in the prefill products: up to PREFILL_WIDE_ROWS it runs
+# through qdec_gemm_wide, which streams each weight once for all rows, and
+# above that O and down split k (prefill_split).  The sums then depend on the
+# prompt's row count, but not on the position chunks it runs in: each takes
+# the whole prompt's route.  Larger prompts take the unsplit products.
 PREFILL_WIDE_ROWS = 128
 PREFILL_SKINNY_ROWS = 2048
 # lm_head output tiles per workgroup from 2 rows (the role plan's 4 stays at
@@ -170,7 +171,7 @@ def prefill_tiles(rows):
 
 
 def prefill_split(rows, n, k):
-    """k parts of O and down of a whole prompt of ``rows`` rows: the most, up
+    """k parts of O and down of a prompt of ``rows`` rows in all: the most, up
     to 8, whose 256 x 128 tiles still run in one round of the 256 CUs.
     MI355X, us with the row norm behind it, unsplit / split: down at 140 rows
     49 / 28.5 (8 parts), 512 62 / 41.5 (4), 1024 96 / 68 (2), 1500 137 / 85
@@ -996,6 +997,8 @@ class Prefill:
         self.max_chunk = max(1, rows // B)
         self.chunk = min(prompt_len, self.max_chunk)
         rows = prefill_tiles(B * self.chunk) * 16
+        if self.chunk == self.max_chunk:  # a chunk of a longer prompt, whose split products take 256-row tiles
+            rows = round_up(rows, PREFILL_ROW_TILE)
         dev, bf = state.model.device, torch.bfloat16
         self.h = torch.zeros((rows, c.hidden), dtype=bf, device=dev)
         self.xn = torch.zeros((rows * c.hidden,), dtype=bf, device=dev)
@@ -1020,7 +1023,7 @@ class Prefill:
         st, m, c = self.state, self.state.model, self.state.model.cfg
         dev, H, nqd = m.device, c.hidden, c.nq * c.head_dim
         split = {role: step_plan(H, k, role, MANY_ROWS_MIN_BATCH)[0] for role, k in (("o", nqd), ("down", c.inter))}
-        rows = min(self.state.batch * self.chunk, PREFILL_WIDE_ROWS)  # the most this path runs
+        rows = max(GEMM_WIDE_MIN_ROWS, min(self.state.batch * self.chunk, PREFILL_WIDE_ROWS))  # the most this path runs
         if self._skinny_bufs is None:
             xn = -(-rows // 16) * 16 * H  # the pre-pass's rows (qdec_gemm_wide_workspace)
             self._skinny_bufs = (torch.empty((rows, H), dtype=torch.bfloat16, device=dev),
@@ -1132,17 +1135,18 @@ class Prefill:
         st = self.state
         m, c, lib = st.model, st.model.cfg, st.lib
         B, S = prompt.shape
-        # The whole prompt in one chunk of at most PREFILL_SKINNY_ROWS rows.
-        # Decided by the prompt, not by the first one this object saw, so a
-        # short prompt gives the same bits whatever ran before it.
-        self.skinny = S <= self.chunk and B * S <= PREFILL_SKINNY_ROWS
+        # The route of a short prompt, decided by the whole prompt: not by its
+        # chunks, nor by the first prompt this object saw.
+        wide = c.wide_widths and GEMM_WIDE_MIN_ROWS <= B * S <= PREFILL_WIDE_ROWS
+        narrow = not c.wide_widths and B * S <= GEMM_MAX_ROWS and S <= self.chunk
+        split = PREFILL_WIDE_ROWS < B * S <= PREFILL_SKINNY_ROWS
         s = (stream or torch.cuda.current_stream(m.device)).cuda_stream
         H, D = c.hidden, c.head_dim
         T, last = self.chunk, self.h
         for c0 in range(0, S, self.chunk):
             T = min(self.chunk, S - c0)
             R = B * T
-            tiles = prefill_tiles(R)
+            tiles = round_up(R, PREFILL_ROW_TILE) // 16 if split else prefill_tiles(R)
             self.ids[:R].view(B, T).copy_(prompt[:, c0:c0 + T])
             e = capi.EmbedArgs()
             e.ids, e.emb, e.h = self.ids.data_ptr(), m.emb.data_ptr(), self.h.data_ptr()
@@ -1159,11 +1163,12 @@ class Prefill:
             at.qkv, at.out, at.sm_scale = self.qkv.data_ptr(), self.att.data_ptr(), D ** -0.5
             at.batch, at.t_rows, at.pos0, at.nq, at.nkv = B, T, c0, c.nq, c.nkv
             at.head_dim, at.cap, at.tiles = D, st.cap, tiles
-            wide = c.wide_widths and 9 <= R <= PREFILL_WIDE_ROWS
-            if self.skinny and (wide or (not c.wide_widths and R <= GEMM_MAX_ROWS)):
+            if wide or narrow:
                 at.tiles = -(-R // 16)  # the fragment order of qdec_gemm
                 product = lib.gemm_wide if wide else lib.gemm
-                layers, merge, pending, last = (self._skinny_layers(R) if wide
+                # (A last chunk of fewer rows than qdec_gemm_wide takes runs
+                # with rows that nothing reads behind it.)
+                layers, merge, pending, last = (self._skinny_layers(max(R, GEMM_WIDE_MIN_ROWS)) if wide
                                                 else (self._gemm_layers(R), None, 0, self.h))
                 for i, (g_qkv, g_o, g_gu, g_dn) in enumerate(layers):
                     product(g_qkv, s)
@@ -1178,11 +1183,10 @@ class Prefill:
                 if merge is not None:
                     lib.rownorm_merge(merge, self._skinny_bufs[1].data_ptr(), pending, last.data_ptr(), s)
                 continue
-            # O and down of a short whole prompt leave k parts of their update
+            # O and down of a short prompt leave k parts of their update
             # (pending) to the next row norm, which merges them into the
             # other of two residual buffers.
-            sp_o = prefill_split(R, H, c.nq * D) if self.skinny and R > PREFILL_WIDE_ROWS else 1
-            sp_dn = prefill_split(R, H, c.inter) if self.skinny and R > PREFILL_WIDE_ROWS else 1
+            sp_o, sp_dn = (prefill_split(B * S, H, k) if split else 1 for k in (c.nq * D, c.inter))
             res, other, parts = self.h, None, None
             if sp_o > 1 or sp_dn > 1:
                 if self._split_bufs is None:  # prefill_split bounds parts x rows x n

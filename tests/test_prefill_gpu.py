@@ -404,19 +404,21 @@ def test_prefill_gemm_split_and_merge(lib, rows, n, k, parts):
         lib.rownorm_merge(r, ps.data_ptr(), parts, rd.data_ptr(), stream())
 
 
-def test_long_prompt_chunking_bitexact(lib):
-    """Past PREFILL_SKINNY_ROWS no product splits k, so position chunks of any
+@pytest.mark.parametrize("B,S", [(3, 701), (1, 1500), (2, 300), (1, 131), (2, 61)])
+def test_prompt_chunking_bitexact(lib, B, S):
+    """A prompt's route depends on all of its rows, so position chunks of any
     length leave the same bits (their attention reads the earlier chunks from
-    the cache)."""
+    the cache): unsplit products past PREFILL_SKINNY_ROWS, k parts below
+    (chunks of more and of fewer rows than a tile), qdec_gemm_wide up to
+    PREFILL_WIDE_ROWS."""
     from qdec.checkpoint import generate_tensors, qwen3_config
-    from qdec.runtime import PREFILL_SKINNY_ROWS, DecodeState, DeviceModel, Prefill
+    from qdec.runtime import PREFILL_SKINNY_ROWS, PREFILL_WIDE_ROWS, DecodeState, DeviceModel, Prefill
     cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024)
     model = DeviceModel(cfg, dict(generate_tensors(cfg, seed=3, norm_jitter=0.05)), DEV)
-    B, S = 3, 701
-    assert B * S > PREFILL_SKINNY_ROWS
+    assert (B * S > PREFILL_SKINNY_ROWS) == (S == 701) and (B * S <= PREFILL_WIDE_ROWS) == (S == 61)
     prompt = torch.randint(0, 1024, (B, S), generator=torch.Generator().manual_seed(1)).to(DEV)
     states = []
-    for rows in (None, 50 * B, 300 * B):
+    for rows in (None, 50 * B, 300 * B if S > 300 else 20 * B):
         st = DecodeState(model, B, S + 18, max_t=16, keep_logits=True)
         if rows:
             st._prefill = Prefill(st, S, rows=rows)
