@@ -534,11 +534,13 @@ __device__ __forceinline__ uint4 head_norm_rope8(const uint4 &raw, const uint4 &
 
 // ROWS = 1: a workgroup per row, its waves taking 4 heads each in turn.
 // ROWS = 8: a workgroup takes the positions of one sequence that share a
-// group of 8 slots, each wave two of them.  The values move in groups of 8 slots, the channel-major
-// V cache's 16-byte cells: two channels of a kv head per thread, 4 bytes of
-// each of the group's rows, element by element at the call's ragged ends.
-// With ROWS = 1 the row that starts a group (its slot a multiple of 8, or
-// the call's first row) writes every row of the group that the call holds.
+// group of 8 slots, each wave two of them.  The values move in groups of 8
+// slots, the channel-major V cache's 16-byte cells: two channels of a kv head
+// per thread, 4 bytes of each of the group's rows, element by element at the
+// call's ragged ends.  With ROWS = 1 the row that starts a whole group writes
+// its 8 rows; at the ragged ends each row writes its own elements (left to
+// one row of the group, that work met on one XCD where t_rows is a multiple
+// of 8: 40 sequences of 32 rows from slot 3 17.3 us, so 10.8).
 template <int ROWS>
 __global__ void __launch_bounds__(256) pqk_kernel(const PqkParams p) {
   constexpr int D = 128;
@@ -574,6 +576,7 @@ __global__ void __launch_bounds__(256) pqk_kernel(const PqkParams p) {
       }
 #pragma unroll
       for (int j = 0; j < kPqBatch; ++j) {
+        if (hb + HS * j >= nh) break;  // no head left for any lane
         const int h = hb + h0 + HS * j;
         const uint4 o = head_norm_rope8(raw[j], h < p.nq ? qw : kw, cw, sw, first_half, p.eps);
         if (h < nh)
@@ -584,8 +587,11 @@ __global__ void __launch_bounds__(256) pqk_kernel(const PqkParams p) {
   const int slot0 = p.pos0 + t0;
   int n = nrow;  // rows to move, from slot0
   if (ROWS == 1) {
-    if ((slot0 & 7) != 0 && t0 != 0) return;  // another row writes this group
-    n = min(8 - (slot0 & 7), T - t0);
+    const int g = slot0 & ~7;
+    if (g >= p.pos0 && g + 8 <= p.pos0 + T) {
+      if (slot0 != g) return;  // the group's first row writes it
+      n = 8;
+    }
   }
   const bool whole = n == 8 && (slot0 & 7) == 0;
   for (int i = threadIdx.x; i < p.nkv * (D / 2); i += blockDim.x) {
@@ -1002,12 +1008,13 @@ hipError_t launch_pgemm(const PgemmParams &p, uint32_t flags, hipStream_t s) {
 // faster with the grouped ones).
 constexpr int kGroupedRows = 4096;
 // Head norms and RoPE by groups of 8 slots from this many rows: us grouped /
-// per row with 32 + 8 heads: 512 rows 12.6 / 6.9, 1000 14.0 / 11.6, 1500
-// 14.2 / 15.4, 4096 23.7 / 30.2, 8192 38 / 54, 32768 162 / 239.  (A lane per
-// 2 channels, and groups aligned to the call instead of the cache: 512 rows
-// 8.3, 8192 62, 32768 225, and 3000 rows from slot 1 the V cache element by
-// element.)
-constexpr int kPqGroupedRows = 1280;
+// per row with 32 + 8 heads: 512 rows 12.7 / 7.4, 1500 14.3 / 12.0, 3000 22.7
+// / 20.2, 4000 23.7 / 25.7, 6000 30.9 / 35.7; with 16 + 8 heads 1500 11.1 /
+// 10.0, 3000 15.2 / 16.9, 4000 17.7 / 20.7; whatever the rows per sequence
+// (1296 rows of 8 13.8 / 11.0).  Before a lane left out the heads that its
+// row does not have, 16 + 8 heads took 10.1 us at 1000 rows (now 8.4) and 26.9
+// at 6000 (21.7).
+constexpr int kPqGroupedRows = 3584;
 
 hipError_t launch_prefill_qk(const PqkParams &p, hipStream_t s) {
   if (p.batch * p.t_rows < kPqGroupedRows) {

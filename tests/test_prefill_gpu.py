@@ -312,10 +312,12 @@ def test_prefill_attention_of_very_low_scores(lib, T, pos0):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs()).all()
 
 
-# Calls of 1280 rows or more work on groups of 8 slots, smaller ones row by
+# Calls of 3584 rows or more work on groups of 8 slots, smaller ones row by
 # row: the same sequences in one grouped call and one call each, bit for bit,
-# with groups cut at the front, at the end and at both.
-@pytest.mark.parametrize("B,T,pos0,nq,nkv", [(1300, 1, 7, 4, 2), (400, 5, 6, 6, 2), (3, 517, 3, 64, 8), (2, 641, 8, 17, 3)])
+# with groups cut at the front, at the end and at both (and row by row in one
+# call of many sequences).
+@pytest.mark.parametrize("B,T,pos0,nq,nkv", [(3600, 1, 7, 4, 2), (900, 5, 6, 6, 2), (3, 1217, 3, 64, 8), (2, 1801, 8, 17, 3),
+                                             (1300, 1, 7, 4, 2), (400, 5, 6, 16, 8), (3, 517, 3, 64, 8), (2, 641, 8, 17, 3)])
 def test_prefill_qk_grouped_rows_bitexact(lib, B, T, pos0, nq, nkv):
     from qdec import capi
     cap = round_up(pos0 + T, 32)
