@@ -272,9 +272,16 @@ static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch, 
   // rows 9.7 / 7.9, 8.3 / 7.9, 20.3 / 19.3, 13.0 / 10.3; 32 rows 12.4 / 9.5,
   // 10.2 / 9.2, 23.3 / 20.6, 16.2 / 11.3; 64 rows 16.9 / 11.4, 14.2 / 12.5,
   // 30.7 / 22.5, 22.5 / 14.6; lm_head (16896 columns) at 64 rows 46.4 / 29.5.
-  // Below 9 rows the rows stay in LDS and are normalised there.
+  // Below 9 rows the rows stay in LDS and are normalised there.  A wave's k
+  // range of 8 steps or fewer is too short for the longer start and end of a
+  // workgroup with many accumulators (graph replays, us at 16 / 32 / 48 / 64
+  // rows: 4096 x 1024 5.7 / 5.4 / 6.0 / 6.9 and 4.9 / 5.1 / 6.3 / 7.1; gate/up
+  // 3072 x 1024 6.0 / 6.6 / 7.5 / 8.3 and 5.9 / 6.9 / 8.0 / 8.8, but 2048 x
+  // 1024, one unit per workgroup, 5.7 / 6.3 / 7.2 / 8.2 and 4.9 / 5.8 / 6.3 /
+  // 7.2).
+  const bool brief = !arg && p->ksw <= 8 && (glu ? a->rows > 16 && a->n > 8 * kWideWorkgroups : a->rows > 32);
   const bool many = a->rows >= kWideMinRows && a->waves == 4 && (arg || a->tiles_per_wg == 1) &&
-                    (a->ksplit == 1 || a->parts_out) && !a->next_norm_w && wide_offsets(a);
+                    (a->ksplit == 1 || a->parts_out) && !a->next_norm_w && wide_offsets(a) && (wide || !brief);
   if (wide) {
     if (!many || arg || xa || a->resident || (!a->x_frag && !(f & QDEC_NORM_IN)))
       return set_error(QDEC_EUNSUPPORTED, "qdec_gemm_wide: needs 4 waves, one tile per workgroup, x_frag = 1 or NORM_IN, "

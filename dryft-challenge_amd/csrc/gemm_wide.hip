@@ -12,7 +12,8 @@
 // operands, for U MT products.  No operand is shared between waves, so there
 // is no LDS traffic and no barrier until the four waves' sums are added, in
 // wave order, through LDS.  One wave per SIMD has 512 registers: the
-// accumulators and a ring of RING k steps (up to 60 KiB in flight per wave).
+// accumulators and a ring of RING k steps (32 to 91 KiB per wave, of which the
+// 6-bit load counter lets 63 be in flight).
 //
 // Sums and order are those of the direct path at four waves (gemm_dev.h):
 // the same bits.  gate/up at 64 rows 30.7 -> 22.5 us per launch (3.2 -> 4.4
@@ -186,7 +187,7 @@ hipError_t launch_wide_mt(const GemmParams &p, hipStream_t s) {
   const int T = GLU ? p.n / 8 : p.n / 16;
   // The fewest units per workgroup that run in one round of the CUs (a unit
   // more costs its own loads; a second round costs the whole first again).
-  auto fits = [&](int u) { return (T + u - 1) / u * p.ksplit <= kWideWorkgroups; };
+  auto rounds = [&](int u) { return ((T + u - 1) / u * p.ksplit + kWideWorkgroups - 1) / kWideWorkgroups; };
   auto go = [&](auto kernel, int u) {
     hipLaunchKernelGGL(kernel, dim3((T + u - 1) / u * p.ksplit), dim3(256), 0, s, p);
     return hipSuccess;
@@ -194,9 +195,40 @@ hipError_t launch_wide_mt(const GemmParams &p, hipStream_t s) {
   if constexpr ((FLAGS & QDEC_ARGMAX) != 0) {
     if constexpr (MT > 4) return hipErrorInvalidValue;
     else return go(wide_kernel<MT, 3, FLAGS>, 3);
-  } else if constexpr (GLU) return fits(3) ? go(wide_kernel<MT, 3, FLAGS>, 3) : go(wide_kernel<MT, 5, FLAGS>, 5);
-  else return fits(1) ? go(wide_kernel<MT, 1, FLAGS>, 1)
-            : fits(2) ? go(wide_kernel<MT, 2, FLAGS>, 2) : go(wide_kernel<MT, 3, FLAGS>, 3);
+  } else if constexpr (GLU) {
+    // gate/up has more units than one round of few takes, and where the 256
+    // CUs do not divide them a last round runs for a few: the least of rounds
+    // x (units + row tiles / 2 beyond the first, whose fragments the
+    // workgroups share through L2).  MI355X, us at 9 / 24 / 48 / 64 rows of
+    // 12288 x 4096: per-tile kernels 32.7 / 36.7 / 41.4 / 46.2; units 2 32.7 /
+    // 38.3 / 44.1 / 49.3, 3 34.0 / 36.2 / 39.6 / 43.6, 5 (308 workgroups) 43.9
+    // / 47.4 / 50.2 / 53.9, 6 35.4 / 36.2 / 37.0 / 38.0; of 3072 x 1024: 5.9 /
+    // 6.6 / 7.5 / 8.3; 6.3 / 6.9 / 8.0 / 8.8, 3 7.3 / 8.1 / 9.4 / 9.8.
+    int best = rounds(1) == 1 ? 1 : 0, least = 0;
+    if (!best)
+      for (const int u : {2, 3, 5, 6}) {
+        if (u == 6 && MT > 6) continue;  // beyond the LDS
+        const int cost = rounds(u) * (25 * u + 13 * (MT - 1));
+        if (!best || cost < least) best = u, least = cost;
+      }
+    switch (best) {
+      case 1: return go(wide_kernel<MT, 1, FLAGS>, 1);
+      case 2: return go(wide_kernel<MT, 2, FLAGS>, 2);
+      case 3: return go(wide_kernel<MT, 3, FLAGS>, 3);
+      case 6:
+        if constexpr (MT <= 6) return go(wide_kernel<MT, 6, FLAGS>, 6);
+      default: return go(wide_kernel<MT, 5, FLAGS>, 5);
+    }
+  } else {
+    // A k split of wide outputs (Qwen3-8B's down, 256 tiles x 4) fills a
+    // round at 4 units: us at 9 / 24 / 48 / 64 rows, per-tile kernels 22.4 /
+    // 28.9 / 32.3 / 37.2, units 3 23.8 / 26.1 / 29.0 / 32.1, 4 19.1 / 19.2 /
+    // 20.7 / 22.4.
+    return rounds(1) == 1           ? go(wide_kernel<MT, 1, FLAGS>, 1)
+           : rounds(2) == 1         ? go(wide_kernel<MT, 2, FLAGS>, 2)
+           : rounds(3) <= rounds(4) ? go(wide_kernel<MT, 3, FLAGS>, 3)
+                                    : go(wide_kernel<MT, 4, FLAGS>, 4);
+  }
 }
 
 template <uint32_t FLAGS>

@@ -130,6 +130,16 @@ def test_many_rows_bitexact(lib, kind, n, k, ksplit, rows):
             assert torch.equal(g.contiguous().view(kindint), w.view(kindint)), (wide, j)
 
 
+@pytest.mark.parametrize("kind,n,k,ksplit", [("glu", 2064, 1280, 1), ("glu", 4112, 384, 1), ("glu", 12288, 384, 1),
+                                             ("parts", 4096, 1536, 4)])
+@pytest.mark.parametrize("rows", [9, 24, 96, 97])
+def test_units_per_workgroup_bitexact(lib, kind, n, k, ksplit, rows):
+    """Widths for which the launch rule picks 2, 3, 2 or 6 or 3 (by the row
+    tiles) and 4 units per workgroup, and, in qdec_gemm, k ranges short enough
+    that the per-tile kernels stay."""
+    test_many_rows_bitexact(lib, kind, n, k, ksplit, rows)
+
+
 @pytest.mark.parametrize("rows,n", [(9, 16), (16, 4112), (33, 784), (64, 16896)])
 def test_many_rows_argmax(lib, rows, n):
     """The lm_head's logits and picks; equal weight rows plant exact ties, so
