@@ -278,8 +278,9 @@ static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch, 
   // rows: 4096 x 1024 5.7 / 5.4 / 6.0 / 6.9 and 4.9 / 5.1 / 6.3 / 7.1; gate/up
   // 3072 x 1024 6.0 / 6.6 / 7.5 / 8.3 and 5.9 / 6.9 / 8.0 / 8.8, but 2048 x
   // 1024, one unit per workgroup, 5.7 / 6.3 / 7.2 / 8.2 and 4.9 / 5.8 / 6.3 /
-  // 7.2).
-  const bool brief = !arg && p->ksw <= 8 && (glu ? a->rows > 16 && a->n > 8 * kWideWorkgroups : a->rows > 32);
+  // 7.2; lm_head 151936 x 1024 at 24 rows, two tiles per wave, 70.7 and 86.3).
+  const bool brief = p->ksw <= 8 &&
+                     (arg ? tw == 2 : glu ? a->rows > 16 && a->n > 8 * kWideWorkgroups : a->rows > 32);
   const bool many = a->rows >= kWideMinRows && a->waves == 4 && (arg || a->tiles_per_wg == 1) &&
                     (a->ksplit == 1 || a->parts_out) && !a->next_norm_w && wide_offsets(a) && (wide || !brief);
   if (wide) {

@@ -327,6 +327,31 @@ def step_plan(n, k, role, batch, split_o=True):
     return 1, waves, tiles
 
 
+def lm_tiles(rows, vocab, hidden, waves, merges):
+    """lm_head output tiles per workgroup from 2 rows (the grouping changes no
+    sum): LM_TILES_BATCHED up to 8 rows.  From 9 the many-row kernel, which
+    takes four waves, groups them itself (1 here) except at 17..32 rows of a
+    k range of at most 8 steps per wave, where the per-tile kernel of two
+    tiles per wave is faster (Qwen3-0.6B, 151936 x 1024: 70.7 / 86.3 us).
+    Other widths stay on the per-tile kernels: 8 tiles where they run two
+    per wave, or where all rows fit LDS and the call does not merge a split
+    update (``merges``), as long as that leaves a workgroup per CU; else 1.
+    us with 8 tiles / 1: 151936 x 320 at 9 rows 54 / 182, 24 rows 40 / 182;
+    151936 x 1344 at 16 rows 116 / 192, 24 rows 422 / 195; 4096 x 2560 at 9
+    rows 36 / 16."""
+    if (vocab // 16) % LM_TILES_BATCHED:
+        return 1
+    if rows <= 8:
+        return LM_TILES_BATCHED
+    ksw = hidden // 32 // waves
+    pairs = WIDE_MIN_ROWS <= rows <= 32 and (ksw % 5 == 0 or ksw % 8 == 0)
+    if waves == 4:
+        return LM_TILES_BATCHED if pairs and ksw <= 8 else 1
+    if vocab < 16 * LM_TILES_BATCHED * 256:
+        return 1
+    return LM_TILES_BATCHED if pairs or (rows <= 32 and rows * hidden <= 24 << 10 and not merges) else 1
+
+
 # From this batch the attention runs 8 waves per workgroup with the
 # residency chunking of attn_chunk.  Same-box A/B, ms per step at 1024-token
 # prompts, 8 waves / 4 waves: batch 8 2.964 / 3.017, batch 6 2.891 / 2.953;
@@ -744,12 +769,7 @@ class DecodeState:
             a.w = m.lm_w.data_ptr()
             a.norm_w = m.norm_w.data_ptr()
             a.n, a.k, a.flags = c.vocab, c.hidden, capi.NORM_IN | capi.ARGMAX
-            # 8 tiles per workgroup from 2 rows; from 9 the many-row kernel
-            # groups them itself (the grouping changes no sum).
-            if rows == 1:
-                a.tiles_per_wg = tiles
-            elif rows <= 8 and (c.vocab // 16) % LM_TILES_BATCHED == 0:
-                a.tiles_per_wg = LM_TILES_BATCHED
+            a.tiles_per_wg = tiles if rows == 1 else lm_tiles(rows, a.n, a.k, waves, bool(a.x_parts))
             a.out = self.logits.data_ptr() if self.logits is not None else None
             a.ids_out = (ids_out if ids_out is not None else self.ids).data_ptr()
             a.lens_inc = lens_inc.data_ptr() if lens_inc is not None else None

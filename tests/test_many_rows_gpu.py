@@ -60,7 +60,7 @@ class Call:
         self.norm_w = rnd(k, scale=0.2, seed=seed + 1)
         self.scratch = torch.zeros(4 << 20, dtype=torch.float32, device=DEV)
         self.counters = torch.zeros(8192, dtype=torch.int32, device=DEV)
-        self.waves, self.row_major = 4, False
+        self.waves, self.row_major, self.tiles = 4, False, 1
 
     def __call__(self, x, res, wide):
         c, rows, n = self.capi, x.shape[0], self.n
@@ -68,7 +68,7 @@ class Call:
         flags = {"norm": c.NORM_IN, "glu": c.NORM_IN | c.GLU, "plain": 0, "res": c.RES_OUT, "parts": c.RES_OUT,
                  "argmax": c.NORM_IN | c.ARGMAX}[self.kind]
         a.w, a.eps, a.rows, a.n, a.k, a.flags = self.w.data_ptr(), 1e-6, rows, n, self.k, flags
-        a.ksplit, a.waves, a.tiles_per_wg = self.ksplit, self.waves, 1
+        a.ksplit, a.waves, a.tiles_per_wg = self.ksplit, self.waves, self.tiles
         a.partial, a.counters = self.scratch.data_ptr(), self.counters.data_ptr()
         if flags & c.NORM_IN:
             a.x, a.norm_w = x.data_ptr(), self.norm_w.data_ptr()
@@ -140,22 +140,51 @@ def test_units_per_workgroup_bitexact(lib, kind, n, k, ksplit, rows):
     test_many_rows_bitexact(lib, kind, n, k, ksplit, rows)
 
 
-@pytest.mark.parametrize("rows,n", [(9, 16), (16, 4112), (33, 784), (64, 16896)])
-def test_many_rows_argmax(lib, rows, n):
-    """The lm_head's logits and picks; equal weight rows plant exact ties, so
-    the lowest of equal indices has to win across units and workgroups."""
-    call = Call(lib, "argmax", n, 256, 1, seed=n)
-    w = rnd(n, 256, scale=0.05, seed=n)
+@pytest.mark.parametrize("rows,n,k", [(9, 16, 256), (16, 4112, 256), (33, 784, 256), (64, 16896, 256),
+                                      (9, 16896, 4096), (16, 16896, 2560), (17, 16896, 2560), (24, 16896, 1024),
+                                      (32, 784, 4096), (33, 16896, 2048), (48, 4112, 1152), (64, 16896, 2560)])
+def test_many_rows_argmax(lib, rows, n, k):
+    """The lm_head's logits and picks, grouped as the runtime groups them (two
+    tiles per wave at 24 rows of k = 1024), over k ranges shorter and longer
+    than the load rings; equal weight rows plant exact ties, so the lowest of
+    equal indices has to win across units and workgroups."""
+    from qdec.runtime import lm_tiles
+    call = Call(lib, "argmax", n, k, 1, seed=n)
+    w = rnd(n, k, scale=0.05, seed=n)
     w[n // 2] = w[3] = w[n - 1] = 4 * w[3]
     call.w = pack(lib, w)
-    x, res = rnd(rows, 256, scale=2.0, seed=rows), rnd(rows, n, seed=1)
-    logits, ids = call(x, res, False)
+    x, res = rnd(rows, k, scale=2.0, seed=rows), rnd(rows, n, seed=1)
     want = [call(x[i:i + 8].contiguous(), res[i:i + 8], False) for i in range(0, rows, 8)]
+    call.tiles = lm_tiles(rows, n, k, 4, False)
+    assert call.tiles == (8 if (rows, k) == (24, 1024) else 1)
+    logits, ids = call(x, res, False)
     assert torch.equal(logits, torch.cat([o[0] for o in want]))
     assert torch.equal(ids, torch.cat([o[1] for o in want]))
     top = logits.float().amax(1, keepdim=True)
     first = torch.where(logits.float() == top, torch.arange(n, device=DEV), n).amin(1)
     assert torch.equal(ids, first)
+
+
+@pytest.mark.parametrize("rows", [9, 40])
+def test_many_rows_argmax_of_infinite_logits(lib, rows):
+    """Logits of -inf, +inf and NaN: a row without a logit above -inf picks
+    QDEC_NAN_ID and one of +inf its first, as the calls of up to 8 rows."""
+    from qdec import capi
+    n, k = 784, 1024
+    call = Call(lib, "argmax", n, k, 1, seed=n)
+    w = rnd(n, k, scale=0.05, seed=n)
+    w[:, 0] = float("-inf")
+    call.w, call.norm_w[0] = pack(lib, w), 1
+    x, res = rnd(rows, k, scale=2.0, seed=rows), rnd(rows, n, seed=1)
+    x[:, 0] = torch.tensor([1.0, -1.0, 0.0], device=DEV).repeat(rows)[:rows]
+    x[5] = float("nan")
+    logits, ids = call(x, res, False)
+    want = [call(x[i:i + 8].contiguous(), res[i:i + 8], False) for i in range(0, rows, 8)]
+    assert torch.equal(logits.isnan(), torch.cat([o[0] for o in want]).isnan())
+    assert torch.equal(ids, torch.cat([o[1] for o in want]))
+    kinds = [capi.NAN_ID if i % 3 != 1 or i == 5 else 0 for i in range(rows)]
+    assert ids.tolist() == kinds
+    assert (logits[0] == float("-inf")).all() and (logits[1] == float("inf")).all() and logits[2].isnan().all()
 
 
 @pytest.mark.parametrize("kind,n,k,waves", [("norm", 4096, 2048, 8), ("norm", 304, 1024, 4), ("glu", 6144, 2048, 4),

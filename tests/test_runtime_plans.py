@@ -39,3 +39,32 @@ def test_lm_head_grouping_divides_the_vocab():
     vocab, hidden = qwen3_config()["vocab_size"], qwen3_config()["hidden_size"]
     assert (vocab // 16) % LM_TILES_BATCHED == 0
     assert (vocab // 16) % role_plan(vocab, hidden, "lm")[2] == 0
+
+
+@pytest.mark.parametrize("hidden,vocab", [(1024, 151936), (2560, 151936), (640, 151936), (320, 151936), (1344, 151936),
+                                          (2080, 151936), (2560, 4096), (320, 1024), (2560, 16896 + 16)])
+def test_lm_head_grouping_is_accepted(hidden, vocab):
+    """Every lm_head call of a state plans, with and without a split update to
+    merge, and from 9 rows takes the grouping measured faster."""
+    from qdec import capi
+    from qdec.runtime import LM_TILES_BATCHED, lm_tiles, role_plan
+    lib = capi.lib()
+    waves = role_plan(vocab, hidden, "lm")[1]
+    got = {}
+    for rows in range(2, 65):
+        for merges in (False, True):
+            t = got[rows, merges] = lm_tiles(rows, vocab, hidden, waves, merges)
+            a = capi.GemmArgs(x=16, w=16, norm_w=16, ids_out=16, eps=1e-6, rows=rows, n=vocab, k=hidden, ksplit=1, waves=waves,
+                              flags=capi.NORM_IN | capi.ARGMAX, tiles_per_wg=t)
+            if merges:
+                if rows < 9:  # states of 9 or more sequences split the down projection
+                    continue
+                a.x_parts, a.x_nparts, a.x_merged = 16, 4, 32
+            lib.gemm_workspace(a)
+    small = vocab < 151936
+    for rows, want in ((8, 8), (9, 8 if hidden in (320, 1344, 2080) and not small else 1),
+                       (24, 8 if hidden in (320, 640, 1024, 2080) and not small else 1), (33, 1), (64, 1)):
+        if (vocab // 16) % LM_TILES_BATCHED == 0:
+            assert got[rows, False] == want, rows
+        else:
+            assert got[rows, False] == 1
