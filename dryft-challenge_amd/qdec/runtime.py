@@ -363,13 +363,16 @@ def lm_tiles(rows, vocab, hidden, waves, merges):
 # is mixed (1024 tokens 2.195 / 2.228, 2048 2.404 / 2.283: ten chunks to
 # merge), and batch 1 (2.089 / 2.077) stays on 4.
 ATTN8_MIN_BATCH = 3
-# Above this batch (8 kv heads: more than one workgroup per CU) a state of at
-# least ATTN4_MIN_CAP slots runs 4 waves again: two workgroups share a CU, and
-# one's prologue and merge run beside the other's stream instead of in a round
-# of their own (four layers, us, 8 / 4 waves: 33 sequences at 1000 tokens 500
-# / 486, 48 at 500 452 / 438, 64 at 500 477 / 471, 64 at 1500 643 / 632; 32 at
-# 4096 652 / 658).  No speculation runs there, so the count may depend on the
-# capacity.
+# Above this batch (no speculation runs there, so the count may depend on the
+# capacity) a state of at least ATTN4_MIN_CAP slots whose batch x kv heads are
+# more than one workgroup per CU runs 4 waves again: two workgroups share a CU,
+# and one's prologue and merge run beside the other's stream instead of in a
+# round of their own (four layers of 8 kv heads, us, 8 / 4 waves: 33 sequences
+# at 1000 tokens 500 / 486, 48 at 500 452 / 438, 64 at 500 477 / 471, 64 at
+# 1500 643 / 632; 32 at 4096 652 / 658).  With fewer kv heads one round holds
+# them all and 8 waves stay ahead (attention alone, 4 kv heads: 33 sequences
+# at 1000 tokens 21.3 / 22.7, 64 at 500 16.3 / 17.1, 64 at 1000 25.5 / 26.9; 2
+# kv heads: 64 at 500 13.9 / 15.0; 8 kv heads 64 at 1000 48.3 / 44.3).
 ATTN8_MAX_BATCH = 32
 ATTN4_MIN_CAP = 512
 # Rows per sequence an 8-wave attention workgroup takes (two M tiles of
@@ -396,6 +399,15 @@ def attn_waves(batch):
     batch alone: plain and speculative states of one batch agree.  8 waves
     take at most ATTN8_MAX_T rows per sequence (max_rows_per_seq)."""
     return 8 if batch >= ATTN8_MIN_BATCH else 4
+
+
+def state_attn_waves(batch, nkv, head_dim, cap):
+    """attn_waves of a state's shape: 4 again where more workgroups than CUs
+    would queue (ATTN8_MAX_BATCH), and at head_dim 64 (the tiny test
+    configurations: four 16-channel output tiles, one per wave)."""
+    if head_dim != 128 or (batch > ATTN8_MAX_BATCH and batch * nkv > 256 and cap >= ATTN4_MIN_CAP):
+        return 4
+    return attn_waves(batch)
 
 
 def max_rows_per_seq(batch, requested=ATTN_MAX_T, group=4):
@@ -559,11 +571,7 @@ class DecodeState:
         dev, bf = model.device, torch.bfloat16
         L, H, D = c.n_layers, c.hidden, c.head_dim
         self.chunk = attn_chunk(batch, c.nkv, self.cap)
-        # head_dim 64 (the tiny test configurations): four 16-channel output
-        # tiles, one per wave of a 4-wave workgroup
-        self.attn_waves = attn_waves(batch) if c.head_dim == 128 else 4
-        if batch > ATTN8_MAX_BATCH and self.cap >= ATTN4_MIN_CAP:
-            self.attn_waves = 4
+        self.attn_waves = state_attn_waves(batch, c.nkv, D, self.cap)
         assert self.attn_waves == 4 or self.max_t <= 8
         cache_shape = (L, batch, c.nkv, self.cap, D)
         self.k_cache = torch.zeros(cache_shape, dtype=bf, device=dev)

@@ -33,6 +33,17 @@ def test_attention_waves_fit_every_state_of_a_batch(batch, group):
     assert batch * (k + 1) <= 16 or k == 0
 
 
+@pytest.mark.parametrize("batch,nkv,head_dim,cap,waves", [
+    (1, 8, 128, 1024, 4), (8, 8, 128, 1024, 8), (32, 8, 128, 4384, 8), (33, 8, 128, 1024, 4), (64, 8, 128, 512, 4),
+    (64, 8, 128, 480, 8), (33, 4, 128, 1024, 8), (64, 4, 128, 2080, 8), (64, 2, 128, 1024, 8), (48, 16, 128, 1024, 4),
+    (8, 2, 64, 128, 4), (64, 8, 64, 1024, 4)])
+def test_state_attention_waves(batch, nkv, head_dim, cap, waves):
+    """4 waves above batch 32 only where batch x kv heads are more workgroups
+    than CUs."""
+    from qdec.runtime import state_attn_waves
+    assert state_attn_waves(batch, nkv, head_dim, cap) == waves
+
+
 def test_lm_head_grouping_divides_the_vocab():
     from qdec.checkpoint import qwen3_config
     from qdec.runtime import LM_TILES_BATCHED, role_plan
