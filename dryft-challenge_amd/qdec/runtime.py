@@ -96,30 +96,22 @@ FRAG_ROWS = 9
 HAND_OVER = False
 # Loss-free speculation needs identical arithmetic in the plain and verify
 # steps, so attention chunking depends on (batch, capacity) only.
-# k splits of the down projection from this batch size (see role_plan).
-DOWN_SPLIT = 4
-DOWN_SPLIT_MIN_BATCH = 16
-# From this batch the O projection runs 4 waves per workgroup instead of 8
-# (see role_plan).
-O_FOUR_WAVES_MIN_BATCH = 9
-# k splits of the O projection at O_SPLIT_MIN_BATCH..O_SPLIT_MAX_BATCH (see
-# role_plan): the partials go to the gate/up call's normalisation pre-pass.
-O_SPLIT = 2
-O_SPLIT_MIN_BATCH = 17
-O_SPLIT_MAX_BATCH = 32
 # From MANY_ROWS_MIN_BATCH sequences (no speculation there) a step's plans are
-# those of qdec_gemm's many-row kernel (step_plan): O and down split k and
+# those of qdec_gemm's many-row kernel (role_plan): O and down split k and
 # leave fp32 partials to the next NORM_IN call's pre-pass at every batch,
 # since their 160 output tiles alone leave a third of the CUs idle.  Same-box
 # A/B, us per launch unsplit / split: down at 13 rows 18.7 / 11.4, O 8.8 /
-# 7.4; four layers (1024-token prompts), per-tile kernels and role_plan
-# against the many-row kernel and step_plan: batch 9 381 / 329 us, 13 390 /
-# 338, 33 592 / 507, 64 684 / 573.  At batch 8 and below the merge costs as
-# much as the split gains (batch 8 3.01 -> 3.09 ms per step, batch 1 2.145 ->
-# 2.155).
+# 7.4; four layers (1024-token prompts), per-tile kernels with splits from
+# batch 16 (down) and at 17..32 (O) / these plans: batch 9 381 / 329 us, 13
+# 390 / 338, 33 592 / 507, 64 684 / 573.  At batch 8 and below the merge costs
+# as much as the split gains (batch 8 3.01 -> 3.09 ms per step, batch 1 2.145
+# -> 2.155).
 MANY_ROWS_MIN_BATCH = 9
+O_SPLIT = 2
+DOWN_SPLIT = 4
 # Output tiles per workgroup of qdec_gemm's two-tiles-per-wave plan (17..32
-# rows); the runtime's own calls take the many-row kernel there.
+# rows); of the runtime's calls only those whose k / 128 is not whole take it,
+# the others the many-row kernel.
 WIDE_TILES = 2
 WIDE_MIN_ROWS = 17
 # gate/up at RESIDENT_ROWS rows runs with its rows resident in LDS
@@ -249,57 +241,29 @@ def rope_tables(cap, head_dim, theta):
     return emb.cos().to(torch.bfloat16), emb.sin().to(torch.bfloat16)
 
 
-def role_plan(n, k, role, batch=1):
-    """(ksplit, waves, tiles_per_wg) of one projection role at a batch size.
+def role_plan(n, k, role, batch=1, split_o=True):
+    """(ksplit, waves, tiles_per_wg) of one projection role in a state of
+    ``batch`` sequences.
 
     Output tiles are 16 columns, one workgroup per tile (4 per workgroup for
-    the lm_head), no k split across workgroups: a split's cross-workgroup
-    reduction cost more than it won back on MI355X.  The roles with few
-    tiles (N = hidden: O and down, 160 tiles for 256 CUs) run 8 waves per
-    workgroup, which doubles the weight blocks each busy CU keeps in flight
-    (O 7.6 -> 7.0 us, down 14.2 -> 13.5 us at batch 1); O goes back to 4
-    from O_FOUR_WAVES_MIN_BATCH.  The lm_head runs 4
-    tiles per workgroup (137 us against 144 us with 8 and 146 us with 2,
-    non-temporal weight loads).  Only (n, k, role) and the batch decide it,
-    never the row count, so a verify pass over batch x (k + 1) rows sums
-    every element as the plain step of the same batch does."""
-    ks = k // 32
-    ntiles = n // 16
-    ksplit = 1
+    the lm_head), no k split across workgroups below MANY_ROWS_MIN_BATCH: a
+    split's cross-workgroup reduction cost more than it won back on MI355X.
+    The roles with few tiles (N = hidden: O and down, 160 tiles for 256 CUs)
+    run 8 waves per workgroup, which doubles the weight blocks each busy CU
+    keeps in flight (O 7.6 -> 7.0 us, down 14.2 -> 13.5 us at batch 1; O at 8
+    rows 7.21, with 4 waves 7.78).  The lm_head runs 4 tiles per workgroup
+    (137 us against 144 us with 8 and 146 us with 2, non-temporal weight
+    loads).  From MANY_ROWS_MIN_BATCH QKV, O and down run 4 waves, as the
+    many-row kernel and the resident plans want, O (``split_o``) in O_SPLIT
+    and down in DOWN_SPLIT k parts where the width allows and the output has
+    at most 256 tiles.  Only (n, k, role) and the batch decide it, never the
+    row count, so a verify pass over batch x (k + 1) rows sums every element
+    as the plain step of the same batch does."""
+    ks, ntiles = k // 32, n // 16
+    if batch >= MANY_ROWS_MIN_BATCH and role in ("qkv", "o", "down") and ks % 4 == 0:
+        split = {"qkv": 1, "o": O_SPLIT if split_o else 1, "down": DOWN_SPLIT}[role]
+        return (split if ks % (4 * split) == 0 and ntiles <= 256 else 1), 4, 1
     waves = 8 if ntiles <= 256 else 4
-    if (role == "down" and batch >= DOWN_SPLIT_MIN_BATCH and DOWN_SPLIT > 1 and ntiles <= 256
-            and ks % (DOWN_SPLIT * 4) == 0):
-        # Few tiles and a long k: split k in DOWN_SPLIT, four waves each, and
-        # leave the partials to the next NORM_IN call (x_parts), whose
-        # normalisation pre-pass merges them (Qwen3-4B: 640 workgroups instead
-        # of 160).  Measured on MI355X, ms per step: batch 32 3.69 -> 3.62;
-        # batch 8 3.01 -> 3.09 and batch 1 2.145 -> 2.155 (QKV then needs the
-        # pre-pass, or merges four partials per workgroup), so only from
-        # DOWN_SPLIT_MIN_BATCH.
-        return DOWN_SPLIT, 4, 1
-    if (role == "o" and O_SPLIT_MIN_BATCH <= batch <= O_SPLIT_MAX_BATCH and O_SPLIT > 1 and ntiles <= 256
-            and ks % (O_SPLIT * 4) == 0):
-        # Split k in O_SPLIT, four waves each, and leave the partials to the
-        # gate/up call's normalisation pre-pass, like the down projection's
-        # to the next QKV's: each part's rows then fit the LDS of the resident
-        # split plan (qdec_gemm resident; 128 KiB per part at 32 rows).
-        # Same-box A/B at batch 32 and 4096-token prompts: O 10.5 -> 7.6 us
-        # per launch.
-        return O_SPLIT, 4, 1
-    if role == "qkv" and batch >= WIDE_MIN_ROWS and not any(lo <= batch <= hi for lo, hi in RESIDENT_QKV_ROWS[1:]):
-        # two tiles per wave (WIDE_TILES): 192 workgroups, 8 waves each; the
-        # resident plan (RESIDENT_QKV_ROWS) splits k over 4 waves
-        waves = 8
-    if role == "o" and batch >= O_FOUR_WAVES_MIN_BATCH:
-        # From 9 rows O takes the direct path (fragments loaded beside each
-        # weight block), where 4 waves of 32 k steps beat 8 of 16.  Same-box
-        # A/B, ms per step at 1024-token prompts (8 waves / 4), measured on
-        # the direct path: batch 8 2.969 / 2.943, 10 3.091 / 3.073, 12 3.143 /
-        # 3.123, 16 3.126 / 3.096, 32 3.609 / 3.610; with the rows staged in
-        # LDS 4 waves lose: batch 7 2.993 / 3.073, 5 2.710 / 2.802, 3 2.404 /
-        # 2.449, and, since 8 rows copy their rows into LDS too (the resident
-        # plan), batch 8: O 7.21 / 7.78 us per launch, 2.448 / 2.467 ms.
-        waves = 4
     while ks % waves:
         waves //= 2
     tiles = 1
@@ -308,22 +272,6 @@ def role_plan(n, k, role, batch=1):
             if ntiles % cand == 0:
                 tiles = cand
                 break
-    return ksplit, waves, tiles
-
-
-def step_plan(n, k, role, batch, split_o=True):
-    """(ksplit, waves, tiles_per_wg) of ``role`` in a state of ``batch``
-    sequences: role_plan's, and from MANY_ROWS_MIN_BATCH that of the many-row
-    kernel -- 4 waves, O (``split_o``) and down in O_SPLIT and DOWN_SPLIT k
-    splits where their widths allow."""
-    ksplit, waves, tiles = role_plan(n, k, role, batch)
-    if batch < MANY_ROWS_MIN_BATCH or role not in ("qkv", "o", "down"):
-        return ksplit, waves, tiles
-    ks = k // 32
-    want = {"qkv": 1, "o": O_SPLIT if split_o else 1, "down": DOWN_SPLIT}[role]
-    for split in (want, 1):
-        if ks % (split * 4) == 0 and (split == 1 or n // 16 <= 256):
-            return split, 4, tiles
     return 1, waves, tiles
 
 
@@ -586,12 +534,12 @@ class DecodeState:
         self.hbuf = torch.zeros((2, R, H), dtype=bf, device=dev)
         self.h = self.hbuf[0]
         self.plans = dict(model.plans)
-        self.plans["down"] = step_plan(H, c.inter, "down", batch)
-        self.plans["qkv"] = step_plan(c.n_qkv, H, "qkv", batch)
+        self.plans["down"] = role_plan(H, c.inter, "down", batch)
+        self.plans["qkv"] = role_plan(c.n_qkv, H, "qkv", batch)
         ks, _, _ = self.plans["down"]
         # O splits only where down does: the residual then always moves by
         # merges (_residual_in).
-        self.plans["o"] = step_plan(H, c.nq * c.head_dim, "o", batch, split_o=ks > 1)
+        self.plans["o"] = role_plan(H, c.nq * c.head_dim, "o", batch, split_o=ks > 1)
         self.down_parts = torch.zeros((ks, R, H), dtype=torch.float32, device=dev) if ks > 1 else None
         # A split O projection leaves its update as partials too (o_parts);
         # the gate/up call's pre-pass merges them into hpost, the residual
@@ -1041,7 +989,7 @@ class Prefill:
     def _skinny_layers(self, R):
         """Every layer's four products over all R prompt rows (row b*S + t)
         as qdec_gemm_wide calls, and the buffer that holds the residual after
-        the last one.  O and down split k as step_plan splits them and leave
+        the last one.  O and down split k as role_plan splits them and leave
         their partials to the next NORM_IN call's pre-pass, which merges them
         into the other of two residual buffers; the last layer's down, which
         no call follows, leaves its parts to the merge that ``run`` adds.
@@ -1050,7 +998,7 @@ class Prefill:
             return self._skinny_calls[R]
         st, m, c = self.state, self.state.model, self.state.model.cfg
         dev, H, nqd = m.device, c.hidden, c.nq * c.head_dim
-        split = {role: step_plan(H, k, role, MANY_ROWS_MIN_BATCH)[0] for role, k in (("o", nqd), ("down", c.inter))}
+        split = {role: role_plan(H, k, role, MANY_ROWS_MIN_BATCH)[0] for role, k in (("o", nqd), ("down", c.inter))}
         rows = max(GEMM_WIDE_MIN_ROWS, min(self.state.batch * self.chunk, PREFILL_WIDE_ROWS))  # the most this path runs
         if self._skinny_bufs is None:
             xn = -(-rows // 16) * 16 * H  # the pre-pass's rows (qdec_gemm_wide_workspace)

@@ -371,15 +371,21 @@ def test_role_plans_do_not_depend_on_rows():
         ks, w, t = role_plan(n, k, role)
         assert (k // 32) % (ks * w) == 0
         assert (n // 16) % t == 0
-    # from batch 16 down splits k four ways (partials merged by the next
-    # NORM_IN call's pre-pass); O always runs whole tiles
-    assert role_plan(2560, 9728, "down") == (1, 8, 1) and role_plan(2560, 4096, "o")[0] == 1
-    assert role_plan(2560, 9728, "down", batch=16)[:2] == (4, 4)
-    assert role_plan(2560, 9728, "down", batch=8) == (1, 8, 1)
-    assert role_plan(2560, 4096, "o", batch=8) == (1, 8, 1) and role_plan(2560, 4096, "o", batch=9) == (1, 4, 1)
-    # QKV from 17 rows: k over 4 waves on the resident plan, else 8 waves of two tiles
-    assert role_plan(6144, 2560, "qkv", batch=17)[:2] == (1, 4) and role_plan(6144, 2560, "qkv", batch=16)[:2] == (1, 4)
-    assert role_plan(6144, 2560, "qkv", batch=33)[:2] == (1, 8)
+    # from batch 9 O and down split k two and four ways (partials merged by the
+    # next NORM_IN call's pre-pass) and every role runs 4 waves; below, whole
+    # tiles on 8 waves
+    for batch in (1, 8):
+        assert role_plan(2560, 9728, "down", batch) == (1, 8, 1) and role_plan(2560, 4096, "o", batch) == (1, 8, 1)
+        assert role_plan(6144, 2560, "qkv", batch) == (1, 4, 1)
+    for batch in (9, 13, 16, 17, 32, 33, 64):
+        assert role_plan(2560, 9728, "down", batch) == (4, 4, 1) and role_plan(2560, 4096, "o", batch) == (2, 4, 1)
+        assert role_plan(6144, 2560, "qkv", batch) == (1, 4, 1) and role_plan(4096, 2560, "qkv", batch) == (1, 4, 1)
+        assert role_plan(2560, 4096, "o", batch, split_o=False) == (1, 4, 1)
+        # more than 256 output tiles (hidden 5120) fill the CUs unsplit
+        assert role_plan(5120, 25600, "down", batch) == (1, 4, 1) and role_plan(5120, 8192, "o", batch) == (1, 4, 1)
+        # k / 32 a multiple of 4 but not of 4 x the split; not of 4
+        assert role_plan(1024, 128 * 9, "down", batch) == (1, 4, 1) and role_plan(1024, 128 * 9, "o", batch) == (1, 4, 1)
+        assert role_plan(1024, 64 * 11, "down", batch) == (1, 2, 1) and role_plan(1024, 32 * 11, "o", batch) == (1, 1, 1)
     # the 160-tile roles run 8 waves, the others 4; the lm_head 4 tiles per workgroup
     assert [role_plan(n, k, r)[1] for r, n, k in (("qkv", 6144, 2560), ("o", 2560, 4096),
                                                   ("gate_up", 9728, 2560), ("down", 2560, 9728),

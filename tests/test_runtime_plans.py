@@ -79,3 +79,16 @@ def test_lm_head_grouping_is_accepted(hidden, vocab):
             assert got[rows, False] == want, rows
         else:
             assert got[rows, False] == 1
+
+
+@pytest.mark.parametrize("n,k", [(2560, 4096), (2560, 9728), (2048, 6144), (1024, 3072), (1024, 2048), (4096, 12288),
+                                 (5120, 25600), (320, 704), (1152, 1152)])
+def test_prefill_split_fills_one_round(n, k):
+    """k parts of a short prompt's O and down: whole 64-element stages in each
+    part, and no more tiles than one round of the CUs."""
+    from qdec.runtime import prefill_split, round_up
+    for rows in range(129, 2049):
+        parts, tiles = prefill_split(rows, n, k), round_up(rows, 256) // 256 * (n // 128)
+        assert 1 <= parts <= 8 and (parts == 1 or (n % 128 == 0 and k % (64 * parts) == 0 and parts * tiles <= 256))
+        if n % 128 == 0 and parts < 8 and k % (128 * parts) == 0:
+            assert 2 * parts * tiles > 256  # the most that fit
