@@ -932,11 +932,11 @@ def test_down_split_merged_by_next_norm_in_call(lib, rows):
 def test_two_tiles_per_wave_bitexact(lib, role, rows):
     """At two M tiles a workgroup with an even number of output tiles runs two
     per wave (each activation fragment feeds both; gate/up keeps one per wave
-    and runs its two in turn): every output bit, the split partials and the
-    argmax equal the one-tile-per-workgroup call's, for each role in the
-    engine's layouts and batch-32 plans (fragment-order activations into O
-    and down, SwiGLU written in fragment order, the normalisation pre-pass of
-    QKV, the 8-tile lm_head)."""
+    and runs its two in turn): every output bit and the split partials equal
+    the one-tile-per-workgroup call's, for each role in the layouts of a
+    batch-32 step (fragment-order activations into O and down, SwiGLU written
+    in fragment order, the normalisation pre-pass of QKV).  The lm_head, which
+    runs the many-row kernel at either grouping, equals the calls of 8 rows."""
     from qdec import capi
     from qdec.runtime import LM_TILES_BATCHED, WIDE_TILES, role_plan
     assert WIDE_TILES == 2
@@ -956,8 +956,10 @@ def test_two_tiles_per_wave_bitexact(lib, role, rows):
     res0 = rnd(rows, n, scale=2.0, seed=seed + 3).to(DEV)
     ws = Gemm(lib, flags, n, k)
 
-    def run(tiles):
-        a = capi.GemmArgs(x=x.data_ptr(), w=W.data_ptr(), eps=1e-6, rows=rows, n=n, k=k, flags=flags, ksplit=ks,
+    def run(tiles, lo=0, hi=rows):
+        rows = hi - lo
+        xs = x[lo:].contiguous() if lo else x
+        a = capi.GemmArgs(x=xs.data_ptr(), w=W.data_ptr(), eps=1e-6, rows=rows, n=n, k=k, flags=flags, ksplit=ks,
                           waves=waves, tiles_per_wg=tiles, partial=ws.partial.data_ptr(),
                           counters=ws.counters.data_ptr())
         outs = []
@@ -989,7 +991,11 @@ def test_two_tiles_per_wave_bitexact(lib, role, rows):
         return [t.cpu() for t in outs]
 
     wide = LM_TILES_BATCHED if role == "lm" else WIDE_TILES
-    one, two = run(1), run(wide)
+    if role == "lm":
+        calls = [run(wide, i, min(i + 8, rows)) for i in range(0, rows, 8)]
+        one, two = [torch.cat(ts) for ts in zip(*calls)], run(wide)
+    else:
+        one, two = run(1), run(wide)
     for t1, t2 in zip(one, two):
         if t1.dtype == torch.bfloat16:
             t1, t2 = t1.view(torch.int16), t2.view(torch.int16)

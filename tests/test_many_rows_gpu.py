@@ -60,7 +60,7 @@ class Call:
         self.norm_w = rnd(k, scale=0.2, seed=seed + 1)
         self.scratch = torch.zeros(4 << 20, dtype=torch.float32, device=DEV)
         self.counters = torch.zeros(8192, dtype=torch.int32, device=DEV)
-        self.waves, self.row_major, self.tiles = 4, False, 1
+        self.waves, self.row_major, self.tiles, self.x_parts = 4, False, 1, None
 
     def __call__(self, x, res, wide):
         c, rows, n = self.capi, x.shape[0], self.n
@@ -72,6 +72,9 @@ class Call:
         a.partial, a.counters = self.scratch.data_ptr(), self.counters.data_ptr()
         if flags & c.NORM_IN:
             a.x, a.norm_w = x.data_ptr(), self.norm_w.data_ptr()
+            if self.x_parts is not None:
+                self.merged = torch.full_like(x, float("nan"))
+                a.x_parts, a.x_nparts, a.x_merged = (self.x_parts.data_ptr(), len(self.x_parts), self.merged.data_ptr())
         elif self.row_major:
             a.x = x.data_ptr()
         else:
@@ -188,7 +191,8 @@ def test_many_rows_argmax_of_infinite_logits(lib, rows):
 
 
 @pytest.mark.parametrize("kind,n,k,waves", [("norm", 4096, 2048, 8), ("norm", 304, 1024, 4), ("glu", 6144, 2048, 4),
-                                            ("glu", 48, 1024, 4), ("res", 304, 2048, 8)])
+                                            ("glu", 48, 1024, 4), ("res", 304, 2048, 8), ("plain", 304, 1024, 4),
+                                            ("argmax", 304, 1024, 4), ("argmax", 4112, 2048, 8)])
 def test_short_ring_bitexact(lib, kind, n, k, waves):
     """Widths whose k range per wave is a multiple of 8 but not of the longer
     load rings (rows staged in LDS, a ring of 8): 1, 3, 5 and 8 rows give the
@@ -196,12 +200,34 @@ def test_short_ring_bitexact(lib, kind, n, k, waves):
     call = Call(lib, kind, n, k, 1, seed=n + k)
     call.waves = waves
     x, res = rnd(12, k, scale=2.0, seed=5), rnd(12, n, seed=6)
-    want = call(x, res, False)[0]
+    want = call(x, res, False)
+    call.row_major = True
     for rows in ([3], [0, 1, 2], [7, 8, 9, 10, 11], list(range(8))):
-        call.row_major = True
-        got = call(x[rows].contiguous(), res[rows].contiguous(), False)[0]
-        call.row_major = False
-        assert torch.equal(got.contiguous().view(torch.int16), want[rows].view(torch.int16)), rows
+        got = call(x[rows].contiguous(), res[rows].contiguous(), False)
+        assert torch.equal(got[0].contiguous().view(torch.int16), want[0][rows].view(torch.int16)), rows
+        assert all(torch.equal(g, w[rows]) for g, w in zip(got[1:], want[1:]))  # the picks
+
+
+@pytest.mark.parametrize("kind,n", [("norm", 304), ("argmax", 4112)])
+@pytest.mark.parametrize("rows,nparts", [(1, 2), (1, 4), (1, 5), (3, 2)])
+def test_short_ring_merges_split_update(lib, kind, n, rows, nparts):
+    """A pending split update merged by a call on the ring of 8: in its
+    prologue at one row and up to four parts, else by the pre-pass.  The
+    merged row is bf16(x + bf16(p0 + p1 + ...)), the output that of the same
+    call on it."""
+    k = 1024
+    call = Call(lib, kind, n, k, 1, seed=n)
+    x, res = rnd(rows, k, scale=2.0, seed=5), rnd(rows, n, seed=6)
+    parts = torch.randn(nparts, rows, k, generator=torch.Generator().manual_seed(7)).to(DEV)
+    upd = parts[0]
+    for p in parts[1:]:
+        upd = upd + p
+    merged = (x.float() + upd.to(torch.bfloat16).float()).to(torch.bfloat16)
+    want = call(merged, res, False)
+    call.x_parts = parts
+    got = call(x, res, False)
+    assert torch.equal(call.merged.view(torch.int16), merged.view(torch.int16))
+    assert all(torch.equal(g, w) for g, w in zip(got, want))
 
 
 @pytest.mark.parametrize("kind,n,k", [("res", 48, 9728), ("plain", 48, 1152)])

@@ -15,6 +15,8 @@ qdec_prefill_attn) on the GPU.
   cached prefix.
 """
 
+import math
+
 import pytest
 import torch
 
@@ -434,10 +436,9 @@ def test_prompt_chunking_bitexact(lib, B, S):
 
 @pytest.mark.parametrize("tile", [(64, 64), (256, 256)])
 def test_prefill_gemm_silu_of_every_gate_value(lib, tile):
-    """One-hot rows pick each finite bf16 value as a gate, with an up value
-    of 1: silu in 64 bits rounded to bf16, at most one unit in the last place
-    away where an fp32 result rounds the other way (fewer than 1 in 1000),
-    and nothing but flushed values below the normal range."""
+    """One-hot rows pick each finite bf16 value as a gate, with an up value of
+    1: silu in 64 bits rounded to bf16, bit for bit, -0 where exp overflows in
+    fp32, and nothing but flushed values below the normal range."""
     from qdec import capi
     k = 256
     g = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
@@ -447,10 +448,28 @@ def test_prefill_gemm_silu_of_every_gate_value(lib, tile):
     tiles = k // 16
     out = pgemm(lib, to_frag(lib, x, tiles), pack(lib, w), k, 512, k, tiles, flags=capi.GLU, tile=tile).cpu()
     gd = g.T.double()
-    ref = (gd / (1 + torch.exp(-gd))).to(torch.bfloat16)
-    normal = gd.abs() >= 2.0 ** -125
-    ulps = (out.view(torch.int16).int() - ref.view(torch.int16).int()).abs()
-    deep = ref.abs().float() < 2.0 ** -120
-    assert ulps[normal & ~deep].max() <= 1
-    assert (ulps[normal & ~deep] == 0).float().mean() >= 0.999
-    assert (out[deep | ~normal].float().abs() < 2.0 ** -119).all()
+    ref = gd / (1 + torch.exp(-gd))
+    ref = torch.where(gd < -88.73, torch.full_like(ref, -0.0), ref).to(torch.bfloat16)  # exp(88.73) is past fp32
+    normal = (gd.abs() >= 2.0 ** -125) & ((ref.abs().float() >= 2.0 ** -126) | (gd < -88.73))
+    assert normal.sum() > 60000 and (gd[normal] == -88.5).any() and (gd[normal] == -89).any()
+    assert torch.equal(out.view(torch.int16)[normal], ref.view(torch.int16)[normal])
+    assert (out[~normal].float().abs() <= 2.0 ** -125).all()
+
+
+@pytest.mark.parametrize("tile", [(64, 64), (256, 256)])
+def test_prefill_gemm_silu_of_infinite_gates(lib, tile):
+    """Gates that overflow to +inf and -inf and that are NaN (inf - inf):
+    +inf, and NaN for the other two, as g / (1 + exp(-g)) gives."""
+    from qdec import capi
+    k = 256
+    big = 2.0 ** 64
+    x = torch.zeros(4, k)
+    x[0, 0] = x[1, 1] = x[2, 0] = x[2, 1] = x[3, 2] = big
+    w = torch.zeros(512, k)
+    w[:256, 0], w[:256, 1], w[:256, 2] = big, -big, 1 / big  # gates 2^128, -2^128, their sum, 1
+    w[256:, :3] = 1 / big  # up values of 1 (2 in row 2)
+    tiles = round_up(4, ROW_TILE) // 16
+    out = pgemm(lib, to_frag(lib, x.to(torch.bfloat16), tiles), pack(lib, w.to(torch.bfloat16)), 4, 512, k, tiles,
+                flags=capi.GLU, tile=tile).float()
+    assert (out[0] == float("inf")).all() and out[1].isnan().all() and out[2].isnan().all()
+    assert (out[3] == bf16(torch.tensor(1 / (1 + math.exp(-1))))).all()
