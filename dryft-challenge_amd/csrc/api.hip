@@ -67,7 +67,7 @@ static bool wide_offsets(const qdec_gemm_args *a) { return (uint64_t)a->n * a->k
 
 // What a GEMM plan is for: a qdec_gemm call; qdec_gemm_wide (the many-row plan
 // or an error); a stage of qdec_layer, whose kernel has no ring of 8 (a down
-// whose k range only that ring divides keeps the direct path it is compiled
+// of k = 1024, which that ring takes, keeps the direct path it is compiled
 // for).
 enum class PlanFor { kCall, kWide, kLayer };
 
@@ -253,7 +253,7 @@ static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch, 
   p->xd = 0;
   p->tw = 1;
   p->xn = nullptr;
-  int ring = gemm_ring(p->ksw, f);
+  int ring = gemm_ring(p->ksw, f, xa || (f & QDEC_NORM_IN));
   if (ring == 8 && what == PlanFor::kLayer) ring = 0;
   // Direct path: two tiles per wave at two M tiles when the workgroup's
   // tiles pair up, without GLU (sums unchanged: every tile keeps its own

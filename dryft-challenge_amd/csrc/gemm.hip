@@ -193,16 +193,18 @@ bool gemm_fast_path(const GemmParams &p, uint32_t flags) {
          (!(flags & QDEC_NORM_IN) || p.ksplit == 1);
 }
 
-int gemm_ring(int ksw, uint32_t flags) {
+int gemm_ring(int ksw, uint32_t flags, bool staged) {
   // 20 and 16 measured faster than passes on MI355X; a 19-register ring
   // (k = 9728 with 4 waves) was slower than 20-block passes.  8 (8 gate|up
   // pairs with GLU) for the widths those do not divide (Qwen3-1.7B's k =
   // 2048): staged rows and a short ring beat the normalisation pre-pass and
-  // the direct path, us at one row QKV 12.6 -> 6.3, gate/up 17.1 -> 11.7.
-  if (flags & QDEC_GLU) return ksw % 10 == 0 ? 10 : ksw % 8 == 0 ? 8 : 0;
-  for (const int rw : {20, 16, 8})
-    if (ksw % rw == 0) return rw;
-  return 0;
+  // the direct path, us at one row QKV 12.6 -> 6.3, gate/up 17.1 -> 11.7.  A
+  // call with no need to stage its rows (neither NORM_IN nor a merge of
+  // attention partials) takes it only for a range of that length: 2048 x 2048
+  // on 8 waves 7.0 -> 4.8, but 2560 x 9216 on 4 (72 steps) 14.2 -> 19.6.
+  const bool eight = ksw % 8 == 0 && (staged || ksw == 8);
+  if (flags & QDEC_GLU) return ksw % 10 == 0 ? 10 : eight ? 8 : 0;
+  return ksw % 20 == 0 ? 20 : ksw % 16 == 0 ? 16 : eight ? 8 : 0;
 }
 
 namespace {

@@ -125,7 +125,7 @@ constexpr uint32_t kHandSpin = 1u << 22;
 constexpr int kHandMaxParts = 4;
 bool gemm_flags_supported(uint32_t flags);
 bool gemm_fast_path(const GemmParams &p, uint32_t flags);
-int gemm_ring(int ksw, uint32_t flags);
+int gemm_ring(int ksw, uint32_t flags, bool staged);
 int gemm_ring_direct(int mt, uint32_t flags, int tw, int ksw, int groups);
 hipError_t launch_rownorm(const GemmParams &p, dim3 block, bool do_norm, hipStream_t s);
 hipError_t launch_gemm(const GemmParams &p, uint32_t flags, hipStream_t s);

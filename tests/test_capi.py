@@ -340,6 +340,7 @@ def _set(obj, **kw):
     # a down whose k / 128 a ring of 8 divides, but not the longer ones, keeps
     # the layer kernel's plan (the attention stage after it is what is refused)
     (dict(fix=_set("down", k=9216), cap=100), -1, "cap"),
+    (dict(fix=_set("down", k=1024), cap=100), -1, "cap"),
 ])
 def test_layer_validation(qlib, kw, code, needle):
     kw = dict(kw)

@@ -320,14 +320,15 @@ def test_layer_launch_equals_its_stage_launches(engine, B, S, seed):
     assert not torch.equal(snap[0], got[0])  # the step did something
 
 
-@pytest.mark.parametrize("B", [1, 4])
-def test_layer_launch_of_a_down_on_the_short_ring(B):
-    """An intermediate width of 9216: its down projection's own call stages
-    its rows with a ring of 8, which the layer kernel does not have; the
-    layer launch takes the shape all the same and gives those bits."""
+@pytest.mark.parametrize("B,inter", [(1, 9216), (1, 1024), (4, 1024)])
+def test_layer_launch_of_a_down_on_the_short_ring(B, inter):
+    """Intermediate widths whose down projection a ring of 8 divides but no
+    longer one (the call for 1024 stages its rows with it), which the layer
+    kernel does not have: the layer launch takes them all the same and gives
+    the calls' bits."""
     from qdec.checkpoint import generate_tensors
     from qdec.runtime import DecodeState, DeviceModel
-    cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024, intermediate_size=9216)
+    cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024, intermediate_size=inter)
     model = DeviceModel(cfg, dict(generate_tensors(cfg, seed=3, norm_jitter=0.05)), "cuda:0")
     st = DecodeState(model, B, 80, max_t=1)
     st.prefill(prompts(B, 50, 44, vocab=1024).to(model.device))

@@ -191,11 +191,12 @@ def test_many_rows_argmax_of_infinite_logits(lib, rows):
 
 
 @pytest.mark.parametrize("kind,n,k,waves", [("norm", 4096, 2048, 8), ("norm", 304, 1024, 4), ("glu", 6144, 2048, 4),
-                                            ("glu", 48, 1024, 4), ("res", 304, 2048, 8), ("plain", 304, 1024, 4),
+                                            ("glu", 48, 1024, 4), ("res", 304, 2048, 8), ("res", 304, 9216, 4), ("plain", 304, 1024, 4),
                                             ("argmax", 304, 1024, 4), ("argmax", 4112, 2048, 8)])
 def test_short_ring_bitexact(lib, kind, n, k, waves):
     """Widths whose k range per wave is a multiple of 8 but not of the longer
-    load rings (rows staged in LDS, a ring of 8): 1, 3, 5 and 8 rows give the
+    load rings (rows staged in LDS, a ring of 8; without NORM_IN only a range of
+    8 steps): 1, 3, 5 and 8 rows give the
     bits that a call of 12 rows, which reads them directly, gives."""
     call = Call(lib, kind, n, k, 1, seed=n + k)
     call.waves = waves
