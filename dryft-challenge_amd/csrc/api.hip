@@ -832,20 +832,24 @@ static int prefill_gemm(const qdec_pgemm_args *a, float *parts, int ksplit, qdec
     // The least of the tiles' costs, in rounds of 256 x 256 tiles: the
     // 256-row tiles run one per CU, so ceil(tiles / 256) rounds, a round of
     // 256 x 160 or 256 x 128 costing 0.80 or 0.59 of one (narrower tiles load
-    // more per MFMA); 64 x 64 tiles run three per CU without whole rounds at
-    // about half the rate.  MI355X, us (64 x 64 / 256 x 128 / 256 x 160 /
-    // 256 x 256): O at 1024 rows 39 / 51 / 66 / 86, at 4096 119 / 108 / 77 /
+    // more per MFMA) and its start and end the time of 40 of k; of 64 x 64
+    // tiles, three of which share a CU, one more for a CU costs 0.15.
+    // MI355X, us (64 x 64 / 256 x 128 / 256 x 160 / 256 x 256): O at 1024 rows
+    // 39 / 51 / 66 / 86, at 1500 55 / 48 / - / 82, at 4096 119 / 108 / 77 /
     // 93, at 8192 226 / 166 / 147 / 186, at 32768 1202 / 641 / 613 / 544;
-    // gate/up at 256 rows 50 / 40 / - / 116, at 512 89 / 75 / - / 67, at 8192
-    // 1148 / 691 / - / 635; QKV at 1024 50 / 39 / - / 63.
+    // gate/up at 256 rows 40 / 34 / - / 52, at 300 46 / 63 / - / 54, at 512 72 /
+    // 62 / - / 55, at 8192 1148 / 691 / - / 635; QKV at 512 27 / 33 / - / 55, at
+    // 700 39 / 34 / - / 56; 4096 x 1024 at 1000 17.3 / 18.9; 10240 x 5120 at
+    // 140 33 / 52.  Over 450 (rows, n, k) the pick is at most 6% from the
+    // best of 64 x 64, 256 x 128 and 256 x 256.
     static const struct { int cols; double cost; } kTiles[] = {{256, 1.0}, {160, 0.80}, {128, 0.59}};
     const int64_t row_tiles = a->tiles / 16;
-    double best = 2.0 * (double)row_tiles * a->n / (256.0 * kPgWorkgroups);
+    auto rounds = [](int64_t n) { return (double)((n + kPgWorkgroups - 1) / kPgWorkgroups); };
+    double best = 0.15 * rounds((int64_t)pg_small_row_tiles(a->rows) * (a->n / 64));
     trows = 64, tcols = 64;
     for (const auto &t : kTiles) {
       if (a->n % t.cols || (glu && t.cols == 160)) continue;
-      const int64_t T = (a->n / t.cols) * row_tiles;
-      const double cost = t.cost * (double)((T + kPgWorkgroups - 1) / kPgWorkgroups);
+      const double cost = t.cost * rounds((a->n / t.cols) * row_tiles) * (1.0 + 40.0 / a->k);
       if (cost < best) best = cost, trows = 256, tcols = t.cols;
     }
   }

@@ -376,11 +376,12 @@ __global__ void __launch_bounds__(256, 1) pgemm_small_kernel(const PgemmParams p
   const int col = lane & 15, grp = lane >> 4;
   const int wn = wave & 1, wm = wave >> 1;
 
-  // Tile order as in pgemm_kernel, one tile per workgroup.
+  // Tile order as in pgemm_kernel, one tile per workgroup; row tiles of the
+  // padding beyond the rows are left out.
   int id = blockIdx.x;
   const int G = gridDim.x;
   if ((G & 7) == 0) id = (id & 7) * (G >> 3) + (id >> 3);
-  const int ntm = p.tiles / 4;
+  const int ntm = pg_small_row_tiles(p.rows);
   const int gsz = kPgGroupN * ntm;
   const int g = id / gsz, r = id - g * gsz;
   const int gn = min(kPgGroupN, p.wg_n - g * kPgGroupN);
@@ -981,7 +982,7 @@ hipError_t launch_pgemm_tile(const PgemmParams &p, uint32_t flags, hipStream_t s
 }
 
 hipError_t launch_pgemm_small(const PgemmParams &p, uint32_t flags, hipStream_t s) {
-  const dim3 grid(p.wg_n * (p.tiles / 4)), block(256);
+  const dim3 grid(p.wg_n * pg_small_row_tiles(p.rows)), block(256);
   switch (flags) {
     case 0u: hipLaunchKernelGGL(pgemm_small_kernel<0u>, grid, block, 0, s, p); break;
     case QDEC_RES_OUT: hipLaunchKernelGGL(pgemm_small_kernel<QDEC_RES_OUT>, grid, block, 0, s, p); break;

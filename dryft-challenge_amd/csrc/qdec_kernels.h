@@ -205,6 +205,8 @@ constexpr int kPqMaxHeads = 80;  // query + key heads per row of qdec_prefill_qk
 constexpr int kPgRows = 256;
 constexpr int kPgRowsSmall = 64;
 constexpr int kPgStageK = 64;
+// Row tiles that a call of 64 x 64 tiles runs.
+constexpr __host__ __device__ int pg_small_row_tiles(int rows) { return (rows + kPgRowsSmall - 1) / kPgRowsSmall; }
 // Workgroups of the 256-row tiles: one per CU, each walking its share of them.
 constexpr int kPgWorkgroups = 256;
 struct PgemmParams {
