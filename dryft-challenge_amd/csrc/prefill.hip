@@ -706,9 +706,11 @@ __global__ void __launch_bounds__(64 * kPnWaves) pnorm_kernel(const uint16_t *__
 // vector instructions), and block j's P.V product covers the LDS reads of
 // block j + 2's keys.  Before that every wave of a workgroup met at the
 // block's barrier, multiplied, then exponentiated, so the two units took
-// turns: 8 x 1024 rows after 3072 cached slots 572 -> 512 us (840 -> 940
-// TFLOP/s), and two heads per kv head, alone 540 -> 326 us.  What bounds it
-// now is shared: LDS reads (a wave's 32 rows take every K/V fragment for two
+// turns: 8 x 1024 rows after 3072 cached slots 575 -> 516 us, 503 now that
+// the last block leaves out the scores of none to follow (840 -> 960
+// TFLOP/s; short prompts were 2 to 12% slower with them: 13 x 187 26.0 ->
+// 27.2, now 26.0), and two heads per kv head 513 -> 269 us.  What bounds it
+// is shared: LDS reads (a wave's 32 rows take every K/V fragment for two
 // MFMAs), the vector units and the matrix cores each cost about a fifth of
 // the time when left out.
 // Online softmax in base 2 with fp32 state per row (running max kept in
@@ -848,9 +850,10 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
   if (kPaRing - 1 < nb) dma_block(kPaRing - 1);
   read_k(1);
 
-  // Block j from its scores S; leaves block j + 1's in N (kf holds its keys;
-  // past the last block they are whatever the ring holds, and unused).
-  auto block = [&](int j, Scores &S, Scores &N) {
+  // Block j from its scores S; leaves block j + 1's in N (kf holds its keys)
+  // unless it is the last.
+  auto block = [&](int j, Scores &S, Scores &N, auto lastc) {
+    constexpr bool LAST = decltype(lastc)::value != 0;
     const int sb = j * 32 + 8 * grp;  // first of this lane's 8 slots
     if (!(rows_full && j * 32 + 31 <= p.pos0 + t0)) {
       // the block crosses some row's position (the diagonal, rows past the end)
@@ -895,8 +898,10 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
         float x = e < 4 ? S.a[u][e] : S.b[u][e - 4];
         pin(x);
         pj[u][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(x, scale, -mc[u]));
-        score1(N, i / (2 * MT), (i >> 1) % MT, i & 1);
-        pin((i & 1) ? N.b[(i >> 1) % MT] : N.a[(i >> 1) % MT]);
+        if constexpr (!LAST) {
+          score1(N, i / (2 * MT), (i >> 1) % MT, i & 1);
+          pin((i & 1) ? N.b[(i >> 1) % MT] : N.a[(i >> 1) % MT]);
+        }
         if (i > 0) psum[(i - 1) >> 3] += pj[(i - 1) >> 3][(i - 1) & 7];
         pin(pj[u][e]);
       }
@@ -907,8 +912,10 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
       pf[u] = pack8(pj[u]);
     }
     // Block j + 2 in LDS; slot j (whose V every wave holds) takes block j + kPaRing.
-    await(min(j + 2, nb - 1), j + kPaRing - 1);
-    if (j + kPaRing < nb) dma_block(j + kPaRing);
+    if constexpr (!LAST) {
+      await(min(j + 2, nb - 1), j + kPaRing - 1);
+      if (j + kPaRing < nb) dma_block(j + kPaRing);
+    }
     if (j * 32 + 31 > last) {  // slots past the last row: zero V
       uint32_t keep[4];
 #pragma unroll
@@ -922,16 +929,23 @@ __global__ void __launch_bounds__(64 * G * kPaWph, 2) pattn_kernel(const PattnPa
         vf[dt].w &= keep[3];
       }
     }
-    read_k(j + 2);
+    if constexpr (!LAST) read_k(j + 2);
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
       for (int u = 0; u < MT; ++u) acc[u][dt] = mfma16x16x32(vf[dt], pf[u], acc[u][dt]);
   };
-  for (int j = 0; j < nb; j += 2) {
-    block(j, s0, s1);
-    if (j + 1 < nb) block(j + 1, s1, s0);
+  int j = 0;
+  if (!(nb & 1)) {  // pairs, then the last block by itself
+    block(0, s0, s1, Int<0>{});
+    s0 = s1;
+    j = 1;
   }
+  for (; j + 1 < nb; j += 2) {
+    block(j, s0, s1, Int<0>{});
+    block(j + 1, s1, s0, Int<0>{});
+  }
+  block(j, s0, s1, Int<1>{});
 
   // Rows in fragment order for the O projection: lane holds channels
   // 16dt + 4*grp .. +3 of its row.
@@ -1041,17 +1055,22 @@ hipError_t launch_pnorm(const void *x, const void *norm_w, void *out, float eps,
 }
 
 namespace {
-// Short prompts: one M tile per wave (32 positions per workgroup) while 64
-// positions leave more than half of the CUs idle -- a block takes a wave
-// about as long as its latencies, however few rows it carries.  MI355X, us
-// (64 positions / 32): one sequence of 300 tokens 19.2 / 12.3, 512 28.2 / 18.0,
-// 1024 49.5 / 31.7; 128 positions after 2000 cached 88 / 52; 8 x 128 13.6 /
-// 10.4.
+// One M tile per wave (32 positions per workgroup) instead of two: for calls
+// of at most 32 positions; while 64 leave more than half of the CUs idle -- a
+// block takes a wave about as long as its latencies, however few rows it
+// carries; and, up to a workgroup per CU, where the positions cover most of
+// the slots they see (pos0 < t_rows), so that the workgroups' lengths differ
+// and two short ones share a CU.  MI355X, us (64 positions / 32): one sequence
+// of 300 tokens 19.2 / 12.3, 512 28.2 / 18.0, 1024 49.5 / 31.7; 128 positions
+// after 2000 cached 88 / 52; 8 x 128 13.6 / 10.4; 64 sequences of 20 on 16
+// heads 10.9 / 8.3; 10 x 67 13.0 / 9.5; 1791 78 / 56; but 5 x 258 after 1479
+// 73 / 84.
 template <int G, int GS>
 void launch_pattn(const PattnParams &p, hipStream_t s) {
   const int cells = p.batch * p.nkv * (GS / G);
   const int b64 = (p.t_rows + kPaRows - 1) / kPaRows * cells, b32 = (p.t_rows + kPaRows / 2 - 1) / (kPaRows / 2) * cells;
-  if (b64 <= 128)
+  const bool few = b64 <= 128 || p.t_rows <= kPaRows / 2 || (b64 <= 256 && p.pos0 < p.t_rows);
+  if (few)
     hipLaunchKernelGGL((pattn_kernel<G, GS, 1>), dim3(b32), dim3(64 * G * kPaWph), 0, s, p);
   else
     hipLaunchKernelGGL((pattn_kernel<G, GS, 2>), dim3(b64), dim3(64 * G * kPaWph), 0, s, p);
