@@ -303,3 +303,28 @@ def test_short_prompt_of_widths_the_wide_product_refuses(lib, monkeypatch, B, S,
     for got, want in ((st.k_cache, ref.k_cache), (st.v_cache, ref.v_cache)):
         assert (got.float() - want.float()).abs().max() <= 2e-2 * want.float().abs().max()
     assert st.lens.tolist() == [S] * B
+
+
+@pytest.mark.parametrize("B", [1, 2])
+def test_attention_merged_in_o_on_the_short_ring(lib, monkeypatch, B):
+    """16 query heads on 4 kv heads: O (k = 2048 on 8 waves, a ring of 8)
+    merges the attention's chunk partials while it stages its rows; the step
+    has the bits of the one whose attention merges them."""
+    from qdec.checkpoint import generate_tensors, qwen3_config
+    from qdec.runtime import DecodeState, DeviceModel
+    cfg = qwen3_config(num_hidden_layers=2, vocab_size=1024, hidden_size=1024, intermediate_size=3072,
+                       num_attention_heads=16, num_key_value_heads=4)
+    model = DeviceModel(cfg, dict(generate_tensors(cfg, seed=3, norm_jitter=0.05)), DEV)
+    prompt = torch.randint(0, 1024, (B, 300), generator=torch.Generator().manual_seed(B)).to(DEV)
+    got = []
+    for merge in (True, False):
+        st = DecodeState(model, B, 640, max_t=1, keep_logits=True)
+        assert st._merge_in_o(1) and st.chunk < 300
+        if not merge:
+            monkeypatch.setattr(st, "_merge_in_o", lambda t: False)
+        st.prefill(prompt)
+        for _ in range(3):
+            st.run_step()
+        torch.cuda.synchronize()
+        got.append((st.logits[:B].clone(), st.ids[:B].clone()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
