@@ -324,8 +324,8 @@ static int plan_gemm(const qdec_gemm_args *a, GemmParams *p, bool need_scratch, 
     }
   }
   // Register staging of 5..8 rows has a window-path instantiation only; on
-  // the pass path (a wave's k range that no ring divides, e.g. the lm_head's
-  // 8 k steps at hidden 1024) the rows are staged through LDS instead.
+  // the pass path (a wave's k range that no ring divides, e.g. the 9 k steps
+  // of k = 1152) the rows are staged through LDS instead.
   if (p->xfast && a->rows > kFastRowsMax && p->rw == 0) p->xfast = 0;
   // A pending split residual update is merged by the register-staged
   // prologue at one row, else by the normalisation pre-pass (once per row;

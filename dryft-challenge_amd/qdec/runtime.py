@@ -38,9 +38,9 @@ GEMM_MAX_ROWS = 64
 GEMM_WIDE_MIN_ROWS = 9  # of qdec_gemm_wide
 ATTN_MAX_T = 16
 # Rows (sequences x positions) of one prefill chunk: activations of 32K rows
-# take about 2.2 GB; at that size O and down still make 1280 workgroups of
-# the 256 x 256 product tile (32 x 4096 prompts: 1.33 s at 16K rows, 1.27 s
-# at 32K, 1.29 s at 64K; the tokens are the same for any chunking).
+# take about 2.2 GB; at that size O and down still make 1280 tiles of 256 x 256,
+# five whole rounds of the CUs (32 x 4096 prompts: 1.33 s at 16K rows, 1.27 s
+# at 32K, 1.29 s at 64K; the bits are the same for any chunking).
 PREFILL_ROWS = 32768
 # Row tile of the prefill product (kPgRows of qdec_kernels.h); a chunk of at
 # most PREFILL_WIDE_ROWS rows is padded to PREFILL_ROW_TILE_SMALL instead

@@ -268,12 +268,13 @@ int qdec_gemm_workspace(const qdec_gemm_args *a, size_t *partial_bytes,
 int qdec_gemm_prepass(const qdec_gemm_args *a, int32_t *threads);
 
 /* qdec_gemm at 9..128 rows on the many-row kernel that qdec_gemm itself takes
- * from 9 to 64 rows at four waves: the same arguments and results, with
+ * from 9 to 64 rows at four waves where it is the faster one (k ranges of more
+ * than 8 steps per wave from 17 or 33 rows): the same arguments and results, with
  * flags 0, NORM_IN, RES_OUT, GLU or NORM_IN | GLU, waves 4, tiles_per_wg 1, k / 32
  * / ksplit a multiple of 4, x_frag = 1 or NORM_IN (whose pre-pass writes the
  * normalised rows to the partial workspace), ksplit > 1 only with parts_out,
- * and no x_attn, next_norm_w or resident; n (2n with GLU) x k below 2 Gi
- * elements.  QDEC_EUNSUPPORTED otherwise.  For the products of a short prompt,
+ * and no x_attn, next_norm_w or resident; n x k (with GLU of either half)
+ * below 2 Gi elements.  QDEC_EUNSUPPORTED otherwise.  For the products of a short prompt,
  * whose weights are read once for all rows.
  * Replaces F.linear as the prefill forward uses it (engine/engine.py:448-461). */
 int qdec_gemm_wide(const qdec_gemm_args *a, qdec_stream_t stream);
@@ -542,8 +543,9 @@ int qdec_prefill_qk(const qdec_prefill_qk_args *a, qdec_stream_t stream);
 /* Causal GQA attention of the rows at positions pos0 .. pos0 + t_rows - 1
  * (queries as qdec_prefill_qk leaves them) over cache slots 0 .. position,
  * written in fragment order (`tiles` M tiles) for the O projection.  A
- * workgroup takes 64 positions of the G = nq / nkv query heads of one kv
- * head (G = 2, 4 or 8; QDEC_EUNSUPPORTED otherwise); same
+ * workgroup takes 64 positions (32 in small calls, the same bits) of 2 or 4
+ * of the G = nq / nkv query heads of one kv head (G = 2, 4 or 8;
+ * QDEC_EUNSUPPORTED otherwise); same
  * arithmetic as qdec_attn (base-2 online softmax in fp32, probabilities
  * rounded to bf16 before P.V, fp32 accumulation, one rounding).
  * Replaces Engine._attend_prefill (engine/engine.py:464-478: SDPA flash

@@ -485,8 +485,8 @@ def test_selfcheck_detects_a_wrong_answer(engine, monkeypatch):
 def test_shape_selfcheck_detects_a_dropped_launch(engine, monkeypatch, what):
     """Every new shape runs the known-answer checks through its own plans
     before its first token (here batch 32: the 8-wave attention over one
-    whole-cache chunk, fragment-order hand-overs, the down projection's k
-    split merged by the next NORM_IN call, two tiles per wave, the 8-tile
+    whole-cache chunk, fragment-order hand-overs, the k splits of O and down
+    merged by the next NORM_IN call, the resident plans, the many-row
     lm_head).  Dropping one of its 32-row launches (simulated on the host)
     makes generate raise before it yields anything, and the shape is not
     kept; with the launch back the same shape serves."""
@@ -529,9 +529,10 @@ def test_shape_selfcheck_detects_a_dropped_launch(engine, monkeypatch, what):
 @pytest.mark.parametrize("B,spec", [(1, False), (3, True), (8, False), (12, False), (20, False), (64, False)])
 def test_shape_selfcheck_passes(ckpt, engine, B, spec):
     """The per-shape checks pass on every plan family: merge in O (1),
-    verify rows of a speculative state (3: t = 1 and k + 1), register-staged
-    rows and 8-wave 512-slot chunks (8, 12), two tiles per wave and the down
-    split (20), four M tiles (64)."""
+    verify rows of a speculative state (3: t = 1 and k + 1), 8-wave strided
+    chunks with rows in LDS (8), the many-row kernel with split O and down
+    (12), the resident plans of two M tiles (20), four M tiles and the 4-wave
+    attention (64)."""
     from engine import spec_k
     from qdec import selfcheck
     from qdec.runtime import DecodeState
