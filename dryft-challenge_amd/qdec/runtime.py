@@ -145,6 +145,9 @@ RESIDENT_SPLIT_ROWS = (17, 32)
 # below 6 rows: 19.0 -> 21.0 us at batch 1, 20.1 -> 21.1 at batch 4.  At
 # 17..32 rows the pre-pass's rows are copied in and k splits over 4 waves
 # (role_plan): batch 32 at 4096-token prompts 5.481 -> 5.449 ms per step.
+# Against the many-row kernel, which the same calls take without these plans
+# (graph replays at 24 rows, pre-pass included, us resident / many-row): QKV
+# 13.3 / 13.7, gate/up 24.7 / 25.0, O 7.6 / 7.5, the split down 13.0 / 11.6.
 RESIDENT_QKV_ROWS = ((1, 8), (17, 32))
 
 
